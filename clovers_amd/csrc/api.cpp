@@ -129,6 +129,8 @@ struct clv_ctx {
   uint32_t cap_paths = 0;
   PathBuf pb;                /* the view of even bounces; odd bounces swap the two entry sets */
   uint32_t *shadeq[MC_COUNT] = {nullptr};
+  F3 *res = nullptr;         /* sample contributions of a whole-path pass, by slot */
+  uint32_t cap_res = 0;
   /* accumulators */
   uint32_t cap_pixels = 0;
   float *acc32 = nullptr;
@@ -258,6 +260,32 @@ struct TraceGeom {
   uint32_t lds_node_base = 0, lds_nodes = 0, lds_unit_base = 0, lds_units = 0;
 };
 
+/* Whole paths in one launch per pass (k_paths) wherever the LDS-cached
+ * traversal is asked for and nothing has to be seen between the bounces: no
+ * guided job (the network runs between tracing and shading), no per-launch
+ * timing, no counting. */
+bool whole_paths(const clv_ctx *c, bool any_guide, uint32_t flags) {
+  return c->trace_variant == TRACE_LDS && !any_guide && !(flags & (CLV_FLAG_TIME_KERNELS | CLV_FLAG_COUNT));
+}
+
+/* a pass of k_paths keeps 12 bytes per sample, so an untuned context runs the
+ * samples of a whole render in one (up to 1.6 GB of contributions) */
+#define DEFAULT_TARGET_PATHS (1u << 22)
+#define WHOLE_TARGET_PATHS (1u << 27)
+
+clv_status paths_geometry(clv_ctx *c, const SceneRes *s, bool ext, bool media, TraceGeom *g) {
+  const size_t stack = paths_lds_bytes(0, 0);
+  size_t budget = c->lds_block_bytes > stack ? c->lds_block_bytes - stack : 0;
+  g->lds_node_base = s->base.nodes;
+  g->lds_unit_base = s->base.units;
+  g->lds_nodes = (uint32_t)std::min<size_t>(s->n_nodes, budget / sizeof(Bvh4Node));
+  budget -= (size_t)g->lds_nodes * sizeof(Bvh4Node);
+  g->lds_units = (uint32_t)std::min<size_t>(s->prim_units, budget / 16u);
+  g->lds_bytes = paths_lds_bytes(g->lds_nodes, g->lds_units);
+  g->blocks = paths_grid_blocks(g->lds_bytes, ext, media);
+  return ensure_spill(c, paths_spill_words(g->blocks));
+}
+
 /* the traversal kernel a batch runs: the tuned one, or the plain one when a
  * scene of the batch has constant media (only it has the media pass) */
 int trace_variant_for(const clv_ctx *c, bool media) { return media ? TRACE_SIMPLE : c->trace_variant; }
@@ -308,6 +336,16 @@ clv_status ensure_paths(clv_ctx *c, uint32_t n) {
   HIPCHK(c, dalloc(&b.hero, n));
   for (uint32_t k = 0; k < MC_COUNT; k++) HIPCHK(c, dalloc(&c->shadeq[k], n));
   c->cap_paths = n;
+  return CLV_OK;
+}
+
+clv_status ensure_res(clv_ctx *c, uint32_t n) {
+  if (n <= c->cap_res) return CLV_OK;
+  dfree(c->res);
+  c->res = nullptr;
+  c->cap_res = 0;
+  HIPCHK(c, dalloc(&c->res, n));
+  c->cap_res = n;
   return CLV_OK;
 }
 
@@ -646,13 +684,23 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
         return fail(c, CLV_EINVAL, "with guide_warmup, image sample indices stay below 2^31");
   HIPCHK(c, hipSetDevice(c->device));
   const bool frozen = (flags & CLV_FLAG_GUIDE_FROZEN) != 0;
+  const bool whole = whole_paths(c, any_guide, flags);
   PassPlan pl;
   /* a frozen network is not trained: no training slices, every pass full size */
-  plan_passes(dj, soff, c->target_paths, std::max<uint32_t>(1, c->guide.train_spp), frozen ? 0u : c->guide.rounds,
+  plan_passes(dj, soff, whole && c->target_paths == DEFAULT_TARGET_PATHS ? WHOLE_TARGET_PATHS : c->target_paths, std::max<uint32_t>(1, c->guide.train_spp), frozen ? 0u : c->guide.rounds,
               c->guide.warmup != 0, &pl);
-  for (DevItem &it : pl.items) it.order = c->tile_order;
+  std::vector<uint32_t> job_left(n);
+  for (uint32_t k = 0; k < n; k++) job_left[k] = dj[k].spp;
+  for (DevItem &it : pl.items) {
+    it.order = c->tile_order;
+    if (it.flags & ITEM_WARMUP) continue;
+    if (job_left[it.job] == dj[it.job].spp) it.flags |= ITEM_FIRST;
+    job_left[it.job] -= it.samples;
+    if (job_left[it.job] == 0) it.flags |= ITEM_LAST;
+  }
   const uint32_t passes = (uint32_t)pl.paths.size();
-  CHK(ensure_paths(c, pl.max_paths));
+  if (whole) CHK(ensure_res(c, pl.max_paths));
+  else CHK(ensure_paths(c, pl.max_paths));
   CHK(ensure_pixels(c, (uint32_t)pixels));
   CHK(ensure_tables(c, n, (uint32_t)pl.items.size()));
   GuideState &gs = c->guide;
@@ -669,7 +717,8 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
     if ((uint64_t)dj[k].width * dj[k].height * dj[k].spp > (uint64_t)dj[big].width * dj[big].height * dj[big].spp) big = k;
   TraceGeom geom;
   const int variant = trace_variant_for(c, any_media);
-  CHK(trace_geometry(c, sres[big], pl.max_paths, &geom, variant));
+  if (whole) CHK(paths_geometry(c, sres[big], any_ext, any_media, &geom));
+  else CHK(trace_geometry(c, sres[big], pl.max_paths, &geom, variant));
   /* the tail launch (k_tail): the resident grid of the plain traversal, never with per-launch timing or
    * counting (those measure the wavefront traversal) */
   const uint32_t tail_depth = (flags & (CLV_FLAG_TIME_KERNELS | CLV_FLAG_COUNT)) ? 0u : c->tail_depth;
@@ -688,7 +737,7 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
   const bool timing = (flags & CLV_FLAG_TIME_KERNELS) != 0;
   const bool counting = (flags & CLV_FLAG_COUNT) != 0;
   uint32_t extends = 0;
-  for (uint32_t p = 0; p < passes; p++) extends += tail_depth ? std::min(pl.depth[p] + 1u, tail_depth + 1u) : pl.depth[p] + 1u;
+  for (uint32_t p = 0; p < passes; p++) extends += whole ? 1u : tail_depth ? std::min(pl.depth[p] + 1u, tail_depth + 1u) : pl.depth[p] + 1u;
   size_t need_events = 2 + (timing ? 2 * (size_t)extends : 0);
   while (c->events.size() < need_events) {
     hipEvent_t e;
@@ -737,6 +786,37 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
   /* every launch of the render; no host synchronisation inside, so the
    * sequence can be captured as a graph */
   auto enqueue = [&]() -> clv_status {
+  if (whole) {
+    for (uint32_t p = 0; p < passes; p++) {
+      GenParams gp;
+      memset(&gp, 0, sizeof(gp));
+      gp.items = c->items + pl.first[p];
+      gp.n_items = pl.first[p + 1] - pl.first[p];
+      gp.paths = pl.paths[p];
+      PathsArgs pa;
+      memset(&pa, 0, sizeof(pa));
+      pa.next = c->counts + CNT_FETCH;
+      pa.spill = c->spill;
+      pa.stats = (unsigned long long *)c->stats;
+      pa.res = c->res;
+      pa.cie = c->cie;
+      pa.lds_node_base = geom.lds_node_base;
+      pa.lds_nodes = geom.lds_nodes;
+      pa.lds_unit_base = geom.lds_unit_base;
+      pa.lds_units = geom.lds_units;
+      /* a pass smaller than the grid is spread over all its blocks */
+      const uint32_t block = paths_block();
+      const uint32_t blocks = std::min(geom.blocks, (gp.paths + 63u) / 64u);
+      pa.first = (uint32_t)std::min<uint64_t>(block, ((uint64_t)gp.paths + 64ull * blocks - 1u) / (64ull * blocks) * 64ull);
+      pa.chunk = block;
+      launch_paths(c->stream, ds, gp, pa, blocks, geom.lds_bytes, p == 0);
+      rp.items = gp.items;
+      rp.n_items = gp.n_items;
+      rp.threads = pl.res[p];
+      launch_resolve_xyz(c->stream, rp, c->res, c->out, any_sq ? c->out_sq : nullptr);
+    }
+    return CLV_OK;
+  }
   launch_zero_u64(c->stream, c->stats, 8);
   launch_zero_accum(c->stream, rp);
   for (uint32_t pr = 0; photon_rounds && pr < gs.pre_rounds; pr++) {
@@ -838,7 +918,7 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
     add(pl.res.data(), pl.res.size() * 4);
     add(pl.depth.data(), pl.depth.size() * 4);
     add(pl.train.data(), pl.train.size());
-    const uint32_t sc[13] = {flags, any_sq, any_guide, frozen, (uint32_t)variant, c->grid_cap, ds.has_xforms,
+    const uint32_t sc[14] = {(uint32_t)whole, flags, any_sq, any_guide, frozen, (uint32_t)variant, c->grid_cap, ds.has_xforms,
                              gs.train_spp, ds.has_ext, gs.credit, tail_depth, photon_rounds ? gs.photons : 0u,
                              photon_rounds ? gs.pre_rounds : 0u};
     add(sc, sizeof(sc));
@@ -848,7 +928,7 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
     add(&pb, sizeof(pb));
     const void *ptrs[] = {c->shadeq[0], c->shadeq[1], c->shadeq[2], c->shadeq[3],
                           c->shadeq[4], c->acc32, c->acc64, c->accsq, c->out, c->out_sq, c->counts, c->stats,
-                          c->spill, c->cie, c->jobs, c->items, gs.lobes, gs.rec, gs.gcnt, gs.list, gs.bcount,
+                          c->spill, c->cie, c->res, c->jobs, c->items, gs.lobes, gs.rec, gs.gcnt, gs.list, gs.bcount,
                           gs.bweight, gs.totals, gs.P, gs.M, gs.V, gs.Wh, gs.partial, gs.cells, gs.cell_tot, gs.gate};
     add(ptrs, sizeof(ptrs));
     for (auto &a : c->arena) add(&a.p, sizeof(a.p));
@@ -1065,6 +1145,7 @@ void clv_destroy(clv_ctx *c) {
   for (auto &a : c->arena) dfree(a.p);
   free_paths(c);
   free_pixels(c);
+  dfree(c->res);
   dfree(c->jobs);
   dfree(c->items);
   guide_free(c->guide);

@@ -182,6 +182,8 @@ typedef struct {
   uint32_t flags;         /* ITEM_WARMUP: the samples train the guiding network only, the image never sees them */
 } DevItem;
 #define ITEM_WARMUP 1u
+#define ITEM_FIRST 2u   /* holds the job's first samples */
+#define ITEM_LAST 4u    /* holds the job's last samples */
 /* warm-up samples take stream indices from here on, apart from any image sample */
 #define WARMUP_SAMPLE_BASE 0x80000000u
 

@@ -461,10 +461,9 @@ __device__ __forceinline__ bool lane_leaf_step(Lane &L, const DevScene &sc, bool
  * [tmin, tmax], so the tree's box culling never changes its outcome, and its
  * uniform is keyed by the medium, so the order of the tests does not matter).
  * Only the traversal instance for batches with media runs this. */
-__device__ __forceinline__ void lane_media(Lane &L, const DevScene &sc, const PathBuf &pb) {
-  const DevJob &jb = sc.jobs[pb.meta[L.path] >> META_JOB_SHIFT];
+__device__ __forceinline__ void lane_media(Lane &L, const DevScene &sc, uint32_t meta, uint64_t state) {
+  const DevJob &jb = sc.jobs[meta >> META_JOB_SHIFT];
   if (jb.n_media == 0) return;
-  const uint64_t state = pb.rng[L.path];
   uint32_t off = jb.media_off;
   for (uint32_t k = 0; k < jb.n_media; k++) {
     const float4 *rec = sc.prims + off;
@@ -531,49 +530,61 @@ __device__ __forceinline__ uint32_t tile_pixel(uint32_t q, uint32_t W, uint32_t 
   return (8u * band + yi) * W + 8u * tc + (q2 - yi * tw);
 }
 
+/* the camera sample of path slot i of a pass: its ray, the state of its
+ * stream after the sampler's draws, and its meta word (depth 0) */
+__device__ __forceinline__ uint32_t camera_sample(const DevScene &sc, const GenParams &gp, uint32_t i, V &org, V &dir,
+                                                  float &time, uint64_t &s) {
+  const DevItem it = gp.items[find_entry(gp.items, gp.n_items, i, &DevItem::path_base)];
+  const DevJob &jb = sc.jobs[it.job];
+  const uint32_t W = jb.width, H = jb.height;
+  uint32_t k = i - it.path_base;
+  uint32_t j = k / it.pixels, o = k - j * it.pixels;
+  if (it.order) o = tile_pixel(o, W, H);
+  uint32_t r = o / W, x = o - r * W;
+  uint32_t y = H - 1u - r;
+  uint32_t sample = it.sample_base + j;
+  s = pcg_for_path(jb.seed, x + y * W, sample);
+  float ox = rnd(s), oy = rnd(s);
+  float lx, ly;
+  for (;;) {
+    lx = rnd_pm1(s);
+    ly = rnd_pm1(s);
+    if (lx * lx + ly * ly <= 1.0f) break;
+  }
+  time = rnd(s); /* the ray's instant (sampler/random.rs:23); carried in ray_d.w */
+  uint32_t wl = (uint32_t)(((uint64_t)pcg_next(s) * 400ull) >> 32);
+  float u = ((float)x + ox) / (float)W;
+  float v = ((float)y + oy) / (float)H;
+  const DevCamera &c = jb.cam;
+  lx *= c.lens_radius;
+  ly *= c.lens_radius;
+  V cu = mk(c.u[0], c.u[1], c.u[2]), cv = mk(c.v[0], c.v[1], c.v[2]);
+  V off = lx * cu + ly * cv;
+  org = mk(c.origin[0], c.origin[1], c.origin[2]);
+  dir = mk(c.llc[0], c.llc[1], c.llc[2]) + u * mk(c.horizontal[0], c.horizontal[1], c.horizontal[2]) +
+        v * mk(c.vertical[0], c.vertical[1], c.vertical[2]) - org - off;
+  dir = unit(dir);
+  org = org + off;
+  return wl | (it.job << META_JOB_SHIFT);
+}
+
 __global__ __launch_bounds__(256) void k_generate(DevScene sc, PathBuf pb, GenParams gp) {
   uint32_t n = gp.paths;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const DevItem it = gp.items[find_entry(gp.items, gp.n_items, i, &DevItem::path_base)];
-    const DevJob &jb = sc.jobs[it.job];
-    const uint32_t W = jb.width, H = jb.height;
-    uint32_t k = i - it.path_base;
-    uint32_t j = k / it.pixels, o = k - j * it.pixels;
-    if (it.order) o = tile_pixel(o, W, H);
-    uint32_t r = o / W, x = o - r * W;
-    uint32_t y = H - 1u - r;
-    uint32_t sample = it.sample_base + j;
-    uint64_t s = pcg_for_path(jb.seed, x + y * W, sample);
-    float ox = rnd(s), oy = rnd(s);
-    float lx, ly;
-    for (;;) {
-      lx = rnd_pm1(s);
-      ly = rnd_pm1(s);
-      if (lx * lx + ly * ly <= 1.0f) break;
-    }
-    const float time = rnd(s); /* the ray's instant (sampler/random.rs:23); carried in ray_d.w */
-    uint32_t wl = (uint32_t)(((uint64_t)pcg_next(s) * 400ull) >> 32);
-    float u = ((float)x + ox) / (float)W;
-    float v = ((float)y + oy) / (float)H;
-    const DevCamera &c = jb.cam;
-    lx *= c.lens_radius;
-    ly *= c.lens_radius;
-    V cu = mk(c.u[0], c.u[1], c.u[2]), cv = mk(c.v[0], c.v[1], c.v[2]);
-    V off = lx * cu + ly * cv;
-    V org = mk(c.origin[0], c.origin[1], c.origin[2]);
-    V dir = mk(c.llc[0], c.llc[1], c.llc[2]) + u * mk(c.horizontal[0], c.horizontal[1], c.horizontal[2]) +
-            v * mk(c.vertical[0], c.vertical[1], c.vertical[2]) - org - off;
-    dir = unit(dir);
-    org = org + off;
+    V org, dir;
+    float time;
+    uint64_t s;
+    const uint32_t meta = camera_sample(sc, gp, i, org, dir, time, s);
+    const uint32_t root = sc.jobs[meta >> META_JOB_SHIFT].root;
     /* slot i is entry i of the first bounce */
-    pb.ray_o[i] = make_float4(org.x, org.y, org.z, __uint_as_float(jb.root));
+    pb.ray_o[i] = make_float4(org.x, org.y, org.z, __uint_as_float(root));
     pb.ray_d[i] = make_float4(dir.x, dir.y, dir.z, time);
     pb.thr[i] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
     pb.rng[i] = s;
-    pb.meta[i] = wl | (it.job << META_JOB_SHIFT); /* depth 0 */
+    pb.meta[i] = meta;
     pb.slot[i] = i;
     pb.rad[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    pb.hero[i] = wl;
+    pb.hero[i] = meta & META_HERO_MASK;
     if (pb.gcnt) {
       pb.gcnt[i] = 0u;
 #pragma unroll
@@ -595,25 +606,27 @@ __global__ __launch_bounds__(256) void k_generate(DevScene sc, PathBuf pb, GenPa
 #define LT_STACK_LDS 8
 #define LT_STACK_GLOBAL (STACK_TOTAL - LT_STACK_LDS)
 
+template <int BLOCK, int DEPTH>
 struct LStack {
-  uint32_t *lst;   /* LDS, stride LT_BLOCK */
-  uint32_t *gst;   /* global slice */
+  uint32_t *lst;   /* LDS: DEPTH entries per lane, stride BLOCK */
+  uint32_t *gst;   /* global slice: the entries from DEPTH on */
+  __device__ __forceinline__ void push(Lane &L, uint32_t w) const {
+    if (L.sp < DEPTH) lds_store(lst + (uint32_t)L.sp * BLOCK, w);
+    else if (L.sp < STACK_TOTAL) gst[L.sp - DEPTH] = w;
+    else return; /* unreachable: the host bounds the BVH depth */
+    L.sp++;
+  }
+  __device__ __forceinline__ void pop(Lane &L) const {
+    if (L.sp == 0) { L.word = CHILD_EMPTY; return; }
+    L.sp--;
+    if (L.sp < DEPTH) L.word = lds_load(lst + (uint32_t)L.sp * BLOCK);
+    else L.word = gst[L.sp - DEPTH];
+  }
 };
-__device__ __forceinline__ void ls_push(Lane &L, const LStack &S, uint32_t w) {
-  if (L.sp < LT_STACK_LDS) lds_store(S.lst + (uint32_t)L.sp * LT_BLOCK, w);
-  else if (L.sp < STACK_TOTAL) S.gst[L.sp - LT_STACK_LDS] = w;
-  else return; /* unreachable: the host bounds the BVH depth */
-  L.sp++;
-}
-__device__ __forceinline__ void ls_pop(Lane &L, const LStack &S) {
-  if (L.sp == 0) { L.word = CHILD_EMPTY; return; }
-  L.sp--;
-  if (L.sp < LT_STACK_LDS) L.word = lds_load(S.lst + (uint32_t)L.sp * LT_BLOCK);
-  else L.word = S.gst[L.sp - LT_STACK_LDS];
-}
 
 /* one interior node whose 8 float4 start at nf (LDS or global) */
-__device__ __forceinline__ void lnode_at(Lane &L, const float4 *nf, const LStack &S) {
+template <class STACK>
+__device__ __forceinline__ void lnode_at(Lane &L, const float4 *nf, const STACK &S) {
   float4 cf = nf[6];
   uint32_t cw[4] = {as_u(cf.x), as_u(cf.y), as_u(cf.z), as_u(cf.w)};
   float tn[4];
@@ -630,9 +643,9 @@ __device__ __forceinline__ void lnode_at(Lane &L, const float4 *nf, const LStack
 #undef CSWAP
 #pragma unroll
   for (int k = 3; k >= 1; k--)
-    if (tn[k] < FLT_MAX) ls_push(L, S, cw[k]);
+    if (tn[k] < FLT_MAX) S.push(L, cw[k]);
   if (tn[0] < FLT_MAX) L.word = cw[0];
-  else ls_pop(L, S);
+  else S.pop(L);
 }
 
 /* one primitive record at rec (LDS or global) */
@@ -649,13 +662,49 @@ __device__ __forceinline__ void lprim_at(Lane &L, const DevScene &sc, const floa
   units = prim_units(hdr & PT_TYPE_MASK);
 }
 
+/* the part of the scene a block keeps in LDS */
+struct LdsWindow {
+  const float4 *nodes, *prims;
+  uint32_t nn, nb;   /* nodes [nb, nb + nn) */
+  uint32_t nu, ub;   /* primitive units [ub, ub + nu) */
+};
+
+/* a lane's whole traversal */
+template <bool COUNT, class STACK>
+__device__ __forceinline__ void lds_traverse(Lane &L, const DevScene &sc, const LdsWindow &w, const STACK &S,
+                                             bool any_xform, uint32_t &nvisit, uint32_t &ntest) {
+  while (L.word != CHILD_EMPTY) {
+    if (!(L.word & CHILD_LEAF)) {
+      const uint32_t rel = L.word - w.nb; /* wraps above nn for nodes below the window */
+      if (rel < w.nn) lnode_at(L, w.nodes + rel * 8u, S);
+      else lnode_at(L, reinterpret_cast<const float4 *>(sc.nodes + L.word), S);
+      if (COUNT) nvisit++;
+    } else {
+      /* one primitive per step: a lane on a leaf of 8 does not hold up the
+       * lanes taking node steps; the leaf word keeps the primitives left
+       * (the same order, so the same hits) */
+      const uint32_t cnt = ((L.word >> 28) & 7u) + 1u;
+      const uint32_t off = L.word & LEAF_OFFSET_MASK;
+      uint32_t units;
+      if (off >= w.ub && off + PREC_QUAD <= w.ub + w.nu)
+        lprim_at(L, sc, w.prims + (off - w.ub), off, any_xform, units);
+      else
+        lprim_at(L, sc, sc.prims + off, off, any_xform, units);
+      if (COUNT) ntest++;
+      if (cnt > 1u) L.word = (L.word & ~(LEAF_OFFSET_MASK | (7u << 28))) | ((cnt - 2u) << 28) | (off + units);
+      else S.pop(L);
+    }
+  }
+}
+
 template <bool COUNT, int MODE>
 __global__ __launch_bounds__(LT_BLOCK) void k_trace_lds(DevScene sc, PathBuf pb, TraceArgs ta) {
   extern __shared__ float4 smem[];
   const uint32_t nn = ta.lds_nodes, nu = ta.lds_units, nb = ta.lds_node_base, ub = ta.lds_unit_base;
   float4 *cnodes = smem;
   float4 *cprims = smem + nn * 8u;
-  LStack S;
+  const LdsWindow win = {cnodes, cprims, nn, nb, nu, ub};
+  LStack<LT_BLOCK, LT_STACK_LDS> S;
   S.lst = reinterpret_cast<uint32_t *>(cprims + nu) + threadIdx.x;
   S.gst = ta.spill + (size_t)(blockIdx.x * LT_BLOCK + threadIdx.x) * LT_STACK_GLOBAL;
   {
@@ -677,26 +726,7 @@ __global__ __launch_bounds__(LT_BLOCK) void k_trace_lds(DevScene sc, PathBuf pb,
     L.path = 0;
     if (active) lane_start(L, pb, i);
     else L.word = CHILD_EMPTY;
-    while (L.word != CHILD_EMPTY) {
-      if (!(L.word & CHILD_LEAF)) {
-        const uint32_t rel = L.word - nb; /* wraps above nn for nodes below the window */
-        if (rel < nn) lnode_at(L, cnodes + rel * 8u, S);
-        else lnode_at(L, reinterpret_cast<const float4 *>(sc.nodes + L.word), S);
-        if (COUNT) nvisit++;
-      } else {
-        /* one primitive per step: a lane on a leaf of 8 does not hold up the
-         * lanes taking node steps; the leaf word keeps the primitives left
-         * (the same order, so the same hits) */
-        const uint32_t cnt = ((L.word >> 28) & 7u) + 1u;
-        const uint32_t off = L.word & LEAF_OFFSET_MASK;
-        uint32_t units;
-        if (off >= ub && off + PREC_QUAD <= ub + nu) lprim_at(L, sc, cprims + (off - ub), off, any_xform, units);
-        else lprim_at(L, sc, sc.prims + off, off, any_xform, units);
-        if (COUNT) ntest++;
-        if (cnt > 1u) L.word = (L.word & ~(LEAF_OFFSET_MASK | (7u << 28))) | ((cnt - 2u) << 28) | (off + units);
-        else ls_pop(L, S);
-      }
-    }
+    lds_traverse<COUNT>(L, sc, win, S, any_xform, nvisit, ntest);
     if (MODE == 0) {
       uint32_t cls = MC_COUNT;
       if (active) {
@@ -776,7 +806,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu((CO
         }
       }
     }
-    if (MEDIA && active) lane_media(L, sc, pb);
+    if (MEDIA && active) lane_media(L, sc, pb.meta[L.path], pb.rng[L.path]);
     if (MODE == 0) {
       uint32_t cls = MC_COUNT;
       if (active) {
@@ -1198,36 +1228,51 @@ __device__ __forceinline__ V specular_dir(const DevMaterial &m, V d, const Hit &
   return (rnd(s) < rp) ? reflect(d, h.n) : refract(d, h.n, ratio);
 }
 
-/* One shading step of the path at entry i; returns true if the path
- * continues, with its next state in `nx`.  EXT adds what only some scenes
- * need (checker textures, surface coordinates, cone lights); batches without
- * them use the leaner instantiation. */
+/* what shading reads of a path and of the hit of its ray */
+struct ShadeIn {
+  float4 o4, d4;     /* as in PathBuf: .w = root node; the ray's instant */
+  float4 T;          /* throughput */
+  uint64_t rng;
+  uint32_t meta, slot;
+  float t;           /* hit distance */
+  uint32_t hit;      /* hit record */
+};
+
+/* how a shading step ended: the path is over and adds nothing, it goes on, or
+ * it is over with the radiance it found (a path has at most one such vertex,
+ * its last: nothing that emits scatters) */
+#define SH_DEAD 0
+#define SH_GOES_ON 1
+#define SH_LIT 2
+
+/* One shading step of the path `in` (entry i of the wavefront: where its
+ * lobes are); its next state goes to `nx`, emitted radiance to `L`.  EXT adds
+ * what only some scenes need (checker textures, surface coordinates, cone
+ * lights); batches without them use the leaner instantiation.  MC_MISS reads
+ * only T, meta and slot. */
 template <uint32_t CLS, bool GUIDE, bool EXT>
-__device__ __forceinline__ bool shade_path(const DevScene &sc, const PathBuf &pb, uint32_t i, const GuideArgs &ga,
-                                           NextPath &nx) {
-  uint32_t meta = pb.meta[i];
-  const uint32_t slot = pb.slot[i];
+__device__ __forceinline__ int shade_vertex(const DevScene &sc, const PathBuf &pb, const ShadeIn &in, uint32_t i,
+                                            const GuideArgs &ga, NextPath &nx, float4 &L) {
+  const uint32_t meta = in.meta, slot = in.slot;
   uint32_t hero_idx = meta & META_HERO_MASK;
   uint32_t depth = (meta >> META_DEPTH_SHIFT) & META_DEPTH_MASK;
   const DevJob &jb = sc.jobs[meta >> META_JOB_SHIFT];
   int wl[4];
   rotate_wl(hero_idx, wl);
-  float4 T = pb.thr[i];
+  float4 T = in.T;
   if (CLS == MC_MISS) {
     const float *bg = sc.spd + jb.bg_spd;
-    float4 L = pb.rad[slot];
-    L.x += T.x * bg[wl[0] - CLV_LAMBDA_MIN];
-    L.y += T.y * bg[wl[1] - CLV_LAMBDA_MIN];
-    L.z += T.z * bg[wl[2] - CLV_LAMBDA_MIN];
-    L.w += T.w * bg[wl[3] - CLV_LAMBDA_MIN];
-    pb.rad[slot] = L;
+    L.x = T.x * bg[wl[0] - CLV_LAMBDA_MIN];
+    L.y = T.y * bg[wl[1] - CLV_LAMBDA_MIN];
+    L.z = T.z * bg[wl[2] - CLV_LAMBDA_MIN];
+    L.w = T.w * bg[wl[3] - CLV_LAMBDA_MIN];
     if (GUIDE && ga.record && jb.guiding) gd_credit(pb, ga, slot, T.x * bg[wl[0] - CLV_LAMBDA_MIN]);
-    return false;
+    return SH_LIT;
   }
-  float4 o4 = pb.ray_o[i], d4 = pb.ray_d[i];
+  const float4 o4 = in.o4, d4 = in.d4;
   V o = xyz(o4), d = xyz(d4);
-  float t = pb.hit_t[i];
-  Hit h = hit_record<EXT>(sc, pb.hit_p[i], o, d, d4.w, t);
+  const float t = in.t;
+  Hit h = hit_record<EXT>(sc, in.hit, o, d, d4.w, t);
   const DevMaterial &m = sc.mats[h.material];
   if (CLS == MC_LIGHT) { /* DiffuseLight / ConeLight: emit on the front face (inside the cone), never scatter */
     bool lit = h.front;
@@ -1237,17 +1282,16 @@ __device__ __forceinline__ bool shade_path(const DevScene &sc, const PathBuf &pb
     }
     if (lit) {
       const float *e = sc.spd + (EXT ? tex_spd(m, m.emit_spd, h) : m.emit_spd);
-      float4 L = pb.rad[slot];
-      L.x += T.x * e[wl[0] - CLV_LAMBDA_MIN];
-      L.y += T.y * e[wl[1] - CLV_LAMBDA_MIN];
-      L.z += T.z * e[wl[2] - CLV_LAMBDA_MIN];
-      L.w += T.w * e[wl[3] - CLV_LAMBDA_MIN];
-      pb.rad[slot] = L;
+      L.x = T.x * e[wl[0] - CLV_LAMBDA_MIN];
+      L.y = T.y * e[wl[1] - CLV_LAMBDA_MIN];
+      L.z = T.z * e[wl[2] - CLV_LAMBDA_MIN];
+      L.w = T.w * e[wl[3] - CLV_LAMBDA_MIN];
       if (GUIDE && ga.record && jb.guiding) gd_credit(pb, ga, slot, T.x * e[wl[0] - CLV_LAMBDA_MIN]);
+      return SH_LIT;
     }
-    return false;
+    return SH_DEAD;
   }
-  uint64_t s = pb.rng[i];
+  uint64_t s = in.rng;
   /* attenuation (trace.rs:61-70; materials.rs:90-102) */
   const bool wdep = m.thin_film || m.kind == CLV_MAT_DISPERSIVE;
   float att[4];
@@ -1311,7 +1355,7 @@ __device__ __forceinline__ bool shade_path(const DevScene &sc, const PathBuf &pb
     if (guided) cp = alpha * gd_pdf(lob, ndn.x, ndn.y, ndn.z) + (1.0f - alpha) * cp;
     float mis = 0.5f * lp + 0.5f * cp;
     float c2 = dot(h.n, ndn);
-    if (c2 < 0.0f) return false; /* scattering_pdf None: return emitted (0 for Lambertian) */
+    if (c2 < 0.0f) return SH_DEAD; /* scattering_pdf None: return emitted (0 for Lambertian) */
     float spdf = c2 / PI_F;
     T.x = T.x * att[0] * spdf / mis;
     T.y = T.y * att[1] * spdf / mis;
@@ -1351,14 +1395,43 @@ __device__ __forceinline__ bool shade_path(const DevScene &sc, const PathBuf &pb
     T.z *= att[2];
     T.w *= att[3];
   }
-  if (depth + 1u > jb.max_depth) return false; /* trace() at depth > max_depth returns 0 */
+  if (depth + 1u > jb.max_depth) return SH_DEAD; /* trace() at depth > max_depth returns 0 */
   nx.thr = T;
   nx.o = make_float4(h.p.x, h.p.y, h.p.z, o4.w); /* .w: root node of the path's scene */
   nx.d = make_float4(nd.x, nd.y, nd.z, d4.w);    /* .w: the ray's instant stays with the path */
   nx.rng = s;
   nx.meta = (meta & ~(META_DEPTH_MASK << META_DEPTH_SHIFT)) | ((depth + 1u) << META_DEPTH_SHIFT);
   nx.slot = slot;
-  return true;
+  return SH_GOES_ON;
+}
+
+/* the wavefront's shading step: the path at entry i of the path state; returns
+ * true if the path continues */
+template <uint32_t CLS, bool GUIDE, bool EXT>
+__device__ __forceinline__ bool shade_path(const DevScene &sc, const PathBuf &pb, uint32_t i, const GuideArgs &ga,
+                                           NextPath &nx) {
+  ShadeIn in;
+  in.meta = pb.meta[i];
+  in.slot = pb.slot[i];
+  in.T = pb.thr[i];
+  if (CLS != MC_MISS) {
+    in.o4 = pb.ray_o[i];
+    in.d4 = pb.ray_d[i];
+    in.t = pb.hit_t[i];
+    in.hit = pb.hit_p[i];
+    in.rng = pb.rng[i];
+  }
+  float4 L;
+  const int r = shade_vertex<CLS, GUIDE, EXT>(sc, pb, in, i, ga, nx, L);
+  if (r == SH_LIT) {
+    float4 sum = pb.rad[in.slot];
+    sum.x += L.x;
+    sum.y += L.y;
+    sum.z += L.z;
+    sum.w += L.w;
+    pb.rad[in.slot] = sum;
+  }
+  return r == SH_GOES_ON;
 }
 
 /* the plain instance is compiled for 7 waves per SIMD (72 VGPRs, none
@@ -1418,6 +1491,308 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GUIDE ? (EX
   }
 }
 
+/* one sample's XYZ contribution (the estimator of draw_cpu.rs:130-142) from
+ * its radiance at the four wavelengths that follow the hero */
+__device__ __forceinline__ void sample_xyz(const float4 *cie, float4 L, uint32_t hero, float c[3]) {
+  c[0] = c[1] = c[2] = 0.0f;
+  if (L.y == 0.0f && L.z == 0.0f && L.w == 0.0f) {
+    float4 x = cie[hero];
+    c[0] = x.x * L.x;
+    c[1] = x.y * L.x;
+    c[2] = x.z * L.x;
+  } else {
+    float Ls[4] = {L.x, L.y, L.z, L.w};
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      float p = Ls[q];
+      if (isnormal(p) && !signbit(p)) {
+        float4 x = cie[(hero + 100u * (uint32_t)q) % 400u];
+        c[0] += x.x * p / 4.0f;
+        c[1] += x.y * p / 4.0f;
+        c[2] += x.z * p / 4.0f;
+      }
+    }
+  }
+}
+
+/* ------------------------------------------------- whole paths, one launch --- */
+/* A plain render's pass in one launch.  The wavefront above moves every path
+ * through HBM twice per bounce and launches three kernels per bounce, and from
+ * the fourth bounce or so on those launches hold a few percent of the paths.
+ * Here a resident block carries BLOCK paths in registers from the camera to
+ * their end.  One turn of its loop is one bounce:
+ *
+ *   trace    every lane follows its ray (the LDS-cached traversal);
+ *   sort     the block's paths change lanes so that they lie in the order of
+ *            their material classes: per-wave ballots give every path its place,
+ *            its 17 words of state travel through LDS in two rounds.  A wave
+ *            then shades one class, or two where a boundary falls inside it;
+ *   shade    shade_vertex, as the wavefront; a path that ends writes its
+ *            sample's XYZ contribution at its slot (k_resolve_xyz sums the
+ *            samples of a pixel in sample order, so no result depends on which
+ *            block ran a path, or when);
+ *   refill   lanes without a path take the next camera samples.  Misses and
+ *            emitters sort first and always end, so whole waves get fresh
+ *            samples, 64 neighbours in tile order, and stay coherent.
+ *
+ * Samples come from a pass-wide cursor in chunks that a block takes ahead of
+ * need (one global atomic per chunk).  The exchange rounds use the memory of
+ * the traversal stacks, which are empty then.  Every path runs the same
+ * operations on the same stream as in the wavefront: the same image, bit for
+ * bit.
+ *
+ * Bound by VALU issue (88% busy on the sphere field).  Against the wavefront at
+ * its default 4M-path passes, whole calls: sphere field 1920x1080 64 spp 60.5
+ * -> 38.1 ms, prism 1024^2 64 spp 33.1 -> 19.4 ms, Cornell 256^2 16 spp 0.695
+ * -> 0.590 ms; with 64M-path passes the wavefront's sphere field takes 40.3. */
+#define PS_WORDS 9 /* LDS words per lane: stack entries, or one round of the exchange */
+template <int BLOCK, bool EXT, bool MEDIA>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4 : 6))) void k_paths(DevScene sc, GenParams gp,
+                                                                                      PathsArgs pa) {
+  constexpr uint32_t WAVES = BLOCK / 64;
+  static_assert(MC_COUNT * WAVES <= 64, "one lane of a wave per (class, wave) count");
+  extern __shared__ float4 smem[];
+  __shared__ uint32_t cnt[64];   /* paths per (class, wave) */
+  __shared__ uint32_t pool[4];   /* sample ids at hand: [0] base and [1] length of the first range, [2] base of the
+                                    second (pa.chunk long), [3] ids taken since the ranges were set */
+  const LdsWindow win = {smem, smem + pa.lds_nodes * 8u, pa.lds_nodes, pa.lds_node_base, pa.lds_units, pa.lds_unit_base};
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  uint32_t *ex = reinterpret_cast<uint32_t *>(smem + pa.lds_nodes * 8u + pa.lds_units);
+  LStack<BLOCK, PS_WORDS> S;
+  S.lst = ex + tid;
+  S.gst = pa.spill + (size_t)(blockIdx.x * BLOCK + tid) * (STACK_TOTAL - PS_WORDS);
+  {
+    const float4 *gn = reinterpret_cast<const float4 *>(sc.nodes + win.nb);
+    for (uint32_t k = tid; k < win.nn * 8u; k += BLOCK) smem[k] = gn[k];
+    for (uint32_t k = tid; k < win.nu; k += BLOCK) smem[win.nn * 8u + k] = sc.prims[win.ub + k];
+    if (tid == 0) {
+      pool[0] = 0u;
+      pool[1] = 0u;
+      pool[2] = 0u;
+      pool[3] = pa.chunk; /* both ranges used up */
+    }
+  }
+  __syncthreads();
+  const uint32_t n = gp.paths;
+  const bool any_xform = sc.has_xforms != 0;
+  const uint64_t below = (1ull << lane) - 1ull;
+  uint32_t rays = 0, unused = 0;
+  bool exhausted = false; /* thread 0: the pass-wide cursor has passed the last sample */
+  /* the lane's path */
+  ShadeIn ps;
+  ps.T = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+  ps.rng = 0;
+  ps.meta = 0;
+  ps.slot = tid < pa.first ? blockIdx.x * pa.first + tid : 0xFFFFFFFFu;
+  V o = mk(0.0f, 0.0f, 0.0f), d = o;
+  float time = 0.0f;
+  bool alive = ps.slot < n;
+  if (alive) ps.meta = camera_sample(sc, gp, ps.slot, o, d, time, ps.rng);
+  for (;;) {
+    /* trace */
+    uint32_t cls = MC_COUNT;
+    Lane L;
+    L.tb = FLT_MAX;
+    L.best = MISS_WORD;
+    rays += (uint32_t)__popcll(__ballot(alive));
+    if (alive) {
+      lane_start_ray(L, o, d, time, sc.jobs[ps.meta >> META_JOB_SHIFT].root);
+      lds_traverse<false>(L, sc, win, S, any_xform, unused, unused);
+      if (MEDIA) lane_media(L, sc, ps.meta, ps.rng);
+      cls = L.best != MISS_WORD ? sc.mats[sc.info[as_u(sc.prims[L.best + 1u].w)].material].mclass : MC_MISS;
+    }
+    /* each path's place in class order */
+    uint32_t rank = 0;
+#pragma unroll
+    for (uint32_t c = 0; c < MC_COUNT; c++) {
+      const uint64_t m = __ballot(cls == c);
+      if (lane == 0) cnt[c * WAVES + wave] = (uint32_t)__popcll(m);
+      if (cls == c) rank = (uint32_t)__popcll(m & below);
+    }
+    __syncthreads();
+    if (tid == 0 && pool[3] >= pool[1]) { /* the first range is used up: the rest of the second follows, and a new one */
+      const uint32_t over = pool[3] - pool[1];
+      pool[0] = pool[2] + over;
+      pool[1] = pa.chunk - over;
+      pool[3] = 0u;
+      uint32_t base = n;
+      if (!exhausted) base = atomicAdd(pa.next, pa.chunk);
+      exhausted = base >= n;
+      pool[2] = base;
+    }
+    uint32_t sum = lane < MC_COUNT * WAVES ? cnt[lane] : 0u;
+    const uint32_t own = sum;
+#pragma unroll
+    for (uint32_t k = 1; k < 64u; k <<= 1) {
+      const uint32_t up = __shfl_up(sum, k);
+      if (lane >= k) sum += up;
+    }
+    const uint32_t total = __builtin_amdgcn_readlane(sum, 63);
+    if (total == 0u) break; /* the same in every wave: nothing left to trace, and the last refill found no sample */
+    const uint32_t excl = sum - own;
+    uint32_t start[MC_COUNT];
+#pragma unroll
+    for (uint32_t c = 1; c < MC_COUNT; c++) start[c] = __builtin_amdgcn_readlane(excl, c * WAVES);
+    const uint32_t dest = __shfl(excl, (int)(min(cls, MC_COUNT - 1u) * WAVES + wave)) + rank;
+    /* the paths change lanes */
+    uint32_t *w = ex + dest;
+    const uint32_t *r = ex + tid;
+    const bool moves = cls < MC_COUNT;
+    alive = tid < total;
+    if (moves) {
+      lds_store(w, as_u(o.x));
+      lds_store(w + BLOCK, as_u(o.y));
+      lds_store(w + 2 * BLOCK, as_u(o.z));
+      lds_store(w + 3 * BLOCK, as_u(d.x));
+      lds_store(w + 4 * BLOCK, as_u(d.y));
+      lds_store(w + 5 * BLOCK, as_u(d.z));
+      lds_store(w + 6 * BLOCK, as_u(time));
+      lds_store(w + 7 * BLOCK, as_u(L.tb));
+      lds_store(w + 8 * BLOCK, L.best);
+    }
+    __syncthreads();
+    if (alive) {
+      o = mk(__uint_as_float(lds_load(r)), __uint_as_float(lds_load(r + BLOCK)), __uint_as_float(lds_load(r + 2 * BLOCK)));
+      d = mk(__uint_as_float(lds_load(r + 3 * BLOCK)), __uint_as_float(lds_load(r + 4 * BLOCK)),
+             __uint_as_float(lds_load(r + 5 * BLOCK)));
+      time = __uint_as_float(lds_load(r + 6 * BLOCK));
+      ps.t = __uint_as_float(lds_load(r + 7 * BLOCK));
+      ps.hit = lds_load(r + 8 * BLOCK);
+    }
+    __syncthreads();
+    if (moves) {
+      lds_store(w, as_u(ps.T.x));
+      lds_store(w + BLOCK, as_u(ps.T.y));
+      lds_store(w + 2 * BLOCK, as_u(ps.T.z));
+      lds_store(w + 3 * BLOCK, as_u(ps.T.w));
+      lds_store(w + 4 * BLOCK, (uint32_t)ps.rng);
+      lds_store(w + 5 * BLOCK, (uint32_t)(ps.rng >> 32));
+      lds_store(w + 6 * BLOCK, ps.meta);
+      lds_store(w + 7 * BLOCK, ps.slot);
+    }
+    __syncthreads();
+    if (alive) {
+      ps.T = make_float4(__uint_as_float(lds_load(r)), __uint_as_float(lds_load(r + BLOCK)),
+                         __uint_as_float(lds_load(r + 2 * BLOCK)), __uint_as_float(lds_load(r + 3 * BLOCK)));
+      ps.rng = (uint64_t)lds_load(r + 4 * BLOCK) | ((uint64_t)lds_load(r + 5 * BLOCK) << 32);
+      ps.meta = lds_load(r + 6 * BLOCK);
+      ps.slot = lds_load(r + 7 * BLOCK);
+    }
+    __syncthreads(); /* the exchange is over: the memory is the stacks' again */
+    /* shade */
+    if (alive) {
+      ps.o4 = make_float4(o.x, o.y, o.z, 0.0f);
+      ps.d4 = make_float4(d.x, d.y, d.z, time);
+      uint32_t c = 0;
+#pragma unroll
+      for (uint32_t k = 1; k < MC_COUNT; k++) c += tid >= start[k] ? 1u : 0u;
+      NextPath nx;
+      float4 lit = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      int end;
+      const PathBuf pb = PathBuf();
+      const GuideArgs ga = GuideArgs();
+      switch (c) {
+        case MC_MISS: end = shade_vertex<MC_MISS, false, EXT>(sc, pb, ps, 0u, ga, nx, lit); break;
+        case MC_LIGHT: end = shade_vertex<MC_LIGHT, false, EXT>(sc, pb, ps, 0u, ga, nx, lit); break;
+        case MC_LAMBERTIAN: end = shade_vertex<MC_LAMBERTIAN, false, EXT>(sc, pb, ps, 0u, ga, nx, lit); break;
+        case MC_METAL: end = shade_vertex<MC_METAL, false, EXT>(sc, pb, ps, 0u, ga, nx, lit); break;
+        default: end = shade_vertex<MC_GLASS, false, EXT>(sc, pb, ps, 0u, ga, nx, lit); break;
+      }
+      if (end == SH_GOES_ON) {
+        o = mk(nx.o.x, nx.o.y, nx.o.z);
+        d = mk(nx.d.x, nx.d.y, nx.d.z);
+        ps.T = nx.thr;
+        ps.rng = nx.rng;
+        ps.meta = nx.meta;
+      } else {
+        alive = false;
+        F3 c3 = {0.0f, 0.0f, 0.0f};
+        if (end == SH_LIT) sample_xyz(pa.cie, lit, ps.meta & META_HERO_MASK, &c3.x);
+        pa.res[ps.slot] = c3;
+      }
+    }
+    /* refill */
+    const uint64_t idle = __ballot(!alive);
+    if (idle) {
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(&pool[3], (uint32_t)__popcll(idle));
+      base = __builtin_amdgcn_readfirstlane(base);
+      if (!alive) {
+        const uint32_t k = base + (uint32_t)__popcll(idle & below), len = pool[1];
+        ps.slot = k < len ? pool[0] + k : pool[2] + (k - len);
+        alive = ps.slot < n;
+        if (alive) {
+          ps.meta = camera_sample(sc, gp, ps.slot, o, d, time, ps.rng);
+          ps.T = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+        }
+      }
+    }
+  }
+  if (lane == 0 && rays) atomicAdd(pa.stats + 2, (unsigned long long)rays);
+}
+
+/* the counters of a pass of k_paths: the sample cursor starts behind the
+ * blocks' first samples; with `stats`, the render's counters too */
+__global__ void k_paths_begin(uint32_t *next, uint32_t value, unsigned long long *stats) {
+  if (threadIdx.x == 0) *next = value;
+  if (stats && threadIdx.x < 8u) stats[threadIdx.x] = 0ull;
+}
+
+/* the per-pixel sums of a pass of k_paths, in sample order, one thread per
+ * (pass item, pixel).  A job whose samples are all in one pass goes straight
+ * to its means; sums of others wait in the accumulators between passes.  The
+ * second moments are summed only where some job returns them. */
+__global__ __launch_bounds__(256) void k_resolve_xyz(ResolveParams rp, const F3 *res, float *out, float *out_sq) {
+  for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < rp.threads; g += gridDim.x * blockDim.x) {
+    const DevItem it = rp.items[find_entry(rp.items, rp.n_items, g, &DevItem::res_base)];
+    const uint32_t q = g - it.res_base; /* slot within a sample */
+    const DevJob &jb = rp.jobs[it.job];
+    const uint32_t o = it.order ? tile_pixel(q, jb.width, jb.height) : q;
+    const bool fp64 = jb.fp64 != 0;
+    const uint32_t a = 3u * (jb.pixel_base + o);
+    float a32[3] = {0.0f, 0.0f, 0.0f};
+    double a64[3] = {0.0, 0.0, 0.0}, sq[3] = {0.0, 0.0, 0.0};
+    if (!(it.flags & ITEM_FIRST))
+      for (int k = 0; k < 3; k++) {
+        sq[k] = rp.acc_sq[a + k];
+        if (fp64) a64[k] = rp.acc64[a + k];
+        else a32[k] = rp.acc32[a + k];
+      }
+    auto add = [&](F3 c) {
+      const float v[3] = {c.x, c.y, c.z};
+      for (int k = 0; k < 3; k++) {
+        if (fp64) a64[k] += (double)v[k];
+        else a32[k] += v[k];
+        if (out_sq) sq[k] += (double)v[k] * (double)v[k];
+      }
+    };
+    /* 8 samples are read before any is added, so that their loads are in
+     * flight together */
+    const F3 *p = res + it.path_base + q;
+    uint32_t j = 0;
+    for (; j + 8u <= it.samples; j += 8u) {
+      F3 b[8];
+#pragma unroll
+      for (uint32_t u = 0; u < 8u; u++) b[u] = p[(size_t)(j + u) * it.pixels];
+#pragma unroll
+      for (uint32_t u = 0; u < 8u; u++) add(b[u]);
+    }
+    for (; j < it.samples; j++) add(p[(size_t)j * it.pixels]);
+    if (it.flags & ITEM_LAST) {
+      for (int k = 0; k < 3; k++) {
+        out[a + k] = fp64 ? (float)(a64[k] / (double)jb.spp) : a32[k] / (float)jb.spp;
+        if (out_sq) out_sq[a + k] = (float)(sq[k] / (double)jb.spp);
+      }
+    } else {
+      for (int k = 0; k < 3; k++) {
+        rp.acc_sq[a + k] = sq[k];
+        if (fp64) rp.acc64[a + k] = a64[k];
+        else rp.acc32[a + k] = a32[k];
+      }
+    }
+  }
+}
+
 /* The tail of a pass.  From bounce `tail_depth` on, few paths are left and
  * each further bounce would cost a traversal and a shading launch for a
  * handful of rays, so one launch finishes them: every thread traces and
@@ -1452,7 +1827,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) void k_tail(DevScene sc, PathBuf pb, T
           lane_pop(L, lst, gst);
         }
       }
-      if (MEDIA) lane_media(L, sc, pb);
+      if (MEDIA) lane_media(L, sc, pb.meta[L.path], pb.rng[L.path]);
       pb.hit_t[i] = L.tb;
       pb.hit_p[i] = L.best;
       const uint32_t cls = L.best != MISS_WORD ? sc.mats[sc.info[as_u(sc.prims[L.best + 1u].w)].material].mclass : MC_MISS;
@@ -1816,28 +2191,9 @@ __global__ __launch_bounds__(256) void k_resolve(PathBuf pb, ResolveParams rp, c
       if (fp64) a64[k] = rp.acc64[a + k];
       else a32[k] = rp.acc32[a + k];
     }
-    /* one sample's XYZ contribution (the estimator of draw_cpu.rs:130-142),
-     * added to the pixel's sums in sample order */
     auto add = [&](float4 L, uint32_t hero) {
-      float c[3] = {0.0f, 0.0f, 0.0f};
-      if (L.y == 0.0f && L.z == 0.0f && L.w == 0.0f) {
-        float4 x = cie[hero];
-        c[0] = x.x * L.x;
-        c[1] = x.y * L.x;
-        c[2] = x.z * L.x;
-      } else {
-        float Ls[4] = {L.x, L.y, L.z, L.w};
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          float p = Ls[q];
-          if (isnormal(p) && !signbit(p)) {
-            float4 x = cie[(hero + 100u * (uint32_t)q) % 400u];
-            c[0] += x.x * p / 4.0f;
-            c[1] += x.y * p / 4.0f;
-            c[2] += x.z * p / 4.0f;
-          }
-        }
-      }
+      float c[3];
+      sample_xyz(cie, L, hero, c);
       for (int k = 0; k < 3; k++) {
         if (fp64) a64[k] += (double)c[k];
         else a32[k] += c[k];
@@ -2135,6 +2491,37 @@ void launch_guide_infer(hipStream_t st, const DevScene &sc, const PathBuf &pb, c
                         const uint32_t *queue, const uint32_t *count, uint32_t max_paths, uint32_t resident) {
   hipLaunchKernelGGL(k_guide_infer, dim3(std::min(resident, grid_for(max_paths, GI_BLOCK, 1u << 30))), dim3(GI_BLOCK), 0,
                      st, sc, pb, ga, queue, count);
+}
+
+/* k_paths: block size, LDS of a window, resident blocks and spill words */
+#define PS_BLOCK 768
+uint32_t paths_block() { return PS_BLOCK; }
+size_t paths_lds_bytes(uint32_t nodes, uint32_t units) {
+  return (size_t)nodes * sizeof(Bvh4Node) + (size_t)units * 16u + (size_t)PS_WORDS * PS_BLOCK * 4u;
+}
+size_t paths_spill_words(uint32_t blocks) { return (size_t)blocks * PS_BLOCK * (STACK_TOTAL - PS_WORDS); }
+
+typedef void (*paths_fn)(DevScene, GenParams, PathsArgs);
+static paths_fn paths_instance(bool ext, bool media) {
+  if (media) return k_paths<PS_BLOCK, true, true>; /* a medium's phase function is an extended material */
+  return ext ? k_paths<PS_BLOCK, true, false> : k_paths<PS_BLOCK, false, false>;
+}
+uint32_t paths_grid_blocks(size_t lds_bytes, bool ext, bool media) {
+  int dev = 0, cus = 0, per_cu = 0;
+  (void)hipGetDevice(&dev);
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(paths_instance(ext, media)),
+                                                     PS_BLOCK, lds_bytes);
+  return (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, cus);
+}
+void launch_paths(hipStream_t st, const DevScene &sc, const GenParams &gp, const PathsArgs &pa, uint32_t blocks,
+                  size_t lds_bytes, bool begin) {
+  hipLaunchKernelGGL(k_paths_begin, dim3(1), dim3(64), 0, st, pa.next, blocks * pa.first, begin ? pa.stats : nullptr);
+  hipLaunchKernelGGL(paths_instance(sc.has_ext != 0, sc.has_media != 0), dim3(blocks), dim3(PS_BLOCK), lds_bytes, st, sc,
+                     gp, pa);
+}
+void launch_resolve_xyz(hipStream_t st, const ResolveParams &rp, const F3 *res, float *out, float *out_sq) {
+  hipLaunchKernelGGL(k_resolve_xyz, dim3(grid_for(rp.threads, 256, 65535)), dim3(256), 0, st, rp, res, out, out_sq);
 }
 
 void launch_resolve(hipStream_t st, const PathBuf &pb, const ResolveParams &rp, const float4 *cie) {

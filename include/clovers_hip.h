@@ -343,10 +343,13 @@ typedef enum {
   CLV_TRACE_SIMPLE = 0,     /* one ray per thread, 256-thread blocks, stack top in LDS */
   CLV_TRACE_PERSISTENT = 1, /* persistent waves refilling lanes from a work counter */
   CLV_TRACE_WW = 2,         /* one ray per thread, node steps and leaf steps in separate loops */
-  CLV_TRACE_LDS_CACHED = 3  /* 768-thread blocks, top of the BVH and leading records cached in LDS */
+  CLV_TRACE_LDS_CACHED = 3  /* 768-thread blocks, top of the BVH and leading records cached in LDS; renders without
+                               guided jobs run every path from the camera to its end in one launch per pass */
 } clv_trace_kernel;
 typedef struct {
-  uint32_t target_paths;    /* paths in flight per wavefront pass (queue and path-state capacity) */
+  uint32_t target_paths;    /* samples per wavefront pass (queue and path-state capacity).  At the default, 2^22, a
+                               pass that runs whole paths in one launch (CLV_TRACE_LDS_CACHED, no guided job, no
+                               CLV_FLAG_TIME_KERNELS or _COUNT) holds up to 2^27: it needs 12 bytes per sample */
   uint32_t trace_kernel;    /* clv_trace_kernel */
   uint32_t lds_bytes;       /* dynamic LDS per block of CLV_TRACE_LDS_CACHED (<= 64512) */
   uint32_t shade_grid_cap;  /* largest grid of the shading kernel, in 256-thread blocks (the library also caps it
