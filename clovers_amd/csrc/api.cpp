@@ -258,6 +258,7 @@ struct TraceGeom {
   uint32_t blocks = 0;
   size_t lds_bytes = 0;
   uint32_t lds_node_base = 0, lds_nodes = 0, lds_unit_base = 0, lds_units = 0;
+  uint32_t full = 0; /* whole-path launches: the scene of every job is in the window, whole */
 };
 
 /* Whole paths in one launch per pass (k_paths) wherever the LDS-cached
@@ -273,17 +274,17 @@ bool whole_paths(const clv_ctx *c, bool any_guide, uint32_t flags) {
 #define DEFAULT_TARGET_PATHS (1u << 22)
 #define WHOLE_TARGET_PATHS (1u << 27)
 
-clv_status paths_geometry(clv_ctx *c, const SceneRes *s, bool ext, bool media, TraceGeom *g) {
-  const size_t stack = paths_lds_bytes(0, 0);
-  size_t budget = c->lds_block_bytes > stack ? c->lds_block_bytes - stack : 0;
-  g->lds_node_base = s->base.nodes;
-  g->lds_unit_base = s->base.units;
-  g->lds_nodes = (uint32_t)std::min<size_t>(s->n_nodes, budget / sizeof(Bvh4Node));
-  budget -= (size_t)g->lds_nodes * sizeof(Bvh4Node);
-  g->lds_units = (uint32_t)std::min<size_t>(s->prim_units, budget / 16u);
-  g->lds_bytes = paths_lds_bytes(g->lds_nodes, g->lds_units);
-  g->blocks = paths_grid_blocks(g->lds_bytes, ext, media);
-  return ensure_spill(c, paths_spill_words(g->blocks));
+clv_status paths_geometry(clv_ctx *c, const SceneRes *s, bool one_scene, const DevScene &ds, TraceGeom *g) {
+  g->full = one_scene && paths_lds_bytes(true, s->n_nodes, s->prim_units) <= c->lds_block_bytes;
+  if (g->full) {
+    g->lds_node_base = s->base.nodes;
+    g->lds_unit_base = s->base.units;
+    g->lds_nodes = s->n_nodes;
+    g->lds_units = s->prim_units;
+  }
+  g->lds_bytes = paths_lds_bytes(g->full != 0, g->lds_nodes, g->lds_units);
+  g->blocks = paths_grid_blocks(g->lds_bytes, ds, g->full != 0);
+  return ensure_spill(c, paths_spill_words(g->full != 0, g->blocks));
 }
 
 /* the traversal kernel a batch runs: the tuned one, or the plain one when a
@@ -717,7 +718,13 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
     if ((uint64_t)dj[k].width * dj[k].height * dj[k].spp > (uint64_t)dj[big].width * dj[big].height * dj[big].spp) big = k;
   TraceGeom geom;
   const int variant = trace_variant_for(c, any_media);
-  if (whole) CHK(paths_geometry(c, sres[big], any_ext, any_media, &geom));
+  bool one_scene = true;
+  for (uint32_t k = 1; k < n; k++) one_scene = one_scene && sres[k] == sres[0];
+  DevScene ds = arena_view(c);
+  ds.has_xforms = any_xform ? 1u : 0u;
+  ds.has_ext = any_ext ? 1u : 0u;
+  ds.has_media = any_media ? 1u : 0u;
+  if (whole) CHK(paths_geometry(c, sres[big], one_scene, ds, &geom));
   else CHK(trace_geometry(c, sres[big], pl.max_paths, &geom, variant));
   /* the tail launch (k_tail): the resident grid of the plain traversal, never with per-launch timing or
    * counting (those measure the wavefront traversal) */
@@ -730,10 +737,6 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
   HIPCHK(c, hipMemcpyAsync(c->jobs, dj.data(), n * sizeof(DevJob), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->items, pl.items.data(), pl.items.size() * sizeof(DevItem), hipMemcpyHostToDevice,
                            c->stream));
-  DevScene ds = arena_view(c);
-  ds.has_xforms = any_xform ? 1u : 0u;
-  ds.has_ext = any_ext ? 1u : 0u;
-  ds.has_media = any_media ? 1u : 0u;
   const bool timing = (flags & CLV_FLAG_TIME_KERNELS) != 0;
   const bool counting = (flags & CLV_FLAG_COUNT) != 0;
   uint32_t extends = 0;
@@ -804,8 +807,9 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
       pa.lds_nodes = geom.lds_nodes;
       pa.lds_unit_base = geom.lds_unit_base;
       pa.lds_units = geom.lds_units;
+      pa.full = geom.full;
       /* a pass smaller than the grid is spread over all its blocks */
-      const uint32_t block = paths_block();
+      const uint32_t block = paths_block(geom.full != 0);
       const uint32_t blocks = std::min(geom.blocks, (gp.paths + 63u) / 64u);
       pa.first = (uint32_t)std::min<uint64_t>(block, ((uint64_t)gp.paths + 64ull * blocks - 1u) / (64ull * blocks) * 64ull);
       pa.chunk = block;

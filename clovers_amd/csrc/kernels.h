@@ -134,6 +134,7 @@ struct PathsArgs {
   const float4 *cie;
   uint32_t lds_node_base, lds_nodes, lds_unit_base, lds_units; /* as TraceArgs */
   uint32_t first;              /* samples a block starts with: [block * first, + first) */
+  uint32_t full;               /* every ray's scene is the one in the window, and it is in there whole */
   uint32_t chunk;              /* samples a block takes from the cursor at a time, at least the block size */
 };
 
@@ -237,13 +238,13 @@ void launch_guide_step(hipStream_t st, const GuideRec *rec, const float *recL, c
 void launch_guide_halves(hipStream_t st, const float *P, _Float16 *Wh);
 void launch_guide_eval(hipStream_t st, const float *in, uint32_t n, const _Float16 *Wh, const float *P, float *raw,
                        float *lobes);
-/* whole paths in one launch (k_paths): its block size, dynamic LDS for a
- * window of the scene, resident blocks, spill words of a grid; `begin` also
- * clears the render's counters */
-uint32_t paths_block();
-size_t paths_lds_bytes(uint32_t nodes, uint32_t units);
-uint32_t paths_grid_blocks(size_t lds_bytes, bool ext, bool media);
-size_t paths_spill_words(uint32_t blocks);
+/* whole paths in one launch (k_paths), from a scene in LDS (full) or in
+ * memory: block size, dynamic LDS, resident blocks, spill words of a grid;
+ * `begin` also clears the render's counters */
+uint32_t paths_block(bool full);
+size_t paths_lds_bytes(bool full, uint32_t nodes, uint32_t units);
+uint32_t paths_grid_blocks(size_t lds_bytes, const DevScene &sc, bool full);
+size_t paths_spill_words(bool full, uint32_t blocks);
 void launch_paths(hipStream_t st, const DevScene &sc, const GenParams &gp, const PathsArgs &pa, uint32_t blocks,
                   size_t lds_bytes, bool begin);
 void launch_resolve_xyz(hipStream_t st, const ResolveParams &rp, const F3 *res, float *out, float *out_sq);

@@ -370,7 +370,8 @@ __device__ __forceinline__ void slab4(const Lane &L, const float4 *nf, float tn[
  * share one address (immediate offsets) and no per-lane row offsets stay in
  * registers; on the 1M-triangle mesh, whose traversal waits on node fetches,
  * the row-picked form was 1% slower */
-__device__ __forceinline__ void slab4_minmax(const Lane &L, const float4 *nf, const uint32_t cw[4], float tn[4]) {
+template <class RAY>
+__device__ __forceinline__ void slab4_minmax(const RAY &L, const float4 *nf, const uint32_t cw[4], float tn[4]) {
   const float4 lx = nf[0], hx = nf[1], ly = nf[2], hy = nf[3], lz = nf[4], hz = nf[5];
   const float lxa[4] = {lx.x, lx.y, lx.z, lx.w}, hxa[4] = {hx.x, hx.y, hx.z, hx.w};
   const float lya[4] = {ly.x, ly.y, ly.z, ly.w}, hya[4] = {hy.x, hy.y, hy.z, hy.w};
@@ -946,11 +947,11 @@ __device__ __forceinline__ void sphere_uv(V p, V c, float r, float &u, float &v)
  * chain forward, evaluate the primitive's record, then unwind RotateY
  * (rotate.rs:115-158: rotate back, set_face_normal with the rotated ray) and
  * Translate (translate.rs:68-77: shift back, set_face_normal with the moved ray). */
-template <bool UV>
+template <bool UV, bool XF = true>
 __device__ Hit hit_record(const DevScene &sc, uint32_t off, V o, V d, float time, float t) {
   const float4 *rec = sc.prims + off;
   float4 f0 = rec[0], f1 = rec[1];
-  uint32_t hdr = as_u(f0.w), type = hdr & PT_TYPE_MASK, xf = hdr >> PT_XF_SHIFT;
+  uint32_t hdr = as_u(f0.w), type = hdr & PT_TYPE_MASK, xf = XF ? hdr >> PT_XF_SHIFT : 0u;
   Hit h;
   h.material = sc.info[as_u(f1.w)].material;
   h.u = h.v = 0.0f;
@@ -1248,9 +1249,9 @@ struct ShadeIn {
 /* One shading step of the path `in` (entry i of the wavefront: where its
  * lobes are); its next state goes to `nx`, emitted radiance to `L`.  EXT adds
  * what only some scenes need (checker textures, surface coordinates, cone
- * lights); batches without them use the leaner instantiation.  MC_MISS reads
- * only T, meta and slot. */
-template <uint32_t CLS, bool GUIDE, bool EXT>
+ * lights), XF instance chains; batches without them use the leaner
+ * instantiations.  MC_MISS reads only T, meta and slot. */
+template <uint32_t CLS, bool GUIDE, bool EXT, bool XF>
 __device__ __forceinline__ int shade_vertex(const DevScene &sc, const PathBuf &pb, const ShadeIn &in, uint32_t i,
                                             const GuideArgs &ga, NextPath &nx, float4 &L) {
   const uint32_t meta = in.meta, slot = in.slot;
@@ -1272,7 +1273,7 @@ __device__ __forceinline__ int shade_vertex(const DevScene &sc, const PathBuf &p
   const float4 o4 = in.o4, d4 = in.d4;
   V o = xyz(o4), d = xyz(d4);
   const float t = in.t;
-  Hit h = hit_record<EXT>(sc, in.hit, o, d, d4.w, t);
+  Hit h = hit_record<EXT, XF>(sc, in.hit, o, d, d4.w, t);
   const DevMaterial &m = sc.mats[h.material];
   if (CLS == MC_LIGHT) { /* DiffuseLight / ConeLight: emit on the front face (inside the cone), never scatter */
     bool lit = h.front;
@@ -1422,7 +1423,7 @@ __device__ __forceinline__ bool shade_path(const DevScene &sc, const PathBuf &pb
     in.rng = pb.rng[i];
   }
   float4 L;
-  const int r = shade_vertex<CLS, GUIDE, EXT>(sc, pb, in, i, ga, nx, L);
+  const int r = shade_vertex<CLS, GUIDE, EXT, true>(sc, pb, in, i, ga, nx, L);
   if (r == SH_LIT) {
     float4 sum = pb.rad[in.slot];
     sum.x += L.x;
@@ -1515,6 +1516,230 @@ __device__ __forceinline__ void sample_xyz(const float4 *cie, float4 L, uint32_t
   }
 }
 
+/* -------------------------------------- traversal of the whole-path kernel --- */
+typedef __attribute__((address_space(3))) float4 lds_f4;
+/* the 32-bit LDS address of a shared-memory pointer */
+__device__ __forceinline__ uint32_t lds_addr(const void *p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p; }
+__device__ __forceinline__ uint32_t lds_ld(uint32_t a) { return *(const lds_u32 *)(uintptr_t)a; }
+__device__ __forceinline__ void lds_st(uint32_t a, uint32_t v) { *(lds_u32 *)(uintptr_t)a = v; }
+__device__ __forceinline__ float4 lds_ld4(uint32_t a) {
+  const __attribute__((address_space(3))) float *p = (const __attribute__((address_space(3))) float *)(uintptr_t)a;
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  const f4 v = *(const __attribute__((address_space(3))) f4 *)p;
+  return make_float4(v.x, v.y, v.z, v.w);
+}
+
+/* A lane's ray on its way through the tree.  FULL: the scene lies in the
+ * block's LDS and its child words were rewritten for it (interior: byte offset
+ * of the node, leaf: unit offset in the window); else they are arena words. */
+struct Trav {
+  V o, d, inv, oi;
+  uint32_t rx, ry, rz;   /* byte offset of the near-plane row per axis */
+  float tb, time;
+  float a, ra;           /* d.d and its reciprocal (sphere tests of rays that are not transformed) */
+  uint32_t best, word;
+  uint32_t sp;           /* LDS address of the next free stack entry; entry 0 holds CHILD_EMPTY */
+};
+
+/* n / a, correctly rounded, from ra = RN(1/a): a quotient and two residual
+ * corrections (Markstein 1990, "Computation of elementary functions on the IBM
+ * RISC System/6000 processor"), half the operations of a full division.  For
+ * 1/2 < a < 2 and quotients far from the ends of the range; elsewhere the
+ * result is still outside every [tmin, tmax] it is compared with, or NaN. */
+__device__ __forceinline__ float div_by(float n, float a, float ra) {
+  float q = n * ra;
+  q = fmaf(fmaf(-a, q, n), ra, q);
+  return fmaf(fmaf(-a, q, n), ra, q);
+}
+
+/* sphere_t for the ray's own d.d and its reciprocal */
+__device__ __forceinline__ bool sphere_hit(V c, float r, const Trav &L, float tmin, float tmax, float &t) {
+  V oc = L.o - c;
+  float half_b = dot(oc, L.d);
+  float cc = dot(oc, oc) - r * r;
+  float disc = half_b * half_b - L.a * cc;
+  if (!(disc > 0.0f)) return false;
+  float root = sqrtf(disc);
+  float t0 = div_by(-half_b - root, L.a, L.ra);
+  if (t0 < tmax && t0 > tmin) { t = t0; return true; }
+  float t1 = div_by(-half_b + root, L.a, L.ra);
+  if (t1 < tmax && t1 > tmin) { t = t1; return true; }
+  return false;
+}
+
+template <int BLOCK, int DEPTH>
+struct TravStack {
+  uint32_t lst;      /* LDS address of the lane's entry 0; entries are BLOCK words apart */
+  uint32_t *spill;   /* this block's slices */
+  static constexpr uint32_t STRIDE = 4u * BLOCK, N = DEPTH;
+  __device__ __forceinline__ uint32_t *deep(uint32_t e) const {
+    return spill + (size_t)threadIdx.x * (STACK_TOTAL - DEPTH) + (e - DEPTH);
+  }
+  __device__ __forceinline__ void start(Trav &L) const {
+    lds_st(lst, CHILD_EMPTY);
+    L.sp = lst + STRIDE;
+  }
+  /* the children at distances tn[1..3] that were hit (sorted: hits first), far to near */
+  __device__ __forceinline__ void push3(Trav &L, const uint32_t cw[4], const float tn[4]) const {
+    if (__any(L.sp > lst + (DEPTH - 3) * STRIDE)) { /* some lane may leave its LDS part */
+#pragma unroll
+      for (int k = 3; k >= 1; k--)
+        if (tn[k] < FLT_MAX) {
+          const uint32_t e = (L.sp - lst) / STRIDE;
+          if (e < DEPTH) lds_st(L.sp, cw[k]);
+          else if (e < STACK_TOTAL) *deep(e) = cw[k]; /* always: the host bounds the BVH depth */
+          L.sp += STRIDE;
+        }
+    } else { /* stores without branches; the stack grows past the ones that were hit */
+#pragma unroll
+      for (int k = 3; k >= 1; k--) {
+        lds_st(L.sp, cw[k]);
+        L.sp += tn[k] < FLT_MAX ? STRIDE : 0u;
+      }
+    }
+  }
+  __device__ __forceinline__ void pop(Trav &L) const {
+    L.sp -= STRIDE;
+    if (__any(L.sp > lst + (DEPTH - 1) * STRIDE)) {
+      const uint32_t e = (L.sp - lst) / STRIDE;
+      L.word = e < DEPTH ? lds_ld(L.sp) : *deep(e);
+    } else {
+      L.word = lds_ld(L.sp);
+    }
+  }
+};
+
+#define TRAV_SORT4(tn, cw)                                                \
+  do {                                                                    \
+    auto swp = [&](int a, int b) {                                        \
+      const bool s_ = tn[b] < tn[a];                                      \
+      const float ta_ = tn[a], tb_ = tn[b];                               \
+      const uint32_t ca_ = cw[a], cb_ = cw[b];                            \
+      tn[a] = s_ ? tb_ : ta_; tn[b] = s_ ? ta_ : tb_;                     \
+      cw[a] = s_ ? cb_ : ca_; cw[b] = s_ ? ca_ : cb_;                     \
+    };                                                                    \
+    swp(0, 1); swp(2, 3); swp(0, 2); swp(1, 3); swp(1, 2);                \
+  } while (0)
+
+/* after the slab tests of a node: on to the nearest child hit, the others on the stack */
+template <class STACK>
+__device__ __forceinline__ void trav_next(Trav &L, float tn[4], uint32_t cw[4], const STACK &S) {
+  TRAV_SORT4(tn, cw);
+  S.push3(L, cw, tn);
+  if (tn[0] < FLT_MAX) L.word = cw[0];
+  else S.pop(L);
+}
+
+/* one node of the window, at LDS address p: near and far planes per axis picked by the ray's signs (slab4) */
+template <class STACK>
+__device__ __forceinline__ void trav_node_lds(Trav &L, uint32_t p, const STACK &S) {
+  const uint32_t px = p + L.rx, py = p + L.ry, pz = p + L.rz;
+  const float4 cf = lds_ld4(p + 96u);
+  const float4 nx = lds_ld4(px), fx = lds_ld4(px ^ 16u), ny = lds_ld4(py), fy = lds_ld4(py ^ 16u), nz = lds_ld4(pz),
+               fz = lds_ld4(pz ^ 16u);
+  const float nxa[4] = {nx.x, nx.y, nx.z, nx.w}, fxa[4] = {fx.x, fx.y, fx.z, fx.w};
+  const float nya[4] = {ny.x, ny.y, ny.z, ny.w}, fya[4] = {fy.x, fy.y, fy.z, fy.w};
+  const float nza[4] = {nz.x, nz.y, nz.z, nz.w}, fza[4] = {fz.x, fz.y, fz.z, fz.w};
+  const float tfar_lim = L.tb * 1.00000024f;
+  uint32_t cw[4] = {as_u(cf.x), as_u(cf.y), as_u(cf.z), as_u(cf.w)};
+  float tn[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const float x0 = fmaf(nxa[k], L.inv.x, -L.oi.x), x1 = fmaf(fxa[k], L.inv.x, -L.oi.x);
+    const float y0 = fmaf(nya[k], L.inv.y, -L.oi.y), y1 = fmaf(fya[k], L.inv.y, -L.oi.y);
+    const float z0 = fmaf(nza[k], L.inv.z, -L.oi.z), z1 = fmaf(fza[k], L.inv.z, -L.oi.z);
+    const float tnear = fmaxf(fmaxf(x0, y0), fmaxf(z0, EPS_ACNE));
+    const float tfar = fminf(fminf(x1, y1), fminf(z1, tfar_lim));
+    tn[k] = tnear <= tfar ? tnear : FLT_MAX;
+  }
+  trav_next(L, tn, cw, S);
+}
+
+/* one node in global memory */
+template <class STACK>
+__device__ __forceinline__ void trav_node_global(Trav &L, const Bvh4Node *nd, const STACK &S) {
+  const float4 *nf = reinterpret_cast<const float4 *>(nd);
+  const uint4 ch = reinterpret_cast<const uint4 *>(nd)[6];
+  uint32_t cw[4] = {ch.x, ch.y, ch.z, ch.w};
+  float tn[4];
+  slab4_minmax(L, nf, cw, tn);
+  trav_next(L, tn, cw, S);
+}
+
+/* the closest hit of a ray (L.tb, L.best: an arena record offset) */
+template <bool FULL, bool XF, class STACK>
+__device__ __forceinline__ void trav_ray(Trav &L, const DevScene &sc, const LdsWindow &w, const STACK &S, uint32_t root) {
+  {
+    Lane s;
+    lane_start_ray(s, L.o, L.d, L.time, FULL ? 0u : root);
+    L.inv = s.inv;
+    L.oi = s.oi;
+    L.word = s.word;
+  }
+  L.tb = FLT_MAX;
+  L.best = MISS_WORD;
+  S.start(L);
+  if (FULL) {
+    L.rx = (as_u(L.inv.x) >> 31) * 16u;
+    L.ry = (as_u(L.inv.y) >> 31) * 16u + 32u;
+    L.rz = (as_u(L.inv.z) >> 31) * 16u + 64u;
+    L.a = dot(L.d, L.d);
+    L.ra = 1.0f / L.a;
+    const uint32_t nodes = lds_addr(w.nodes), prims = lds_addr(w.prims);
+    while (L.word != CHILD_EMPTY) {
+      if (!(L.word & CHILD_LEAF)) {
+        trav_node_lds(L, nodes + L.word, S);
+      } else {
+        /* one primitive per step: a lane on a leaf of 8 does not hold up the
+         * lanes taking node steps; the leaf word counts its primitives down
+         * and its offset up (the same order, so the same hits) */
+        const uint32_t off = L.word & LEAF_OFFSET_MASK, p = prims + off * 16u;
+        const bool last = ((L.word >> 28) & 7u) == 0u;
+        const float4 f0 = lds_ld4(p), f1 = lds_ld4(p + 16u), *rec = w.prims + off;
+        const uint32_t hdr = as_u(f0.w), type = hdr & PT_TYPE_MASK;
+        float t;
+        bool h;
+        if (XF && (hdr >> PT_XF_SHIFT)) h = test_prim<true>(sc, rec, hdr, L.o, L.d, L.time, EPS_ACNE, L.tb, t);
+        else if (type == PT_SPHERE) h = sphere_hit(xyz(f0), f1.x, L, EPS_ACNE, L.tb, t);
+        else if (type == PT_MSPHERE) h = sphere_hit(xyz(f0) + L.time * xyz(rec[2]), f1.x, L, EPS_ACNE, L.tb, t);
+        else if (type == PT_TRI) h = plane_t<true>(rec, L.o, L.d, EPS_ACNE, L.tb, t);
+        else h = plane_t<false>(rec, L.o, L.d, EPS_ACNE, L.tb, t);
+        if (h) {
+          L.tb = t;
+          L.best = off + w.ub;
+        }
+        if (last) S.pop(L);
+        else L.word += prim_units(type) - (1u << 28);
+      }
+    }
+  } else {
+    /* nodes and records come from L2 and beyond, the lanes of a wave from as
+     * many places; the wave takes node steps while most of its lanes have one
+     * to take, then leaf steps, so that each round of fetches serves more
+     * lanes */
+    for (;;) {
+      const bool leaf = L.word >= CHILD_LEAF && L.word != CHILD_EMPTY, node = L.word < CHILD_LEAF;
+      const uint32_t nn = (uint32_t)__popcll(__ballot(node)), nl = (uint32_t)__popcll(__ballot(leaf));
+      if (nn + nl == 0u) break;
+      if (nn >= nl) {
+        if (node) trav_node_global(L, sc.nodes + L.word, S);
+      } else if (leaf) {
+        const uint32_t off = L.word & LEAF_OFFSET_MASK;
+        const bool last = ((L.word >> 28) & 7u) == 0u;
+        const float4 *rec = sc.prims + off;
+        const uint32_t hdr = as_u(rec[0].w);
+        float t;
+        if (test_prim<XF>(sc, rec, hdr, L.o, L.d, L.time, EPS_ACNE, L.tb, t)) {
+          L.tb = t;
+          L.best = off;
+        }
+        if (last) S.pop(L);
+        else L.word += prim_units(hdr & PT_TYPE_MASK) - (1u << 28);
+      }
+    }
+  }
+}
+
 /* ------------------------------------------------- whole paths, one launch --- */
 /* A plain render's pass in one launch.  The wavefront above moves every path
  * through HBM twice per bounce and launches three kernels per bounce, and from
@@ -1541,30 +1766,60 @@ __device__ __forceinline__ void sample_xyz(const float4 *cie, float4 L, uint32_t
  * operations on the same stream as in the wavefront: the same image, bit for
  * bit.
  *
- * Bound by VALU issue (88% busy on the sphere field).  Against the wavefront at
- * its default 4M-path passes, whole calls: sphere field 1920x1080 64 spp 60.5
- * -> 38.1 ms, prism 1024^2 64 spp 33.1 -> 19.4 ms, Cornell 256^2 16 spp 0.695
- * -> 0.590 ms; with 64M-path passes the wavefront's sphere field takes 40.3. */
+ * FULL: the scene of every job lies in the block's LDS, its child words
+ * rewritten to LDS offsets; else nodes and records come from memory.  In LDS
+ * the kernel is bound by VALU issue: 512-thread blocks, three to a CU beside
+ * a sphere field's 33 KB, at 6 waves per SIMD (80 VGPRs); 768 threads take
+ * 29.4 ms where 512 take 29.2 and leave less room for larger scenes, 512
+ * threads at 5 waves and no spills 36.4.  From memory it waits on node
+ * fetches: two-wave blocks, so that few rays wait for the longest one of the
+ * block, at 8 waves per SIMD: the 1M-triangle mesh takes 63.7 ms, 66.8 in
+ * blocks of 256 threads, 73.4 at 6 waves, 68.6 / 69.1 with node and leaf steps
+ * taken in another order than by majority (node-first / both each turn).  XF, EXT and
+ * MEDIA leave out of the registers what a batch has none of: without XF the
+ * sphere field goes from 32.7 to 29.2 ms.
+ *
+ * A wave is refilled once 16 of its lanes are free: below that the camera
+ * code costs more than the idle lanes (sphere field 32.8 ms at 1, 31.4 at 8 and
+ * 16, 31.8 at 32, 33.9 at 64); what is left over sorts to the block's end.
+ *
+ * Whole calls, before this kernel -> now: sphere field 1920x1080 64 spp 60.5
+ * -> 31.1 ms, prism 1024^2 64 spp 33.1 -> 17.7, mesh 4 views 8 spp 138.5 -> 68,
+ * Cornell 256^2 16 spp 0.695 -> 0.616. */
+#define PS_REFILL 16u
 #define PS_WORDS 9 /* LDS words per lane: stack entries, or one round of the exchange */
-template <int BLOCK, bool EXT, bool MEDIA>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4 : 6))) void k_paths(DevScene sc, GenParams gp,
+/* lanes of mask m below this one */
+__device__ __forceinline__ uint32_t below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+template <int BLOCK, bool EXT, bool MEDIA, bool FULL, bool XF>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4 : (FULL ? 6 : 8)))) void k_paths(DevScene sc, GenParams gp,
                                                                                       PathsArgs pa) {
   constexpr uint32_t WAVES = BLOCK / 64;
   static_assert(MC_COUNT * WAVES <= 64, "one lane of a wave per (class, wave) count");
-  extern __shared__ float4 smem[];
+  extern __shared__ __attribute__((aligned(128))) float4 scene[]; /* rows of a plane pair differ in address bit 4 */
   __shared__ uint32_t cnt[64];   /* paths per (class, wave) */
   __shared__ uint32_t pool[4];   /* sample ids at hand: [0] base and [1] length of the first range, [2] base of the
                                     second (pa.chunk long), [3] ids taken since the ranges were set */
-  const LdsWindow win = {smem, smem + pa.lds_nodes * 8u, pa.lds_nodes, pa.lds_node_base, pa.lds_units, pa.lds_unit_base};
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  uint32_t *ex = reinterpret_cast<uint32_t *>(smem + pa.lds_nodes * 8u + pa.lds_units);
-  LStack<BLOCK, PS_WORDS> S;
-  S.lst = ex + tid;
-  S.gst = pa.spill + (size_t)(blockIdx.x * BLOCK + tid) * (STACK_TOTAL - PS_WORDS);
+  const LdsWindow win = {scene, scene + pa.lds_nodes * 8u, pa.lds_nodes, pa.lds_node_base, pa.lds_units, pa.lds_unit_base};
+  const uint32_t tid = threadIdx.x, lane = __lane_id(), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint32_t *ex = reinterpret_cast<uint32_t *>(scene + pa.lds_nodes * 8u + pa.lds_units);
+  TravStack<BLOCK, PS_WORDS> S;
+  S.lst = lds_addr(ex + tid);
+  S.spill = pa.spill + (size_t)blockIdx.x * BLOCK * (STACK_TOTAL - PS_WORDS);
   {
     const float4 *gn = reinterpret_cast<const float4 *>(sc.nodes + win.nb);
-    for (uint32_t k = tid; k < win.nn * 8u; k += BLOCK) smem[k] = gn[k];
-    for (uint32_t k = tid; k < win.nu; k += BLOCK) smem[win.nn * 8u + k] = sc.prims[win.ub + k];
+    auto local = [&](float f) { /* a child word for FULL (struct Trav) */
+      const uint32_t c = as_u(f);
+      return __uint_as_float(c == CHILD_EMPTY ? c : (c & CHILD_LEAF) ? c - win.ub : (c - win.nb) * 128u);
+    };
+    for (uint32_t k = tid; k < win.nn * 8u; k += BLOCK) {
+      float4 v = gn[k];
+      if (FULL && (k & 7u) == 6u) v = make_float4(local(v.x), local(v.y), local(v.z), local(v.w));
+      scene[k] = v;
+    }
+    for (uint32_t k = tid; k < win.nu; k += BLOCK) scene[win.nn * 8u + k] = sc.prims[win.ub + k];
     if (tid == 0) {
       pool[0] = 0u;
       pool[1] = 0u;
@@ -1574,9 +1829,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
   }
   __syncthreads();
   const uint32_t n = gp.paths;
-  const bool any_xform = sc.has_xforms != 0;
-  const uint64_t below = (1ull << lane) - 1ull;
-  uint32_t rays = 0, unused = 0;
+  uint32_t rays = 0;
   bool exhausted = false; /* thread 0: the pass-wide cursor has passed the last sample */
   /* the lane's path */
   ShadeIn ps;
@@ -1591,14 +1844,25 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
   for (;;) {
     /* trace */
     uint32_t cls = MC_COUNT;
-    Lane L;
+    Trav L;
     L.tb = FLT_MAX;
     L.best = MISS_WORD;
     rays += (uint32_t)__popcll(__ballot(alive));
     if (alive) {
-      lane_start_ray(L, o, d, time, sc.jobs[ps.meta >> META_JOB_SHIFT].root);
-      lds_traverse<false>(L, sc, win, S, any_xform, unused, unused);
-      if (MEDIA) lane_media(L, sc, ps.meta, ps.rng);
+      L.o = o;
+      L.d = d;
+      L.time = time;
+      trav_ray<FULL, XF>(L, sc, win, S, FULL ? 0u : sc.jobs[ps.meta >> META_JOB_SHIFT].root);
+      if (MEDIA) {
+        Lane m;
+        m.o = o;
+        m.d = d;
+        m.tb = L.tb;
+        m.best = L.best;
+        lane_media(m, sc, ps.meta, ps.rng);
+        L.tb = m.tb;
+        L.best = m.best;
+      }
       cls = L.best != MISS_WORD ? sc.mats[sc.info[as_u(sc.prims[L.best + 1u].w)].material].mclass : MC_MISS;
     }
     /* each path's place in class order */
@@ -1607,7 +1871,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
     for (uint32_t c = 0; c < MC_COUNT; c++) {
       const uint64_t m = __ballot(cls == c);
       if (lane == 0) cnt[c * WAVES + wave] = (uint32_t)__popcll(m);
-      if (cls == c) rank = (uint32_t)__popcll(m & below);
+      if (cls == c) rank = below(m);
     }
     __syncthreads();
     if (tid == 0 && pool[3] >= pool[1]) { /* the first range is used up: the rest of the second follows, and a new one */
@@ -1692,11 +1956,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
       const PathBuf pb = PathBuf();
       const GuideArgs ga = GuideArgs();
       switch (c) {
-        case MC_MISS: end = shade_vertex<MC_MISS, false, EXT>(sc, pb, ps, 0u, ga, nx, lit); break;
-        case MC_LIGHT: end = shade_vertex<MC_LIGHT, false, EXT>(sc, pb, ps, 0u, ga, nx, lit); break;
-        case MC_LAMBERTIAN: end = shade_vertex<MC_LAMBERTIAN, false, EXT>(sc, pb, ps, 0u, ga, nx, lit); break;
-        case MC_METAL: end = shade_vertex<MC_METAL, false, EXT>(sc, pb, ps, 0u, ga, nx, lit); break;
-        default: end = shade_vertex<MC_GLASS, false, EXT>(sc, pb, ps, 0u, ga, nx, lit); break;
+        case MC_MISS: end = shade_vertex<MC_MISS, false, EXT, XF>(sc, pb, ps, 0u, ga, nx, lit); break;
+        case MC_LIGHT: end = shade_vertex<MC_LIGHT, false, EXT, XF>(sc, pb, ps, 0u, ga, nx, lit); break;
+        case MC_LAMBERTIAN: end = shade_vertex<MC_LAMBERTIAN, false, EXT, XF>(sc, pb, ps, 0u, ga, nx, lit); break;
+        case MC_METAL: end = shade_vertex<MC_METAL, false, EXT, XF>(sc, pb, ps, 0u, ga, nx, lit); break;
+        default: end = shade_vertex<MC_GLASS, false, EXT, XF>(sc, pb, ps, 0u, ga, nx, lit); break;
       }
       if (end == SH_GOES_ON) {
         o = mk(nx.o.x, nx.o.y, nx.o.z);
@@ -1713,12 +1977,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
     }
     /* refill */
     const uint64_t idle = __ballot(!alive);
-    if (idle) {
+    if ((uint32_t)__popcll(idle) >= PS_REFILL) {
       uint32_t base = 0;
       if (lane == 0) base = atomicAdd(&pool[3], (uint32_t)__popcll(idle));
       base = __builtin_amdgcn_readfirstlane(base);
       if (!alive) {
-        const uint32_t k = base + (uint32_t)__popcll(idle & below), len = pool[1];
+        const uint32_t k = base + below(idle), len = pool[1];
         ps.slot = k < len ? pool[0] + k : pool[2] + (k - len);
         alive = ps.slot < n;
         if (alive) {
@@ -2493,32 +2757,43 @@ void launch_guide_infer(hipStream_t st, const DevScene &sc, const PathBuf &pb, c
                      st, sc, pb, ga, queue, count);
 }
 
-/* k_paths: block size, LDS of a window, resident blocks and spill words */
-#define PS_BLOCK 768
-uint32_t paths_block() { return PS_BLOCK; }
-size_t paths_lds_bytes(uint32_t nodes, uint32_t units) {
-  return (size_t)nodes * sizeof(Bvh4Node) + (size_t)units * 16u + (size_t)PS_WORDS * PS_BLOCK * 4u;
+/* k_paths: blocks of 12 waves that share a scene in LDS, or of 4 that read it from memory */
+#define PS_BLOCK_LDS 512
+#define PS_BLOCK_GLOBAL 128
+uint32_t paths_block(bool full) { return full ? PS_BLOCK_LDS : PS_BLOCK_GLOBAL; }
+size_t paths_lds_bytes(bool full, uint32_t nodes, uint32_t units) {
+  return (size_t)nodes * sizeof(Bvh4Node) + (size_t)units * 16u + (size_t)PS_WORDS * paths_block(full) * 4u;
 }
-size_t paths_spill_words(uint32_t blocks) { return (size_t)blocks * PS_BLOCK * (STACK_TOTAL - PS_WORDS); }
+size_t paths_spill_words(bool full, uint32_t blocks) {
+  return (size_t)blocks * paths_block(full) * (STACK_TOTAL - PS_WORDS);
+}
 
 typedef void (*paths_fn)(DevScene, GenParams, PathsArgs);
-static paths_fn paths_instance(bool ext, bool media) {
-  if (media) return k_paths<PS_BLOCK, true, true>; /* a medium's phase function is an extended material */
-  return ext ? k_paths<PS_BLOCK, true, false> : k_paths<PS_BLOCK, false, false>;
+template <int BLOCK, bool FULL, bool XF>
+static paths_fn paths_instance_of(bool ext, bool media) {
+  if (media) return k_paths<BLOCK, true, true, FULL, XF>; /* a medium's phase function is an extended material */
+  return ext ? k_paths<BLOCK, true, false, FULL, XF> : k_paths<BLOCK, false, false, FULL, XF>;
 }
-uint32_t paths_grid_blocks(size_t lds_bytes, bool ext, bool media) {
+static paths_fn paths_instance(const DevScene &sc, bool full) {
+  const bool ext = sc.has_ext != 0, media = sc.has_media != 0, xf = sc.has_xforms != 0;
+  if (full)
+    return xf ? paths_instance_of<PS_BLOCK_LDS, true, true>(ext, media) : paths_instance_of<PS_BLOCK_LDS, true, false>(ext, media);
+  return xf ? paths_instance_of<PS_BLOCK_GLOBAL, false, true>(ext, media)
+            : paths_instance_of<PS_BLOCK_GLOBAL, false, false>(ext, media);
+}
+uint32_t paths_grid_blocks(size_t lds_bytes, const DevScene &sc, bool full) {
   int dev = 0, cus = 0, per_cu = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(paths_instance(ext, media)),
-                                                     PS_BLOCK, lds_bytes);
+  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(paths_instance(sc, full)),
+                                                     (int)paths_block(full), lds_bytes);
   return (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, cus);
 }
 void launch_paths(hipStream_t st, const DevScene &sc, const GenParams &gp, const PathsArgs &pa, uint32_t blocks,
                   size_t lds_bytes, bool begin) {
   hipLaunchKernelGGL(k_paths_begin, dim3(1), dim3(64), 0, st, pa.next, blocks * pa.first, begin ? pa.stats : nullptr);
-  hipLaunchKernelGGL(paths_instance(sc.has_ext != 0, sc.has_media != 0), dim3(blocks), dim3(PS_BLOCK), lds_bytes, st, sc,
-                     gp, pa);
+  hipLaunchKernelGGL(paths_instance(sc, pa.full != 0), dim3(blocks),
+                     dim3(paths_block(pa.full != 0)), lds_bytes, st, sc, gp, pa);
 }
 void launch_resolve_xyz(hipStream_t st, const ResolveParams &rp, const F3 *res, float *out, float *out_sq) {
   hipLaunchKernelGGL(k_resolve_xyz, dim3(grid_for(rp.threads, 256, 65535)), dim3(256), 0, st, rp, res, out, out_sq);

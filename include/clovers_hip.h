@@ -344,7 +344,8 @@ typedef enum {
   CLV_TRACE_PERSISTENT = 1, /* persistent waves refilling lanes from a work counter */
   CLV_TRACE_WW = 2,         /* one ray per thread, node steps and leaf steps in separate loops */
   CLV_TRACE_LDS_CACHED = 3  /* 768-thread blocks, top of the BVH and leading records cached in LDS; renders without
-                               guided jobs run every path from the camera to its end in one launch per pass */
+                               guided jobs run every path from the camera to its end in one launch per pass, from
+                               LDS if the scene of all jobs fits in lds_bytes whole, else from memory */
 } clv_trace_kernel;
 typedef struct {
   uint32_t target_paths;    /* samples per wavefront pass (queue and path-state capacity).  At the default, 2^22, a

@@ -31,7 +31,7 @@ def same(a, b):
 
 @pytest.mark.parametrize("name", ["cornell", "spheres", "motion", "prism", "features", "media", "mesh"])
 @pytest.mark.parametrize("size", [(1, 1, 1), (63, 1, 1), (65, 1, 1), (13, 59, 1), (8, 96, 1), (769, 1, 1),
-                                  (127, 33, 96), (641, 617, 1)])
+                                  (127, 33, 96), (641, 617, 1), (129, 1, 1), (511, 1, 1), (513, 1, 1)])
 def test_whole_paths_equal_the_wavefront(name, size):
     make = {"cornell": synth.cornell, "spheres": synth.spheres, "motion": lambda: synth.spheres(moving=True),
             "prism": synth.prism, "features": synth.features, "media": synth.media,
@@ -58,3 +58,21 @@ def test_batches_of_scenes_and_passes(target):
         for k, (sid, o) in enumerate(jobs):  # and each job alone
             img, sq = r.render(sid, o, want_sq=True)
             assert np.array_equal(img, x[0][2 * k]) and np.array_equal(sq, x[0][2 * k + 1])
+
+
+def test_scenes_that_share_a_batch_are_read_from_memory():
+    """a batch of several scenes is not in LDS: instance chains, checkers, a cone light, moving
+    spheres and media through the kernel that reads nodes and records from memory, and a scene
+    that fits in LDS but not in the tuned share of it"""
+    with clovers_amd.Renderer(0) as r:
+        a, b, c = r.upload(synth.features()), r.upload(synth.media()), r.upload(synth.spheres(moving=True))
+        o = abi.render_opts(90, 70, 7, 11, seed=8)
+        for jobs in ([(a, o), (c, o)], [(a, o), (b, o), (c, o)]):
+            x, y = both(r, jobs)
+            same(x, y)
+            r.set_tuning(trace_kernel=abi.TRACE_LDS_CACHED)
+            for k, (sid, _) in enumerate(jobs):
+                assert np.array_equal(r.render(sid, o)[0], x[0][2 * k])
+        want = r.render(c, o)[0]
+        r.set_tuning(lds_bytes=16384)
+        assert np.array_equal(r.render(c, o)[0], want)
