@@ -77,8 +77,9 @@ struct GuideState {
   _Float16 *Wh = nullptr;                          /* fp16 operand copies */
   float *partial = nullptr;                        /* per-wave gradient slices */
   uint32_t partial_waves = 0;
-  uint32_t cap_paths = 0;                          /* path capacity of the buffers below */
+  uint32_t cap_lobes = 0;                          /* paths the lobes are kept for */
   uint32_t *lobes = nullptr;
+  uint32_t cap_paths = 0;                          /* paths of a training pass: capacity of the buffers below */
   GuideRec *rec = nullptr;
   float *recL = nullptr;     /* radiance credited to each record this pass */
   uint32_t *gcnt = nullptr;
@@ -273,6 +274,11 @@ bool whole_paths(const clv_ctx *c, bool any_guide, uint32_t flags) {
  * samples of a whole render in one (up to 1.6 GB of contributions) */
 #define DEFAULT_TARGET_PATHS (1u << 22)
 #define WHOLE_TARGET_PATHS (1u << 27)
+
+/* an untuned context's wavefront passes behind the last training round grow to
+ * this many paths: the late bounces of a pass launch four kernels each for a
+ * few paths (274 bytes of state and lobes per path, 4.6 GB) */
+#define MERGED_TARGET_PATHS (1u << 24)
 
 clv_status paths_geometry(clv_ctx *c, const SceneRes *s, bool one_scene, const DevScene &ds, TraceGeom *g) {
   g->full = one_scene && paths_lds_bytes(true, s->n_nodes, s->prim_units) <= c->lds_block_bytes;
@@ -525,19 +531,30 @@ void guide_free(GuideState &g) {
   dfree(g.lobes); dfree(g.rec); dfree(g.recL); dfree(g.gcnt); dfree(g.list); dfree(g.bcount); dfree(g.bweight);
 }
 
-/* record space: GD_SLOTS per path slot, then the light-traced records of a
- * round (g.photons) */
+/* lobes of `paths` path slots of any pass */
+clv_status guide_ensure_lobes(clv_ctx *c, uint32_t paths) {
+  GuideState &g = c->guide;
+  if (paths <= g.cap_lobes) return CLV_OK;
+  dfree(g.lobes);
+  g.lobes = nullptr;
+  g.cap_lobes = 0;
+  HIPCHK(c, dalloc(&g.lobes, (size_t)paths * GD_LWORDS));
+  g.cap_lobes = paths;
+  return CLV_OK;
+}
+
+/* record space of a training pass: GD_SLOTS per path slot, then the
+ * light-traced records of a round (g.photons) */
 clv_status guide_ensure_paths(clv_ctx *c, uint32_t paths) {
   GuideState &g = c->guide;
   if (paths <= g.cap_paths && g.photons <= g.cap_photons) return CLV_OK;
-  dfree(g.lobes); dfree(g.rec); dfree(g.recL); dfree(g.gcnt); dfree(g.list); dfree(g.bcount); dfree(g.bweight);
-  g.lobes = nullptr; g.rec = nullptr; g.recL = nullptr; g.gcnt = nullptr; g.list = nullptr; g.bcount = nullptr;
+  dfree(g.rec); dfree(g.recL); dfree(g.gcnt); dfree(g.list); dfree(g.bcount); dfree(g.bweight);
+  g.rec = nullptr; g.recL = nullptr; g.gcnt = nullptr; g.list = nullptr; g.bcount = nullptr;
   g.bweight = nullptr;
   paths = std::max(paths, g.cap_paths);
   g.cap_paths = 0;
   g.cap_photons = 0;
   const size_t slots = (size_t)paths * GD_SLOTS + g.photons;
-  HIPCHK(c, dalloc(&g.lobes, (size_t)paths * GD_LWORDS));
   HIPCHK(c, dalloc(&g.rec, slots));
   HIPCHK(c, dalloc(&g.recL, slots));
   HIPCHK(c, dalloc(&g.gcnt, paths));
@@ -688,8 +705,10 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
   const bool whole = whole_paths(c, any_guide, flags);
   PassPlan pl;
   /* a frozen network is not trained: no training slices, every pass full size */
-  plan_passes(dj, soff, whole && c->target_paths == DEFAULT_TARGET_PATHS ? WHOLE_TARGET_PATHS : c->target_paths, std::max<uint32_t>(1, c->guide.train_spp), frozen ? 0u : c->guide.rounds,
-              c->guide.warmup != 0, &pl);
+  const bool untuned = c->target_paths == DEFAULT_TARGET_PATHS;
+  plan_passes(dj, soff, whole && untuned ? WHOLE_TARGET_PATHS : c->target_paths, std::max<uint32_t>(1, c->guide.train_spp),
+              frozen ? 0u : c->guide.rounds, c->guide.warmup != 0, &pl);
+  if (!whole && untuned) merge_passes(&pl, MERGED_TARGET_PATHS);
   std::vector<uint32_t> job_left(n);
   for (uint32_t k = 0; k < n; k++) job_left[k] = dj[k].spp;
   for (DevItem &it : pl.items) {
@@ -706,7 +725,11 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
   CHK(ensure_tables(c, n, (uint32_t)pl.items.size()));
   GuideState &gs = c->guide;
   if (any_guide) {
-    CHK(guide_ensure_paths(c, pl.max_paths));
+    uint32_t recorded = 0; /* the largest pass that writes training records */
+    for (uint32_t p = 0; p < passes; p++)
+      if (!frozen && pl.train[p]) recorded = std::max(recorded, pl.paths[p]);
+    CHK(guide_ensure_lobes(c, pl.max_paths));
+    CHK(guide_ensure_paths(c, recorded));
     CHK(guide_ensure_partial(c, gs.step / 64u));
     const bool fresh = !(flags & CLV_FLAG_GUIDE_KEEP) || !gs.init;
     if (fresh) CHK(guide_reset(c, guide_seed));
@@ -760,8 +783,6 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
   sq.counts = c->counts + CNT_SHADE;
   size_t ev = 2;
   PathBuf pb = c->pb;
-  pb.gcnt = any_guide ? gs.gcnt : nullptr;
-  pb.recL = any_guide ? gs.recL : nullptr;
   GuideArgs ga;
   memset(&ga, 0, sizeof(ga));
   if (any_guide) {
@@ -840,12 +861,15 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
     gp.items = c->items + pl.first[p];
     gp.n_items = pl.first[p + 1] - pl.first[p];
     gp.paths = pl.paths[p];
+    const bool recording = any_guide && !frozen && pl.train[p];
+    pb.gcnt = recording ? gs.gcnt : nullptr;
+    pb.recL = recording ? gs.recL : nullptr;
     launch_set_count(c->stream, c->counts, CNT_QA, gp.paths);
     launch_generate(c->stream, ds, pb, gp);
     if (any_guide) {
       /* plain sampling until the network has had a training round (or, frozen, always the network) */
       ga.alpha = (gs.trained || frozen) ? gs.alpha : 0.0f;
-      ga.record = (!frozen && pl.train[p]) ? 1u : 0u;
+      ga.record = recording ? 1u : 0u;
       ga.gate = gs.photons && gs.gate_density > 0.0f && gs.gate_valid && gs.gate_jobs >= n ? gs.gate : nullptr;
       ga.stamp = ++gs.stamp;
     }
@@ -907,8 +931,9 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
   launch_finalize(c->stream, rp, c->out, any_sq ? c->out_sq : nullptr);
   return CLV_OK;
   };
-  const bool keep = (flags & CLV_FLAG_GUIDE_KEEP) != 0;
-  const bool use_graph = c->use_graph && !timing && !(any_guide && keep);
+  /* not guided renders: a captured training round runs all the steps its record buffer could fill, most of
+   * them empty (a 64-spp prism 27 ms of 72), where an eager one reads the round's count back first */
+  const bool use_graph = c->use_graph && !timing && !any_guide;
   std::string sig;
   if (use_graph) {
     /* everything a launch argument depends on; pass ids of guided renders

@@ -1248,5 +1248,45 @@ void plan_passes(const std::vector<DevJob> &jobs, const std::vector<uint32_t> &s
   pl->first.push_back((uint32_t)pl->items.size());
 }
 
+void merge_passes(PassPlan *pl, uint32_t target) {
+  const size_t n = pl->paths.size();
+  size_t keep = 0; /* passes up to the last training one stay as they are */
+  for (size_t p = 0; p < n; p++)
+    if (pl->train[p]) keep = p + 1;
+  PassPlan out;
+  for (size_t p = 0; p < n; p++) {
+    const bool join = p > keep && (uint64_t)out.paths.back() + pl->paths[p] <= target;
+    if (!join) {
+      out.first.push_back((uint32_t)out.items.size());
+      out.paths.push_back(0);
+      out.depth.push_back(0);
+      out.train.push_back(pl->train[p]);
+    }
+    for (uint32_t i = pl->first[p]; i < pl->first[p + 1]; i++) {
+      /* a job's slices follow each other: one item per job and pass */
+      const DevItem &it = pl->items[i];
+      size_t k = out.first.back();
+      while (k < out.items.size() && out.items[k].job != it.job) k++;
+      if (k < out.items.size()) out.items[k].samples += it.samples;
+      else out.items.push_back(it);
+      out.paths.back() += it.pixels * it.samples;
+    }
+    out.depth.back() = std::max(out.depth.back(), pl->depth[p]);
+    out.max_paths = std::max(out.max_paths, out.paths.back());
+  }
+  out.first.push_back((uint32_t)out.items.size());
+  for (size_t p = 0; p < out.paths.size(); p++) {
+    uint32_t base = 0, res = 0;
+    for (uint32_t i = out.first[p]; i < out.first[p + 1]; i++) {
+      DevItem &it = out.items[i];
+      it.path_base = base;
+      it.res_base = res;
+      base += it.pixels * it.samples;
+      res += it.pixels;
+    }
+    out.res.push_back(res);
+  }
+  *pl = out;
+}
 
 }  // namespace clv

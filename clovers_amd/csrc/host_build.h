@@ -82,6 +82,10 @@ struct PassPlan {
  * max_depth, guiding of `jobs`. */
 void plan_passes(const std::vector<DevJob> &jobs, const std::vector<uint32_t> &sample_offset, uint32_t target,
                  uint32_t guided_cap, uint32_t rounds, bool warmup, PassPlan *pl);
+/* join the passes behind the last training one, in order, into passes of at
+ * most `target` paths (a pass already larger stays): no training round lies
+ * between them, so no path changes */
+void merge_passes(PassPlan *pl, uint32_t target);
 
 /* Camera::new (camera.rs:59-99) for the given aspect ratio. */
 DevCamera make_camera(const clv_camera_init &ci, float aspect);
