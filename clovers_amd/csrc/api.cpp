@@ -75,8 +75,8 @@ struct SceneRes {
 struct GuideState {
   float *P = nullptr, *M = nullptr, *V = nullptr;  /* fp32 parameters, Adam moments */
   _Float16 *Wh = nullptr;                          /* fp16 operand copies */
-  float *partial = nullptr;                        /* per-wave gradient slices */
-  uint32_t partial_waves = 0;
+  float *partial = nullptr;                        /* gradient slices, one per 64 records of a step */
+  uint32_t partial_groups = 0;
   uint32_t cap_lobes = 0;                          /* paths the lobes are kept for */
   uint32_t *lobes = nullptr;
   uint32_t cap_paths = 0;                          /* paths of a training pass: capacity of the buffers below */
@@ -105,6 +105,7 @@ struct GuideState {
   uint32_t photons = 1u << 20; /* clv_tuning.guide_photons: light-traced records per training round */
   /* the guiding gate (guide.h GD_GRID): light-traced record counts per cell and job, their totals, the open cells */
   uint32_t *cells = nullptr, *cell_tot = nullptr;
+  uint32_t *fresh = nullptr;   /* the counts of the round in flight, in gate_copies(jobs) copies of cells */
   uint8_t *gate = nullptr;
   uint32_t gate_jobs = 0;      /* jobs the buffers hold */
   bool gate_valid = false;     /* the gate has been built since the counts were cleared */
@@ -156,6 +157,7 @@ struct clv_ctx {
   size_t lds_block_bytes = 64512; /* dynamic LDS budget of one block of the LDS-cached traversal (64 KB less static use) */
   uint32_t trace_blocks = 0;      /* resident blocks of the persistent traversal */
   uint32_t infer_blocks = 1;      /* resident blocks of the network inference kernel */
+  uint32_t photon_blocks = 1;     /* resident blocks of the light-traced records' kernel */
   uint32_t shade_blocks[4] = {1u << 30, 1u << 30, 1u << 30, 1u << 30}; /* resident blocks per shading instance */
   uint32_t tail_depth = 0;        /* bounce from which a pass finishes its paths in one launch (0: never) */
   void *na_scratch = nullptr;     /* this device's copy of the allocation-free probe's scratch array */
@@ -512,21 +514,21 @@ clv_status guide_ensure_net(clv_ctx *c) {
   return CLV_OK;
 }
 
-clv_status guide_ensure_partial(clv_ctx *c, uint32_t waves) {
+clv_status guide_ensure_partial(clv_ctx *c, uint32_t groups) {
   GuideState &g = c->guide;
-  if (waves <= g.partial_waves) return CLV_OK;
+  if (groups <= g.partial_groups) return CLV_OK;
   dfree(g.partial);
   g.partial = nullptr;
-  g.partial_waves = 0;
-  HIPCHK(c, dalloc(&g.partial, (size_t)(waves + (waves + 15u) / 16u) * GD_NPARAM)); /* wave slices + chunk sums */
-  g.partial_waves = waves;
+  g.partial_groups = 0;
+  HIPCHK(c, dalloc(&g.partial, (size_t)groups * GD_NPARAM));
+  g.partial_groups = groups;
   return CLV_OK;
 }
 
 void guide_free(GuideState &g) {
   if (g.host_totals) (void)hipHostFree(g.host_totals);
   g.host_totals = nullptr;
-  dfree(g.cells); dfree(g.cell_tot); dfree(g.gate);
+  dfree(g.cells); dfree(g.cell_tot); dfree(g.gate); dfree(g.fresh);
   dfree(g.P); dfree(g.M); dfree(g.V); dfree(g.Wh); dfree(g.partial); dfree(g.totals);
   dfree(g.lobes); dfree(g.rec); dfree(g.recL); dfree(g.gcnt); dfree(g.list); dfree(g.bcount); dfree(g.bweight);
 }
@@ -603,16 +605,23 @@ clv_status guide_reset(clv_ctx *c, uint64_t seed) {
   return CLV_OK;
 }
 
+/* copies of the gate's fresh counts: the contention they relieve is a job's, so one job gets the most of them.
+ * A buffer of gate_fresh_jobs(n) jobs holds the copies of a batch of n jobs and of every smaller one */
+#define GATE_COPIES 16u
+uint32_t gate_copies(uint32_t n_jobs) { return std::max<uint32_t>(1u, GATE_COPIES / n_jobs); }
+size_t gate_fresh_jobs(uint32_t n_jobs) { return std::max<uint32_t>(GATE_COPIES, n_jobs); }
+
 /* gate buffers for n jobs; clear = zero the counts (a fresh network) */
 clv_status guide_ensure_gate(clv_ctx *c, uint32_t n, bool clear) {
   GuideState &g = c->guide;
   if (n > g.gate_jobs) {
-    dfree(g.cells); dfree(g.cell_tot); dfree(g.gate);
-    g.cells = g.cell_tot = nullptr;
+    dfree(g.cells); dfree(g.cell_tot); dfree(g.gate); dfree(g.fresh);
+    g.cells = g.cell_tot = g.fresh = nullptr;
     g.gate = nullptr;
     g.gate_jobs = 0;
     HIPCHK(c, dalloc(&g.cells, (size_t)n * GD_CELLS));
     HIPCHK(c, dalloc(&g.cell_tot, n));
+    HIPCHK(c, dalloc(&g.fresh, gate_fresh_jobs(n) * GD_CELLS));
     HIPCHK(c, dalloc(&g.gate, (size_t)n * GD_CELLS));
     g.gate_jobs = n;
     clear = true;
@@ -620,6 +629,8 @@ clv_status guide_ensure_gate(clv_ctx *c, uint32_t n, bool clear) {
   if (clear) {
     HIPCHK(c, hipMemsetAsync(g.cells, 0, (size_t)g.gate_jobs * GD_CELLS * sizeof(uint32_t), c->stream));
     HIPCHK(c, hipMemsetAsync(g.cell_tot, 0, (size_t)g.gate_jobs * sizeof(uint32_t), c->stream));
+    HIPCHK(c, hipMemsetAsync(g.fresh, 0, gate_fresh_jobs(g.gate_jobs) * GD_CELLS * sizeof(uint32_t),
+                             c->stream));
     g.gate_valid = false;
   }
   return CLV_OK;
@@ -632,7 +643,7 @@ void guide_photons(clv_ctx *c, const DevScene &ds, uint32_t n_jobs, uint32_t pat
   GuideState &g = c->guide;
   const size_t base = (size_t)paths * GD_SLOTS;
   launch_guide_photons(c->stream, ds, n_jobs, g.rec + base, g.recL + base, g.photons, stamp, round, seed, c->spill,
-                       c->trace_blocks, g.cells);
+                       std::min(c->photon_blocks, c->trace_blocks), g.fresh, gate_copies(n_jobs));
 }
 
 /* one training round on the records of pass `stamp` (n path slots), and
@@ -849,7 +860,7 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
     const uint32_t st = ++gs.stamp;
     guide_photons(c, ds, n, 0, st, rounds_run, guide_seed);
     guide_train_round(c, 0, st, nullptr, gs.wclip, gs.photons);
-    launch_guide_gate(c->stream, gs.cells, gs.cell_tot, gs.gate, n, gs.gate_density);
+    launch_guide_gate(c->stream, gs.fresh, gate_copies(n), gs.cells, gs.cell_tot, gs.gate, n, gs.gate_density);
     if (end) (void)hipEventRecord(end, c->stream);
     gs.trained = true;
     gs.gate_valid = true;
@@ -920,7 +931,7 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
       if (photon_rounds) guide_photons(c, ds, n, gp.paths, ga.stamp, rounds_run, guide_seed);
       guide_train_round(c, gp.paths, ga.stamp, nullptr, gs.wclip, photon_rounds ? gs.photons : 0u);
       if (photon_rounds) {
-        launch_guide_gate(c->stream, gs.cells, gs.cell_tot, gs.gate, n, gs.gate_density);
+        launch_guide_gate(c->stream, gs.fresh, gate_copies(n), gs.cells, gs.cell_tot, gs.gate, n, gs.gate_density);
         gs.gate_valid = true;
       }
       if (end) (void)hipEventRecord(end, c->stream);
@@ -1128,6 +1139,7 @@ clv_status clv_create(int hip_device, clv_ctx **out) {
   }
   c->trace_blocks = trace_grid_blocks();
   c->infer_blocks = guide_infer_grid_blocks();
+  c->photon_blocks = guide_photon_grid_blocks();
   shade_grid_blocks(c->shade_blocks);
   /* the device address of the allocation-free probe's scratch array on this
    * device (the device is current); left NULL if the runtime has none */

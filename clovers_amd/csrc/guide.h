@@ -120,7 +120,8 @@ typedef float gf4 __attribute__((ext_vector_type(4)));
  * hardware sine and cosine (which take revolutions and reduce them exactly:
  * |a| / 2 pi <= 32 here) and the double angle from them (one rounding each,
  * below the features' fp16 precision). */
-__device__ __forceinline__ void gd_encode(const float p[3], const float n[3], float lam, gh4 x[4]) {
+__device__ __forceinline__ void gd_encode(const float p[3], const float n[3], float lam, gh4 x[4],
+                                          float *sin2 = nullptr /* sin 2a of the position cells, in fp32 */) {
   const int g = (threadIdx.x & 63) >> 4;
 #pragma unroll
   for (int kt = 0; kt < 4; kt++) {
@@ -135,6 +136,7 @@ __device__ __forceinline__ void gd_encode(const float p[3], const float n[3], fl
     }
     const float sn = __builtin_amdgcn_sinf(rev), cs = __builtin_amdgcn_cosf(rev);
     float v0 = sn, v1 = cs, v2 = 2.0f * sn * cs, v3 = 1.0f - 2.0f * sn * sn;
+    if (sin2 && kt < 3) sin2[kt] = v2;
     if (kt == 3 && g >= 2) {
       v0 = g == 2 ? p[0] : n[0];
       v1 = g == 2 ? p[1] : n[1];

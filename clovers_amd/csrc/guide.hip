@@ -7,11 +7,11 @@
  *       into a list, in slot order (deterministic), and compute their mean
  *       MC weight F/p;
  *   k_guide_train (per step)
- *       one wave per 64 records: forward on MFMA, d(loss)/d(outputs) per
- *       record, backward on MFMA; every wave writes its summed parameter
+ *       four waves per group of 64 records: forward on MFMA, d(loss)/d(outputs)
+ *       per record, backward on MFMA; every group writes its summed parameter
  *       gradient to its own slice of a partial buffer (no atomics);
  *   k_guide_adam (per step)
- *       sums the slices in wave order, Adam update of the fp32 master
+ *       sums the slices in group order, Adam update of the fp32 master
  *       parameters, refresh of the fp16 operand copies.
  * k_guide_eval and the gradient mode of k_guide_adam serve the C ABI's
  * network probes (clv_guide_eval, clv_guide_grad).
@@ -30,10 +30,10 @@ namespace clv {
 /* The back-propagated gradients go through fp16 (MFMA operands), whose
  * largest finite value is 65504: a record with a large weight F/p and a
  * sharp lobe (the gradient grows with kappa, up to ~5000) overflows it, and
- * one inf turns the whole network into NaN.  So each wave holds its fp16
+ * one inf turns the whole network into NaN.  So each group of 64 records holds its fp16
  * gradients in units of 2^se, a power of two chosen per layer from the
- * wave's largest magnitude so that it lands in [2^(GT_TOP-1), 2^GT_TOP);
- * partial sums leave the wave multiplied by 2^-se, which is exact. */
+ * group's largest magnitude so that it lands in [2^(GT_TOP-1), 2^GT_TOP);
+ * partial sums leave it multiplied by 2^-se, which is exact. */
 #define GT_TOP 12
 #define GT_EMAX 100
 
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256) void k_guide_count(const GuideRec *rec, const 
  * (as float bits): each source's weights are used relative to their own mean */
 __global__ __launch_bounds__(1024) void k_guide_scan(uint32_t *bcount, const float *bweight, uint32_t nb,
                                                      uint32_t *totals, uint32_t cap, unsigned long long *used) {
-  __shared__ uint32_t part[1024], lpart[1024];
+  __shared__ uint32_t part[1024];
   __shared__ double wpart[1024], wlpart[1024];
   const uint32_t per = (nb + 1023u) / 1024u;
   const uint32_t b0 = threadIdx.x * per, b1 = min(nb, b0 + per);
@@ -129,27 +129,45 @@ __global__ __launch_bounds__(1024) void k_guide_scan(uint32_t *bcount, const flo
     w += (double)bweight[2 * b];
     wl += (double)bweight[2 * b + 1];
   }
-  part[threadIdx.x] = s;
-  lpart[threadIdx.x] = sl;
   wpart[threadIdx.x] = w;
   wlpart[threadIdx.x] = wl;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t acc = 0, lacc = 0;
-    double wacc = 0.0, wlacc = 0.0;
-    for (uint32_t t = 0; t < 1024; t++) {
-      uint32_t v = part[t];
-      part[t] = acc;
-      acc += v;
-      lacc += lpart[t];
-      wacc += wpart[t];
-      wlacc += wlpart[t];
+  /* the counts' exclusive prefix by waves; the weights are added one after
+   * the other (their order is part of the result), each source by a thread of
+   * its own beside that: 23 -> 9 us, most of it that chain of additions */
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  uint32_t pre = s, lpre = sl;
+#pragma unroll
+  for (uint32_t k = 1; k < 64u; k <<= 1) {
+    const uint32_t u = __shfl_up(pre, k), lu = __shfl_up(lpre, k);
+    if (lane >= k) {
+      pre += u;
+      lpre += lu;
     }
-    totals[0] = acc;
-    const uint32_t cam = acc - lacc;
-    totals[1] = __float_as_uint(cam ? (float)(wacc / (double)cam) : 0.0f);
-    totals[2] = __float_as_uint(lacc ? (float)(wlacc / (double)lacc) : 0.0f);
-    if (used) *used += (unsigned long long)min(acc, cap);
+  }
+  __shared__ uint32_t wsum[16], lwsum[16];
+  if (lane == 63u) {
+    wsum[wave] = pre;
+    lwsum[wave] = lpre;
+  }
+  __syncthreads();
+  uint32_t base = 0, all = 0, lall = 0;
+  for (uint32_t k = 0; k < 16u; k++) {
+    if (k < wave) base += wsum[k];
+    all += wsum[k];
+    lall += lwsum[k];
+  }
+  part[threadIdx.x] = base + pre - s;
+  if (threadIdx.x == 0 || threadIdx.x == 64) {
+    const double *src = threadIdx.x == 0 ? wpart : wlpart;
+    const uint32_t cnt = threadIdx.x == 0 ? all - lall : lall;
+    double acc = 0.0;
+#pragma unroll 16
+    for (uint32_t t = 0; t < 1024u; t++) acc += src[t];
+    totals[threadIdx.x == 0 ? 1 : 2] = __float_as_uint(cnt ? (float)(acc / (double)cnt) : 0.0f);
+  }
+  if (threadIdx.x == 128) {
+    totals[0] = all;
+    if (used) *used += (unsigned long long)min(all, cap);
   }
   __syncthreads();
   uint32_t run = part[threadIdx.x];
@@ -182,52 +200,65 @@ __global__ __launch_bounds__(256) void k_guide_scatter(const GuideRec *rec, cons
 }
 
 /* ------------------------------------------------------------ training --- */
-/* d(-w log q)/d(outputs) of one record; o = raw outputs, g = 48 gradients */
-__device__ void gd_loss_grad(const float *o, const float d[3], float w, float *g) {
-  for (int k = 0; k < GD_OUT_PAD; k++) g[k] = 0.0f;
-  if (!(w > 0.0f)) return;
-  GdLobes L;
-  gd_decode(o, L);
-  float f[GD_LOBES], c[GD_LOBES], q = 0.0f;
-  for (int j = 0; j < GD_LOBES; j++) {
-    c[j] = L.mu[j][0] * d[0] + L.mu[j][1] * d[1] + L.mu[j][2] * d[2];
-    f[j] = gd_vmf_norm(L.kappa[j]) * expf(L.kappa[j] * (c[j] - 1.0f));
-    q += L.w[j] * f[j];
+/* d(-w log q)/d(outputs) of a record by the 4 lanes that share it (lane group g
+ * of 16 records: lobes g and g + 4): o = the record's raw outputs, gr = the
+ * gradients of the lane's two lobes, 5 each.  Sums over the lobes run in lobe
+ * order on every lane. */
+__device__ __forceinline__ float gd_lobe_sum(const float v[2], int r) {
+  float s = 0.0f;
+#pragma unroll
+  for (int j = 0; j < GD_LOBES; j++) s += __shfl(v[j >> 2], r + 16 * (j & 3));
+  return s;
+}
+__device__ void gd_loss_grad(const float *o, const float d[3], float w, int r, int g, float gr[2][5]) {
+  float mx = fmaxf(o[5 * g + 4], o[5 * (g + 4) + 4]);
+  mx = fmaxf(mx, __shfl_xor(mx, 16));
+  mx = fmaxf(mx, __shfl_xor(mx, 32));
+  float mu[2][3], kappa[2], wt[2], f[2], c[2], wf[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int j = g + 4 * h;
+    const float a = o[5 * j], b = o[5 * j + 1], cc = o[5 * j + 2];
+    const float len = sqrtf(a * a + b * b + cc * cc);
+    const bool ok = len > 1e-12f;
+    mu[h][0] = ok ? a / len : 0.0f;
+    mu[h][1] = ok ? b / len : 0.0f;
+    mu[h][2] = ok ? cc / len : 1.0f;
+    kappa[h] = expf(gd_clamp_logk(o[5 * j + 3]));
+    wt[h] = expf(o[5 * j + 4] - mx);
   }
+  const float sum = gd_lobe_sum(wt, r);
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    wt[h] /= sum;
+    c[h] = mu[h][0] * d[0] + mu[h][1] * d[1] + mu[h][2] * d[2];
+    f[h] = gd_vmf_norm(kappa[h]) * expf(kappa[h] * (c[h] - 1.0f));
+    wf[h] = wt[h] * f[h];
+  }
+  float q = gd_lobe_sum(wf, r);
   if (!(q > 1e-30f)) q = 1e-30f;
-  for (int j = 0; j < GD_LOBES; j++) {
-    const float r = L.w[j] * f[j] / q;
-    const float k = L.kappa[j];
-    g[5 * j + 4] = -w * (r - L.w[j]);
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int j = g + 4 * h;
+#pragma unroll
+    for (int t = 0; t < 5; t++) gr[h][t] = 0.0f;
+    if (!(w > 0.0f)) continue;
+    const float rr = wf[h] / q;
+    const float k = kappa[h];
+    gr[h][4] = -w * (rr - wt[h]);
     const float s = o[5 * j + 3];
     if (s > GD_LOGK_MIN && s < GD_LOGK_MAX) {
-      const float dlogf = 1.0f / k - 2.0f / expm1f(2.0f * k) + (c[j] - 1.0f);
-      g[5 * j + 3] = -w * r * k * dlogf;
+      const float dlogf = 1.0f / k - 2.0f / expm1f(2.0f * k) + (c[h] - 1.0f);
+      gr[h][3] = -w * rr * k * dlogf;
     }
     const float a = o[5 * j], b = o[5 * j + 1], cc = o[5 * j + 2];
     const float len = sqrtf(a * a + b * b + cc * cc);
     if (len > 1e-12f) {
-      const float gm[3] = {-w * r * k * d[0], -w * r * k * d[1], -w * r * k * d[2]};
-      const float mg = L.mu[j][0] * gm[0] + L.mu[j][1] * gm[1] + L.mu[j][2] * gm[2];
-      for (int t = 0; t < 3; t++) g[5 * j + t] = (gm[t] - L.mu[j][t] * mg) / len;
-    }
-  }
-}
-
-/* D^T[16*MT x 16] = A[16*MT x 16*KT] . B[16*KT x 16]: A fp16 row-major with
- * leading dimension lda (global or LDS), B operands in registers */
-template <int MT, int KT>
-__device__ __forceinline__ void gd_gemm_ab(const _Float16 *A, int lda, const gh4 *b, gf4 *acc) {
-  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+      const float gm[3] = {-w * rr * k * d[0], -w * rr * k * d[1], -w * rr * k * d[2]};
+      const float mg = mu[h][0] * gm[0] + mu[h][1] * gm[1] + mu[h][2] * gm[2];
 #pragma unroll
-  for (int mt = 0; mt < MT; mt++) {
-    gf4 c = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int kt = 0; kt < KT; kt++) {
-      const gh4 a = *reinterpret_cast<const gh4 *>(A + (16 * mt + r) * lda + 16 * kt + 4 * g);
-      c = __builtin_amdgcn_mfma_f32_16x16x16f16(a, b[kt], c, 0, 0, 0);
+      for (int t = 0; t < 3; t++) gr[h][t] = (gm[t] - mu[h][t] * mg) / len;
     }
-    acc[mt] = c;
   }
 }
 
@@ -242,22 +273,33 @@ struct GuideTrainArgs {
   float wclip;             /* weight cap in units of the mean weight */
   const _Float16 *Wh;
   const float *P;
-  float *partial;          /* [wave][GD_NPARAM] */
+  float *partial;          /* [group][GD_NPARAM] */
+  uint32_t *steps;         /* Adam's step count, one more for a step with records (an empty step changes nothing);
+                              NULL in the gradient mode */
 };
 
-/* one wave = one block = 64 records */
-__global__ __launch_bounds__(64) void k_guide_train(GuideTrainArgs a) {
-  __shared__ float rin[64][8];
+/* One block = a group of 64 records, 4 waves.  Wave w carries the tile of
+ * records 16w .. 16w + 15 through the forward pass, its output gradients and the
+ * back-propagated rows, and rows 16w .. of every weight gradient (a contraction
+ * over the 64 records of the group, read from LDS).  A step is a chain of
+ * short dependent phases and 256 groups, one to a CU, so its time is the
+ * latency of one group: with the group on one wave 34.1 us a step of 16,384
+ * records, 27.5 on four (12 of them up to the end of the forward pass, 2 the
+ * output gradients, 14 the backward pass and the 16 MB of slices).  Asking for
+ * the weights' cache lines ahead changed nothing. */
+__global__ __launch_bounds__(256) void k_guide_train(GuideTrainArgs a) {
+  __shared__ float rin[64][12];           /* inputs (7), direction (3), weight */
   __shared__ __attribute__((aligned(16))) _Float16 H[4][64 * GT_LD]; /* activations A0..A3, [feature][record] */
   __shared__ __attribute__((aligned(16))) _Float16 DZ[64 * GT_LD];   /* back-propagated rows, [neuron][record] */
   __shared__ float OG[64 * GT_OG];        /* outputs, then their gradients, [record][48] */
-  const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
+  __shared__ float wmax[4];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, g = lane >> 4, q = 16 * w + r;
   const uint32_t nvalid = a.totals[0];
   const uint32_t nuse = min(nvalid, a.cap);
-  const uint32_t u = a.step_base + blockIdx.x * 64u + (uint32_t)lane;
-  float wgt = 0.0f, dir[3] = {0.0f, 0.0f, 1.0f};
-  {
-    float in[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (a.steps && blockIdx.x == 0 && tid == 0 && a.step_base < nuse) *a.steps += 1u;
+  if (tid < 64) {
+    const uint32_t u = a.step_base + blockIdx.x * 64u + (uint32_t)tid;
+    float in[7] = {0, 0, 0, 0, 0, 0, 0}, wgt = 0.0f, dir[3] = {0.0f, 0.0f, 1.0f};
     if (u < nuse) {
       const uint32_t slot = a.list[(uint32_t)(((uint64_t)u * nvalid) / nuse)];
       const GuideRec R = a.rec[slot];
@@ -270,183 +312,197 @@ __global__ __launch_bounds__(64) void k_guide_train(GuideTrainArgs a) {
       }
       in[6] = R.lam;
     }
-    for (int k = 0; k < 8; k++) rin[lane][k] = in[k];
+    for (int k = 0; k < 7; k++) rin[tid][k] = in[k];
+    for (int k = 0; k < 3; k++) rin[tid][7 + k] = dir[k];
+    rin[tid][10] = wgt;
   }
   __syncthreads();
-  /* forward, layer by layer over the wave's 4 tiles of 16 records: a layer's
-   * weight operands (the same for every tile) are loaded once and the four
-   * tiles' MFMA chains are independent; every activation to LDS */
+  /* forward; every activation to LDS */
   {
-    gh4 cur[4][4]; /* [tile][k-step]: B operands of the current layer */
+    gh4 cur[4];
+    const float p[3] = {rin[q][0], rin[q][1], rin[q][2]}, n[3] = {rin[q][3], rin[q][4], rin[q][5]};
+    float sin2[3];
+    gd_encode(p, n, rin[q][6], cur, sin2);
+    /* sin 2a = 2 sin a cos a goes to fp16 in one rounding (v_fma_mixlo), except
+     * in the first layer's operands of the group's last tile, where the product
+     * is rounded to fp32 before: the last bit of a feature decides a seed's
+     * network and image, so each use keeps the rounding it has always had */
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-      const int q = 16 * nt + r;
-      const float p[3] = {rin[q][0], rin[q][1], rin[q][2]}, n[3] = {rin[q][3], rin[q][4], rin[q][5]};
-      gd_encode(p, n, rin[q][6], cur[nt]);
+    for (int kt = 0; kt < 4; kt++)
 #pragma unroll
-      for (int kt = 0; kt < 4; kt++)
+      for (int i = 0; i < 4; i++) {
+        _Float16 f = cur[kt][i];
+        asm volatile("" : "+v"(f));
+        cur[kt][i] = f;
+        H[0][(16 * kt + 4 * g + i) * GT_LD + q] = f;
+      }
+    if (w == 3)
 #pragma unroll
-        for (int i = 0; i < 4; i++) H[0][(16 * kt + 4 * g + i) * GT_LD + q] = cur[nt][kt][i];
-    }
+      for (int kt = 0; kt < 3; kt++) {
+        asm volatile("" : "+v"(sin2[kt]));
+        cur[kt][2] = (_Float16)sin2[kt];
+      }
 #pragma unroll
     for (int l = 0; l < 4; l++) {
       const int mts = l == 3 ? 3 : 4;
       const _Float16 *W = a.Wh + GD_H_W(l);
       const float *bias = a.P + (l == 0 ? GD_B1 : (l == 1 ? GD_B2 : (l == 2 ? GD_B3 : GD_B4)));
-      gh4 wa[4][4];
-      gf4 bv[4];
+      gf4 acc[4];
 #pragma unroll
       for (int mt = 0; mt < 4; mt++) {
         if (mt >= mts) break;
+        gf4 c;
 #pragma unroll
-        for (int kt = 0; kt < 4; kt++) wa[mt][kt] = *reinterpret_cast<const gh4 *>(W + (16 * mt + r) * 64 + 16 * kt + 4 * g);
+        for (int i = 0; i < 4; i++) c[i] = bias[16 * mt + 4 * g + i];
 #pragma unroll
-        for (int i = 0; i < 4; i++) bv[mt][i] = bias[16 * mt + 4 * g + i];
+        for (int kt = 0; kt < 4; kt++) {
+          const gh4 wa = *reinterpret_cast<const gh4 *>(W + (16 * mt + r) * 64 + 16 * kt + 4 * g);
+          c = __builtin_amdgcn_mfma_f32_16x16x16f16(wa, cur[kt], c, 0, 0, 0);
+        }
+        acc[mt] = c;
       }
+      if (l < 3) {
 #pragma unroll
-      for (int nt = 0; nt < 4; nt++) {
-        const int q = 16 * nt + r;
-        gf4 acc[4];
+        for (int k = 0; k < 4; k++) {
+          cur[k] = gd_relu_h(acc[k]);
 #pragma unroll
-        for (int mt = 0; mt < 4; mt++) {
-          if (mt >= mts) break;
-          gf4 c = bv[mt];
-#pragma unroll
-          for (int kt = 0; kt < 4; kt++) c = __builtin_amdgcn_mfma_f32_16x16x16f16(wa[mt][kt], cur[nt][kt], c, 0, 0, 0);
-          acc[mt] = c;
+          for (int i = 0; i < 4; i++) H[l + 1][(16 * k + 4 * g + i) * GT_LD + q] = cur[k][i];
         }
-        if (l < 3) {
+      } else {
 #pragma unroll
-          for (int k = 0; k < 4; k++) {
-            cur[nt][k] = gd_relu_h(acc[k]);
+        for (int mt = 0; mt < 3; mt++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) H[l + 1][(16 * k + 4 * g + i) * GT_LD + q] = cur[nt][k][i];
-          }
-        } else {
-#pragma unroll
-          for (int mt = 0; mt < 3; mt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) OG[q * GT_OG + 16 * mt + 4 * g + i] = acc[mt][i];
-        }
+          for (int i = 0; i < 4; i++) OG[q * GT_OG + 16 * mt + 4 * g + i] = acc[mt][i];
       }
     }
   }
   __syncthreads();
-  /* output gradient of this lane's record */
-  float gmax = 0.0f;
+  /* output gradients of the wave's records */
   {
-    float o[GD_OUT_PAD], gr[GD_OUT_PAD];
-    for (int k = 0; k < GD_OUT_PAD; k++) o[k] = OG[lane * GT_OG + k];
-    gd_loss_grad(o, dir, wgt, gr);
+    float gr[2][5];
+    const float dir[3] = {rin[q][7], rin[q][8], rin[q][9]};
+    gd_loss_grad(&OG[q * GT_OG], dir, rin[q][10], r, g, gr);
     bool fin = true;
-    for (int k = 0; k < GD_OUT_PAD; k++) {
-      fin = fin && isfinite(gr[k]);
-      gmax = fmaxf(gmax, fabsf(gr[k]));
-    }
-    if (!fin) gmax = 0.0f; /* a record whose gradient is not finite is left out */
-    for (int k = 0; k < GD_OUT_PAD; k++) OG[lane * GT_OG + k] = fin ? gr[k] : 0.0f;
+    float gmax = 0.0f;
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int t = 0; t < 5; t++) {
+        fin = fin && isfinite(gr[h][t]);
+        gmax = fmaxf(gmax, fabsf(gr[h][t]));
+      }
+    /* a record whose gradient is not finite is left out */
+    const uint64_t bad = __ballot(!fin);
+    fin = ((bad >> r) & 0x0001000100010001ull) == 0ull;
+    if (!fin) gmax = 0.0f;
+    __syncthreads(); /* the outputs are read */
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int t = 0; t < 5; t++) OG[q * GT_OG + 5 * (g + 4 * h) + t] = fin ? gr[h][t] : 0.0f;
+    OG[q * GT_OG + GD_OUT + 2 * g] = 0.0f; /* the padding rows */
+    OG[q * GT_OG + GD_OUT + 2 * g + 1] = 0.0f;
+    gmax = gt_wave_max(gmax);
+    if (lane == 0) wmax[w] = gmax;
   }
-  int se = gt_exponent(gt_wave_max(gmax), 0);
   __syncthreads();
+  int se = gt_exponent(fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])), 0);
   float *part = a.partial + (size_t)blockIdx.x * GD_NPARAM;
   /* layer 4: D = output gradients (48 rows), fp16 in units of 2^se */
-  gh4 din[4][4]; /* [record tile][k-step]: B operands of the current layer's D */
-  for (int nt = 0; nt < 4; nt++)
+  gh4 din[4]; /* [k-step]: B operands of the current layer's D for the wave's records */
 #pragma unroll
-    for (int kt = 0; kt < 3; kt++) {
-      gh4 v;
+  for (int kt = 0; kt < 3; kt++) {
+    gh4 v;
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const _Float16 gv = (_Float16)ldexpf(OG[(16 * nt + r) * GT_OG + 16 * kt + 4 * g + i], se);
-        v[i] = gv;
-        DZ[(16 * kt + 4 * g + i) * GT_LD + 16 * nt + r] = gv;
-      }
-      din[nt][kt] = v;
+    for (int i = 0; i < 4; i++) {
+      const _Float16 gv = (_Float16)ldexpf(OG[q * GT_OG + 16 * kt + 4 * g + i], se);
+      v[i] = gv;
+      DZ[(16 * kt + 4 * g + i) * GT_LD + q] = gv;
     }
-  if (lane < GD_OUT_PAD) {
+    din[kt] = v;
+  }
+  if (w == 3 && lane < GD_OUT_PAD) {
     /* four independent sums, so the LDS reads are not one dependent chain */
     float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
 #pragma unroll
-    for (int q = 0; q < 64; q += 4) {
-      s0 += OG[q * GT_OG + lane];
-      s1 += OG[(q + 1) * GT_OG + lane];
-      s2 += OG[(q + 2) * GT_OG + lane];
-      s3 += OG[(q + 3) * GT_OG + lane];
+    for (int k = 0; k < 64; k += 4) {
+      s0 += OG[k * GT_OG + lane];
+      s1 += OG[(k + 1) * GT_OG + lane];
+      s2 += OG[(k + 2) * GT_OG + lane];
+      s3 += OG[(k + 3) * GT_OG + lane];
     }
     part[GD_B4 + lane] = (s0 + s1) + (s2 + s3);
   }
   __syncthreads();
+#pragma unroll
   for (int layer = 4; layer >= 1; layer--) {
     const int rows = layer == 4 ? GD_OUT_PAD : GD_HID;
     const int wofs = layer == 1 ? GD_W1 : (layer == 2 ? GD_W2 : (layer == 3 ? GD_W3 : GD_W4));
-    /* dW = D . A_{layer-1}^T : M = rows, N = 64 features, K = 64 records */
-    for (int mt = 0; mt < rows / 16; mt++)
+    /* W^T's operands for D_{layer-1}, on their way while dW is computed */
+    const int kts = rows / 16, lda = rows;
+    gh4 wt[4][4];
+    if (layer > 1) {
+      const _Float16 *WT = a.Wh + GD_H_WT(layer - 1);
+#pragma unroll
+      for (int mt = 0; mt < 4; mt++)
+#pragma unroll
+        for (int kt = 0; kt < 4; kt++)
+          if (kt < kts) wt[mt][kt] = *reinterpret_cast<const gh4 *>(WT + (16 * mt + r) * lda + 16 * kt + 4 * g);
+    }
+    /* dW = D . A_{layer-1}^T : M = rows (16 a wave), N = 64 features, K = 64 records */
+    if (16 * w < rows) {
+      gh4 av[4];
+#pragma unroll
+      for (int kt = 0; kt < 4; kt++) av[kt] = *reinterpret_cast<const gh4 *>(&DZ[(16 * w + r) * GT_LD + 16 * kt + 4 * g]);
+#pragma unroll
       for (int nt = 0; nt < 4; nt++) {
         gf4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int kt = 0; kt < 4; kt++) {
-          const gh4 av = *reinterpret_cast<const gh4 *>(&DZ[(16 * mt + r) * GT_LD + 16 * kt + 4 * g]);
           const gh4 bv = *reinterpret_cast<const gh4 *>(&H[layer - 1][(16 * nt + r) * GT_LD + 16 * kt + 4 * g]);
-          c = __builtin_amdgcn_mfma_f32_16x16x16f16(av, bv, c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_16x16x16f16(av[kt], bv, c, 0, 0, 0);
         }
 #pragma unroll
-        for (int i = 0; i < 4; i++) part[wofs + (16 * mt + 4 * g + i) * 64 + 16 * nt + r] = ldexpf(c[i], -se);
+        for (int i = 0; i < 4; i++) part[wofs + (16 * w + 4 * g + i) * 64 + 16 * nt + r] = ldexpf(c[i], -se);
       }
+    }
     if (layer == 1) break;
     /* D_{layer-1} = (W^T . D) masked by A_{layer-1} > 0, in fp32 until the
-     * wave has picked its new scale */
-    gf4 acc[4][4];
+     * group has picked its new scale */
+    gf4 acc[4];
     float amax = 0.0f;
-    /* W^T's operands are the same for the 4 tiles: loaded once per layer */
-    const _Float16 *WT = a.Wh + GD_H_WT(layer - 1);
-    const int kts = rows / 16, lda = rows;
-    gh4 wt[4][4];
 #pragma unroll
-    for (int mt = 0; mt < 4; mt++)
+    for (int mt = 0; mt < 4; mt++) {
+      gf4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int kt = 0; kt < 4; kt++)
-        if (kt < kts) wt[mt][kt] = *reinterpret_cast<const gh4 *>(WT + (16 * mt + r) * lda + 16 * kt + 4 * g);
-    for (int nt = 0; nt < 4; nt++) {
+        if (kt < kts) c = __builtin_amdgcn_mfma_f32_16x16x16f16(wt[mt][kt], din[kt], c, 0, 0, 0);
 #pragma unroll
-      for (int mt = 0; mt < 4; mt++) {
-        gf4 c = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int kt = 0; kt < 4; kt++)
-          if (kt < kts) c = __builtin_amdgcn_mfma_f32_16x16x16f16(wt[mt][kt], din[nt][kt], c, 0, 0, 0);
-        acc[nt][mt] = c;
+      for (int i = 0; i < 4; i++) {
+        const bool on = (float)H[layer - 1][(16 * mt + 4 * g + i) * GT_LD + q] > 0.0f;
+        const float x = on ? c[i] : 0.0f;
+        c[i] = x;
+        amax = fmaxf(amax, fabsf(x));
       }
-#pragma unroll
-      for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int f = 16 * mt + 4 * g + i;
-          const bool on = (float)H[layer - 1][f * GT_LD + 16 * nt + r] > 0.0f;
-          const float x = on ? acc[nt][mt][i] : 0.0f;
-          acc[nt][mt][i] = x;
-          amax = fmaxf(amax, fabsf(x));
-        }
+      acc[mt] = c;
     }
-    const int se_new = gt_exponent(gt_wave_max(amax), se);
-    gh4 dnew[4][4];
-    for (int nt = 0; nt < 4; nt++)
+    amax = gt_wave_max(amax);
+    if (lane == 0) wmax[w] = amax;
+    __syncthreads(); /* every wave is done reading DZ */
+    const int se_new = gt_exponent(fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])), se);
 #pragma unroll
-      for (int mt = 0; mt < 4; mt++) {
-        gh4 v;
+    for (int mt = 0; mt < 4; mt++) {
+      gh4 v;
 #pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = (_Float16)ldexpf(acc[nt][mt][i], se_new - se);
-        dnew[nt][mt] = v;
+      for (int i = 0; i < 4; i++) {
+        v[i] = (_Float16)ldexpf(acc[mt][i], se_new - se);
+        DZ[(16 * mt + 4 * g + i) * GT_LD + q] = v[i];
       }
+      din[mt] = v;
+    }
     se = se_new;
-    __syncthreads(); /* every lane is done reading DZ */
-    for (int nt = 0; nt < 4; nt++)
-#pragma unroll
-      for (int mt = 0; mt < 4; mt++) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) DZ[(16 * mt + 4 * g + i) * GT_LD + 16 * nt + r] = dnew[nt][mt][i];
-        din[nt][mt] = dnew[nt][mt];
-      }
     __syncthreads();
-    {
+    if (w == layer - 2) {
       const int bofs = layer == 2 ? GD_B1 : (layer == 3 ? GD_B2 : GD_B3);
       /* this lane's row of 64 records, 8 halfs per LDS read, four independent sums */
       const gh8 *row = reinterpret_cast<const gh8 *>(&DZ[lane * GT_LD]);
@@ -462,31 +518,15 @@ __global__ __launch_bounds__(64) void k_guide_train(GuideTrainArgs a) {
   }
 }
 
-/* first stage of the gradient sum: chunk c of GD_RCHUNK wave slices per
- * parameter (grid.y = chunks), in wave order */
+/* the gradient's sum runs over chunks of GD_RCHUNK groups, each in group
+ * order, then over the chunks in order */
 #define GD_RCHUNK 16u
-__global__ __launch_bounds__(256) void k_guide_reduce(const float *partial, const uint32_t *totals, uint32_t cap,
-                                                      uint32_t step_base, uint32_t step_len, float *chunks,
-                                                      uint32_t *steps) {
-  const uint32_t p = blockIdx.x * 256u + threadIdx.x;
-  if (p >= GD_NPARAM) return;
-  const uint32_t nuse = min(totals[0], cap);
-  if (step_base >= nuse) return;
-  /* Adam's step count: steps with records only (an empty step changes nothing) */
-  if (p == 0 && blockIdx.y == 0 && steps) *steps += 1u;
-  const uint32_t waves = (min(step_len, nuse - step_base) + 63u) / 64u;
-  const uint32_t w0 = blockIdx.y * GD_RCHUNK, w1 = min(waves, w0 + GD_RCHUNK);
-  float s = 0.0f;
-  for (uint32_t w = w0; w < w1; w++) s += partial[(size_t)w * GD_NPARAM + p];
-  chunks[(size_t)blockIdx.y * GD_NPARAM + p] = s;
-}
-
 struct GuideAdamArgs {
   float *P;
   float *m;
   float *v;
   _Float16 *Wh;
-  const float *chunks;      /* first-stage sums, [chunk][GD_NPARAM] */
+  const float *partial;     /* [group][GD_NPARAM] */
   const uint32_t *totals;
   uint32_t cap, step_base, step_len;
   float lr, beta1, beta2, eps;
@@ -508,15 +548,40 @@ __device__ __forceinline__ void refresh_half(_Float16 *Wh, uint32_t p, float val
   Wh[GD_H_WT(layer) + col * rows + row] = (_Float16)val;
 }
 
-__global__ __launch_bounds__(256) void k_guide_adam(GuideAdamArgs a) {
-  const uint32_t p = blockIdx.x * 256u + threadIdx.x;
-  if (p >= GD_NPARAM) return;
+/* One step's gradient sum and Adam update: a block takes 64 parameters, wave
+ * c of it the chunks c, c + 16, .. of their group slices; wave 0 adds the chunks and
+ * updates.  (As two launches, with the chunk sums through memory, the pair took
+ * 13.4 us a step; together 6.0.) */
+__global__ __launch_bounds__(1024) void k_guide_adam(GuideAdamArgs a) {
+  __shared__ float sums[16][64];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, p = blockIdx.x * 64u + lane;
   const uint32_t nuse = min(a.totals[0], a.cap);
   if (a.step_base >= nuse) return; /* an empty step: no update */
   const uint32_t len = min(a.step_len, nuse - a.step_base);
-  const uint32_t nchunk = ((len + 63u) / 64u + GD_RCHUNK - 1u) / GD_RCHUNK;
+  const uint32_t groups = (len + 63u) / 64u, nchunk = (groups + GD_RCHUNK - 1u) / GD_RCHUNK;
   float gsum = 0.0f;
-  for (uint32_t c = 0; c < nchunk; c++) gsum += a.chunks[(size_t)c * GD_NPARAM + p];
+  for (uint32_t c0 = 0; c0 < nchunk; c0 += 16u) { /* block-uniform */
+    const uint32_t w0 = (c0 + wave) * GD_RCHUNK, w1 = min(groups, w0 + GD_RCHUNK);
+    float s = 0.0f;
+    if (p < GD_NPARAM) {
+      const float *src = a.partial + (size_t)w0 * GD_NPARAM + p;
+      if (w0 + GD_RCHUNK <= groups) {
+        float v[GD_RCHUNK];
+#pragma unroll
+        for (uint32_t k = 0; k < GD_RCHUNK; k++) v[k] = src[(size_t)k * GD_NPARAM];
+#pragma unroll
+        for (uint32_t k = 0; k < GD_RCHUNK; k++) s += v[k];
+      } else {
+        for (uint32_t k = w0; k < w1; k++) s += a.partial[(size_t)k * GD_NPARAM + p];
+      }
+    }
+    sums[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0)
+      for (uint32_t k = 0; k < min(16u, nchunk - c0); k++) gsum += sums[k][lane];
+    __syncthreads();
+  }
+  if (wave != 0 || p >= GD_NPARAM) return;
   const float gr = gsum / (float)len;
   if (a.grad_out) {
     a.grad_out[p] = gr;
@@ -618,19 +683,14 @@ void launch_guide_step(hipStream_t st, const GuideRec *rec, const float *recL, c
   ta.Wh = Wh;
   ta.P = P;
   ta.partial = partial;
-  const uint32_t waves = (step_len + 63u) / 64u;
-  hipLaunchKernelGGL(k_guide_train, dim3(waves), dim3(64), 0, st, ta);
-  /* chunk sums go behind the wave slices of the partial buffer */
-  float *chunks = partial + (size_t)waves * GD_NPARAM;
-  const uint32_t nchunk = (waves + GD_RCHUNK - 1u) / GD_RCHUNK;
-  hipLaunchKernelGGL(k_guide_reduce, dim3((GD_NPARAM + 255u) / 256u, nchunk), dim3(256), 0, st, partial, totals, cap,
-                     step_base, step_len, chunks, grad_out ? nullptr : totals + 3);
+  ta.steps = grad_out ? nullptr : totals + 3;
+  hipLaunchKernelGGL(k_guide_train, dim3((step_len + 63u) / 64u), dim3(256), 0, st, ta);
   GuideAdamArgs aa;
   aa.P = P;
   aa.m = m;
   aa.v = v;
   aa.Wh = Wh;
-  aa.chunks = chunks;
+  aa.partial = partial;
   aa.totals = totals;
   aa.cap = cap;
   aa.step_base = step_base;
@@ -641,7 +701,7 @@ void launch_guide_step(hipStream_t st, const GuideRec *rec, const float *recL, c
   aa.eps = 1e-8f;
   aa.steps = totals + 3;
   aa.grad_out = grad_out;
-  hipLaunchKernelGGL(k_guide_adam, dim3((GD_NPARAM + 255u) / 256u), dim3(256), 0, st, aa);
+  hipLaunchKernelGGL(k_guide_adam, dim3((GD_NPARAM + 63u) / 64u), dim3(1024), 0, st, aa);
 }
 
 void launch_guide_halves(hipStream_t st, const float *P, _Float16 *Wh) {

@@ -213,17 +213,19 @@ void launch_na_setup(hipStream_t st, const DevJob &jb, const DevItem &it, const 
 /* the rest of a pass' bounces in one launch (k_tail): entries of counts[ta.in_slot] */
 void launch_tail(hipStream_t st, const DevScene &sc, const PathBuf &pb, const TraceArgs &ta, uint32_t blocks,
                  const GuideArgs &ga);
+uint32_t guide_photon_grid_blocks();
 /* light-traced training records (k_guide_photons): n paths over the batch's
  * jobs into rec/recL[0, n), their streams keyed by (seed, round, path); grid
  * of at most `blocks` traversal blocks with a spill buffer of
  * trace_spill_words(blocks) words */
 void launch_guide_photons(hipStream_t st, const DevScene &sc, uint32_t n_jobs, GuideRec *rec, float *recL, uint32_t n,
                           uint32_t stamp, uint32_t round, uint64_t seed, uint32_t *spill, uint32_t blocks,
-                          uint32_t *cells);
-/* the guiding gate from the light-traced record counts cells[job][GD_CELLS]
- * (their job totals into cell_tot[job]) -> gate[job][GD_CELLS] */
-void launch_guide_gate(hipStream_t st, const uint32_t *cells, uint32_t *cell_tot, uint8_t *gate, uint32_t n_jobs,
-                       float density);
+                          uint32_t *fresh, uint32_t copies);
+/* the guiding gate: the record counts of the latest round, fresh[copies][job]
+ * [GD_CELLS], go into cells[job][GD_CELLS] and the job totals cell_tot[job] and
+ * are cleared; then gate[job][GD_CELLS] from these */
+void launch_guide_gate(hipStream_t st, uint32_t *fresh, uint32_t copies, uint32_t *cells, uint32_t *cell_tot,
+                       uint8_t *gate, uint32_t n_jobs, float density);
 uint32_t guide_infer_grid_blocks();
 void launch_guide_infer(hipStream_t st, const DevScene &sc, const PathBuf &pb, const GuideArgs &ga,
                         const uint32_t *queue, const uint32_t *count, uint32_t max_paths, uint32_t resident);

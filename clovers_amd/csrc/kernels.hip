@@ -2139,65 +2139,110 @@ __global__ __launch_bounds__(TRACE_BLOCK) void k_tail(DevScene sc, PathBuf pb, T
  * cosine are 1.  Records go to rec/recL[base + k]; recL = 0 where none. */
 #define PH_MAX_BOUNCES 16
 #define PH_EMITTER_TRIES 16
+/* free lanes a wave waits for before it starts new light paths */
+#define PH_REFILL 24u
+/* whether a light-sampling leaf starts light paths: a plain emitter */
+__device__ __forceinline__ bool ph_emitter(const DevScene &sc, uint32_t l) {
+  const DevMaterial &m = sc.mats[sc.lights[l].mat];
+  return m.mclass == MC_LIGHT && !m.cone && m.emit_spd >= 0;
+}
+/* A wave works through its own range of light paths: a path's length varies
+ * from one bounce to 16, so each turn of the loop is one bounce of every lane,
+ * and lanes whose path has ended start the next ones of the range together.
+ * Most of a start goes into the light tree's density, and with many
+ * light-sampling targets few of them emit: a single job's emitters are looked
+ * up once per wave instead of at every try.  2^20 paths on the prism (15
+ * targets, 2 of them emitters): 941 us with one path per thread and launch, 903
+ * so (1065 refilling every free lane, 891 from 36 on), 503 with the record
+ * counts in copies (k_guide_cell_fold). */
 __global__ __launch_bounds__(TRACE_BLOCK) void k_guide_photons(DevScene sc, uint32_t n_jobs, GuideRec *rec,
                                                                float *recL, uint32_t n, uint32_t stamp, uint32_t round,
-                                                               uint64_t seed, uint32_t *spill, uint32_t *cells) {
+                                                               uint64_t seed, uint32_t *spill, uint32_t *fresh,
+                                                               uint32_t copies) {
   __shared__ uint32_t lds_stack[STACK_LDS * TRACE_BLOCK];
   uint32_t *lst = lds_stack + threadIdx.x;
   uint32_t *gst = spill + (size_t)(blockIdx.x * TRACE_BLOCK + threadIdx.x) * STACK_GLOBAL;
+  uint32_t *cells = fresh + (size_t)(blockIdx.x % copies) * n_jobs * GD_CELLS; /* this block's copy of the counts */
   const bool any_xform = sc.has_xforms != 0;
-  for (uint32_t k = blockIdx.x * TRACE_BLOCK + threadIdx.x; k < n; k += gridDim.x * TRACE_BLOCK) {
-    const uint32_t job = k % n_jobs;
-    const DevJob &jb = sc.jobs[job];
-    uint64_t s = pcg_for_path(seed ^ 0xA0761D6478BD642Full, k, round); /* the render's seed and round */
-    float carried = 0.0f;
-    uint32_t li = 0xFFFFFFFFu;
-    if (jb.guiding && jb.n_lights)
-      for (int t = 0; t < PH_EMITTER_TRIES; t++) {
-        const uint32_t l = jb.light_base + min((uint32_t)(rnd(s) * (float)jb.n_lights), jb.n_lights - 1u);
-        const DevMaterial &lm = sc.mats[sc.lights[l].mat];
-        if (lm.mclass == MC_LIGHT && !lm.cone && lm.emit_spd >= 0) {
-          li = l;
-          break;
-        }
-      }
-    if (li != 0xFFFFFFFFu) {
-      const DevLight &E = sc.lights[li];
-      V pe, ne;
-      float area;
-      if (E.type == PT_SPHERE) {
-        const float r = E.u[0];
-        ne = random_unit_vector(s);
-        pe = mk(E.q[0], E.q[1], E.q[2]) + r * ne;
-        area = 4.0f * PI_F * r * r;
-      } else {
-        float a = rnd(s), b = rnd(s);
-        if (E.type == PT_TRI && a + b > 1.0f) {
-          a = 1.0f - a;
-          b = 1.0f - b;
-        }
-        pe = mk(E.q[0], E.q[1], E.q[2]) + a * mk(E.u[0], E.u[1], E.u[2]) + b * mk(E.v[0], E.v[1], E.v[2]);
-        ne = mk(E.n[0], E.n[1], E.n[2]);
-        area = E.w[3];
-      }
-      const uint32_t hero = (uint32_t)(((uint64_t)pcg_next(s) * 400ull) >> 32);
-      const float time = rnd(s);
-      V d = unit(tree_sample(sc, jb, pe, s));
-      const float pd = tree_pdf(sc, jb, pe, d);
-      float T = sc.spd[sc.mats[E.mat].emit_spd + hero] * dot(d, ne) * area / pd;
-      V o = pe;
-      bool specular = false;
-      for (int b = 0; b < PH_MAX_BOUNCES && T > 0.0f && isfinite(T); b++) {
-        Lane L;
-        lane_start_ray(L, o, d, time, jb.root);
-        while (L.word != CHILD_EMPTY) {
-          if (!(L.word & CHILD_LEAF)) {
-            lane_node(L, sc, lst, gst);
-          } else if (lane_leaf_step(L, sc, any_xform)) {
-            lane_pop(L, lst, gst);
+  const uint32_t waves = gridDim.x * (TRACE_BLOCK / 64), wave = blockIdx.x * (TRACE_BLOCK / 64) + (threadIdx.x >> 6);
+  uint32_t next = (uint32_t)((uint64_t)n * wave / waves);
+  const uint32_t end = (uint32_t)((uint64_t)n * (wave + 1u) / waves);
+  /* bit l: leaf l of the only job emits */
+  const bool masked = n_jobs == 1u && sc.jobs[0].n_lights <= 64u;
+  uint64_t emitters = 0;
+  if (masked) emitters = __ballot(__lane_id() < sc.jobs[0].n_lights && ph_emitter(sc, sc.jobs[0].light_base + __lane_id()));
+  bool alive = false, specular = false;
+  uint32_t k = 0, job = 0, hero = 0, bounce = 0;
+  uint64_t s = 0;
+  float T = 0.0f, time = 0.0f;
+  V o = mk(0.0f, 0.0f, 0.0f), d = o;
+  for (;;) {
+    const uint64_t idle = __ballot(!alive);
+    if (next < end && (uint32_t)__popcll(idle) >= PH_REFILL) {
+      const uint32_t id = next + __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
+      next += (uint32_t)__popcll(idle);
+      if (!alive && id < end) {
+        k = id;
+        job = k % n_jobs;
+        const DevJob &jb = sc.jobs[job];
+        s = pcg_for_path(seed ^ 0xA0761D6478BD642Full, k, round); /* the render's seed and round */
+        uint32_t li = 0xFFFFFFFFu;
+        if (jb.guiding && jb.n_lights)
+          for (int t = 0; t < PH_EMITTER_TRIES; t++) {
+            const uint32_t leaf = min((uint32_t)(rnd(s) * (float)jb.n_lights), jb.n_lights - 1u);
+            if (masked ? ((emitters >> leaf) & 1u) != 0u : ph_emitter(sc, jb.light_base + leaf)) {
+              li = jb.light_base + leaf;
+              break;
+            }
           }
+        T = 0.0f;
+        if (li != 0xFFFFFFFFu) {
+          const DevLight &E = sc.lights[li];
+          V pe, ne;
+          float area;
+          if (E.type == PT_SPHERE) {
+            const float r = E.u[0];
+            ne = random_unit_vector(s);
+            pe = mk(E.q[0], E.q[1], E.q[2]) + r * ne;
+            area = 4.0f * PI_F * r * r;
+          } else {
+            float a = rnd(s), b = rnd(s);
+            if (E.type == PT_TRI && a + b > 1.0f) {
+              a = 1.0f - a;
+              b = 1.0f - b;
+            }
+            pe = mk(E.q[0], E.q[1], E.q[2]) + a * mk(E.u[0], E.u[1], E.u[2]) + b * mk(E.v[0], E.v[1], E.v[2]);
+            ne = mk(E.n[0], E.n[1], E.n[2]);
+            area = E.w[3];
+          }
+          hero = (uint32_t)(((uint64_t)pcg_next(s) * 400ull) >> 32);
+          time = rnd(s);
+          d = unit(tree_sample(sc, jb, pe, s));
+          const float pd = tree_pdf(sc, jb, pe, d);
+          T = sc.spd[sc.mats[E.mat].emit_spd + hero] * dot(d, ne) * area / pd;
+          o = pe;
+          specular = false;
+          bounce = 0;
         }
-        if (L.best == MISS_WORD) break;
+        alive = T > 0.0f && isfinite(T);
+        if (!alive) recL[k] = 0.0f;
+      }
+      continue; /* until enough lanes have a path, or the range is used up */
+    }
+    if (!__any(alive)) break;
+    if (alive) {
+      float carried = 0.0f;
+      bool ends = true;
+      Lane L;
+      lane_start_ray(L, o, d, time, sc.jobs[job].root);
+      while (L.word != CHILD_EMPTY) {
+        if (!(L.word & CHILD_LEAF)) {
+          lane_node(L, sc, lst, gst);
+        } else if (lane_leaf_step(L, sc, any_xform)) {
+          lane_pop(L, lst, gst);
+        }
+      }
+      if (L.best != MISS_WORD) {
         const Hit h = hit_record<false>(sc, L.best, o, d, time, L.tb);
         const DevMaterial &m = sc.mats[h.material];
         if (m.mclass == MC_METAL || m.mclass == MC_GLASS) {
@@ -2207,11 +2252,11 @@ __global__ __launch_bounds__(TRACE_BLOCK) void k_guide_photons(DevScene sc, uint
           d = m.mclass == MC_METAL ? specular_dir<true>(m, d, h, hero, s) : specular_dir<false>(m, d, h, hero, s);
           o = h.p;
           specular = true;
-          continue;
-        }
-        if (m.mclass == MC_LAMBERTIAN && m.kind != CLV_MAT_ISOTROPIC && specular) {
+          bounce++;
+          ends = !(bounce < PH_MAX_BOUNCES && T > 0.0f && isfinite(T));
+        } else if (m.mclass == MC_LAMBERTIAN && m.kind != CLV_MAT_ISOTROPIC && specular) {
           GuideRec r;
-          gd_norm_pos(jb, h.p, r.p);
+          gd_norm_pos(sc.jobs[job], h.p, r.p);
           r.n[0] = h.n.x;
           r.n[1] = h.n.y;
           r.n[2] = h.n.z;
@@ -2231,10 +2276,12 @@ __global__ __launch_bounds__(TRACE_BLOCK) void k_guide_photons(DevScene sc, uint
           if (isfinite(T) && T > 0.0f) /* the gate's evidence: integer counts, so the result is deterministic */
             atomicAdd(cells + (size_t)job * GD_CELLS + gd_cell(r.p), 1u);
         }
-        break;
+      }
+      if (ends) {
+        recL[k] = isfinite(carried) && carried > 0.0f ? carried : 0.0f;
+        alive = false;
       }
     }
-    recL[k] = isfinite(carried) && carried > 0.0f ? carried : 0.0f;
   }
 }
 
@@ -2684,27 +2731,60 @@ void launch_tail(hipStream_t st, const DevScene &sc, const PathBuf &pb, const Tr
 #undef CLV_TAIL
 }
 
+/* resident blocks of the light-traced records' kernel on the current device */
+uint32_t guide_photon_grid_blocks() {
+  int per_cu = 0, dev = 0, cus = 0;
+  (void)hipGetDevice(&dev);
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_guide_photons, TRACE_BLOCK, 0);
+  return (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, cus);
+}
 void launch_guide_photons(hipStream_t st, const DevScene &sc, uint32_t n_jobs, GuideRec *rec, float *recL, uint32_t n,
                           uint32_t stamp, uint32_t round, uint64_t seed, uint32_t *spill, uint32_t blocks,
-                          uint32_t *cells) {
+                          uint32_t *fresh, uint32_t copies) {
   if (n == 0 || n_jobs == 0) return;
   hipLaunchKernelGGL(k_guide_photons, dim3(std::min(blocks, grid_for(n, TRACE_BLOCK, 1u << 30))), dim3(TRACE_BLOCK), 0,
-                     st, sc, n_jobs, rec, recL, n, stamp, round, seed, spill, cells);
+                     st, sc, n_jobs, rec, recL, n, stamp, round, seed, spill, fresh, copies);
 }
 
-/* the job totals of the light-traced record counts: one block per job */
-__global__ __launch_bounds__(1024) void k_guide_cell_tot(const uint32_t *cells, uint32_t *cell_tot) {
-  __shared__ uint32_t part[1024];
-  const uint32_t *jc = cells + (size_t)blockIdx.x * GD_CELLS;
+/* A round's record counts come in `copies` copies (launch_guide_photons):
+ * caustics put most of a round's records in a few cells, and adds to one
+ * address from all over the device wait for each other (half of the
+ * light-traced round with one copy, 2^20 paths on the prism).  Here the copies
+ * are added to the counts so far and to the job totals, and cleared.  A block
+ * covers GF_PER cells of one job. */
+#define GF_PER 4096u
+__global__ __launch_bounds__(256) void k_guide_cell_fold(uint32_t *fresh, uint32_t copies, uint32_t n_jobs, uint32_t *cells,
+                                                         uint32_t *cell_tot) {
+  __shared__ uint32_t part[4];
+  const size_t first = (size_t)blockIdx.x * GF_PER, stride = (size_t)n_jobs * GD_CELLS;
   uint32_t acc = 0;
-  for (uint32_t c = threadIdx.x; c < GD_CELLS; c += 1024u) acc += jc[c];
-  part[threadIdx.x] = acc;
-  __syncthreads();
-  for (uint32_t s = 512; s > 0; s >>= 1) {
-    if (threadIdx.x < s) part[threadIdx.x] += part[threadIdx.x + s];
-    __syncthreads();
+  for (uint32_t c = threadIdx.x * 4u; c < GF_PER; c += 1024u) {
+    uint4 sum = make_uint4(0u, 0u, 0u, 0u);
+    for (uint32_t r = 0; r < copies; r++) {
+      uint4 *p = reinterpret_cast<uint4 *>(fresh + r * stride + first + c);
+      const uint4 v = *p;
+      if (v.x | v.y | v.z | v.w) *p = make_uint4(0u, 0u, 0u, 0u);
+      sum.x += v.x;
+      sum.y += v.y;
+      sum.z += v.z;
+      sum.w += v.w;
+    }
+    if (sum.x | sum.y | sum.z | sum.w) {
+      uint4 *q = reinterpret_cast<uint4 *>(cells + first + c);
+      const uint4 v = *q;
+      *q = make_uint4(v.x + sum.x, v.y + sum.y, v.z + sum.z, v.w + sum.w);
+      acc += sum.x + sum.y + sum.z + sum.w;
+    }
   }
-  if (threadIdx.x == 0) cell_tot[blockIdx.x] = part[0];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+  if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const uint32_t t = part[0] + part[1] + part[2] + part[3];
+    if (t) atomicAdd(cell_tot + first / GD_CELLS, t);
+  }
 }
 
 /* the gate: a cell is open if the records in it and its 26 neighbours, per
@@ -2732,10 +2812,10 @@ __global__ __launch_bounds__(256) void k_guide_gate(const uint32_t *cells, const
     gate[i] = open ? 1u : 0u;
   }
 }
-void launch_guide_gate(hipStream_t st, const uint32_t *cells, uint32_t *cell_tot, uint8_t *gate, uint32_t n_jobs,
-                       float density) {
+void launch_guide_gate(hipStream_t st, uint32_t *fresh, uint32_t copies, uint32_t *cells, uint32_t *cell_tot,
+                       uint8_t *gate, uint32_t n_jobs, float density) {
   const size_t n = (size_t)n_jobs * GD_CELLS;
-  hipLaunchKernelGGL(k_guide_cell_tot, dim3(n_jobs), dim3(1024), 0, st, cells, cell_tot);
+  hipLaunchKernelGGL(k_guide_cell_fold, dim3((uint32_t)(n / GF_PER)), dim3(256), 0, st, fresh, copies, n_jobs, cells, cell_tot);
   hipLaunchKernelGGL(k_guide_gate, dim3((uint32_t)std::min<size_t>((n + 255u) / 256u, 16384u)), dim3(256), 0, st, cells,
                      cell_tot, gate, n_jobs, density);
 }
