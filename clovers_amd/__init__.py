@@ -255,8 +255,8 @@ class Renderer:
     def render(self, scene_id, opts, want_sq=False):
         """clv_render -> (xyz[H, W, 3] f32, mean of squared samples or None)."""
         W, H = opts.width, opts.height
-        out = np.zeros((H, W, 3), np.float32)
-        sq = np.zeros((H, W, 3), np.float32) if want_sq else None
+        out = np.empty((H, W, 3), np.float32)
+        sq = np.empty((H, W, 3), np.float32) if want_sq else None
         self._check(self.lib.clv_render(self.h, scene_id, C.byref(opts), out.ctypes.data,
                                         sq.ctypes.data if sq is not None else None))
         return out, sq
@@ -281,8 +281,8 @@ class Renderer:
                 out = self._reuse(outs_in[k][0], shape, "outs[%d][0]" % k)
                 sq = self._reuse(outs_in[k][1], shape, "outs[%d][1]" % k) if want_sq else None
             else:
-                out = np.zeros(shape, np.float32)
-                sq = np.zeros(shape, np.float32) if want_sq else None
+                out = np.empty(shape, np.float32)
+                sq = np.empty(shape, np.float32) if want_sq else None
             arr[k].scene_id = sid
             arr[k].use_camera = 1 if cam is not None else 0
             if cam is not None:
@@ -353,15 +353,15 @@ class Renderer:
 
     def primary_hits(self, scene_id, opts):
         W, H = opts.width, opts.height
-        ids = np.zeros((H, W), np.uint32)
-        ts = np.zeros((H, W), np.float32)
+        ids = np.empty((H, W), np.uint32)
+        ts = np.empty((H, W), np.float32)
         self._check(self.lib.clv_primary_hits(self.h, scene_id, C.byref(opts), ids.ctypes.data, ts.ctypes.data))
         return ids, ts
 
     def render_debug(self, scene_id, opts, mode):
         """clv_render_debug: abi.MODE_NORMAL_MAP / MODE_BVH_TEST_COUNT /
         MODE_PRIMITIVE_TEST_COUNT image, Xyz<E> [H, W, 3]."""
-        img = np.zeros((opts.height, opts.width, 3), np.float32)
+        img = np.empty((opts.height, opts.width, 3), np.float32)
         self._check(self.lib.clv_render_debug(self.h, scene_id, C.byref(opts), int(mode), img.ctypes.data))
         return img
 
