@@ -1595,17 +1595,33 @@ __device__ __forceinline__ bool sphere_hit(V c, float r, const Trav &L, float tm
   return false;
 }
 
+/* entries of a stack: the pending children the host allows, CHILD_EMPTY below them, and the word of a ray that is
+ * left on its way above them */
+#define TRAV_TOTAL (STACK_TOTAL + 2)
 template <int BLOCK, int DEPTH>
 struct TravStack {
   uint32_t lst;      /* LDS address of the lane's entry 0; entries are BLOCK words apart */
   uint32_t *spill;   /* this block's slices */
   static constexpr uint32_t STRIDE = 4u * BLOCK, N = DEPTH;
   __device__ __forceinline__ uint32_t *deep(uint32_t e) const {
-    return spill + (size_t)threadIdx.x * (STACK_TOTAL - DEPTH) + (e - DEPTH);
+    return spill + (size_t)threadIdx.x * (TRAV_TOTAL - DEPTH) + (e - DEPTH);
   }
   __device__ __forceinline__ void start(Trav &L) const {
     lds_st(lst, CHILD_EMPTY);
     L.sp = lst + STRIDE;
+  }
+  /* a ray that is left on its way: its word on top of the stack, the stack's end in entry 0 */
+  __device__ __forceinline__ void leave(const Trav &L) const {
+    const uint32_t e = (L.sp - lst) / STRIDE;
+    if (e < DEPTH) lds_st(L.sp, L.word);
+    else *deep(e) = L.word;
+    lds_st(lst, L.sp);
+  }
+  __device__ __forceinline__ void resume(Trav &L) const {
+    L.sp = lds_ld(lst);
+    lds_st(lst, CHILD_EMPTY);
+    const uint32_t e = (L.sp - lst) / STRIDE;
+    L.word = e < DEPTH ? lds_ld(L.sp) : *deep(e);
   }
   /* the children at distances tn[1..3] that were hit (sorted: hits first), far to near */
   __device__ __forceinline__ void push3(Trav &L, const uint32_t cw[4], const float tn[4]) const {
@@ -1615,7 +1631,7 @@ struct TravStack {
         if (tn[k] < FLT_MAX) {
           const uint32_t e = (L.sp - lst) / STRIDE;
           if (e < DEPTH) lds_st(L.sp, cw[k]);
-          else if (e < STACK_TOTAL) *deep(e) = cw[k]; /* always: the host bounds the BVH depth */
+          else if (e < TRAV_TOTAL) *deep(e) = cw[k]; /* always: the host bounds the BVH depth */
           L.sp += STRIDE;
         }
     } else { /* stores without branches; the stack grows past the ones that were hit */
@@ -1694,9 +1710,22 @@ __device__ __forceinline__ void trav_node_global(Trav &L, const Bvh4Node *nd, co
   trav_next(L, tn, cw, S);
 }
 
-/* the closest hit of a ray (L.tb, L.best: an arena record offset) */
+/* rays of a wave that are left on their way: less than one in PS_LEAVE (mesh of 1M triangles: 63.6 ms without,
+ * 57.5 at 32, 53.0 at 16, 49.6 at 8, 48.0 at 4, 48.3 at 3) */
+#define PS_LEAVE 4u
+/* The closest hit of a ray (L.tb, L.best: an arena record offset), from its
+ * start or, with `resumed`, from where it was left.  A few rays of a wave go on
+ * for long: over a third of the steps are taken for less than a quarter of its
+ * lanes.  From memory, a wave leaves once fewer than 1 / PS_LEAVE of the rays it
+ * came with are on their way: those keep their stacks, best hits and lanes
+ * (false) and go on beside the wave's next rays; a wave with a handful finishes
+ * them.  In LDS the steps are too short for that: the rounds that the leftovers
+ * fill less cost more than they save (sphere field 28.6 -> 30.2 ms, prism 16.1
+ * -> 18.8). */
 template <bool FULL, bool XF, class STACK>
-__device__ __forceinline__ void trav_ray(Trav &L, const DevScene &sc, const LdsWindow &w, const STACK &S, uint32_t root) {
+__device__ __forceinline__ bool trav_ray(Trav &L, const DevScene &sc, const LdsWindow &w, const STACK &S, uint32_t root,
+                                         bool resumed) {
+  const uint32_t few = FULL ? 0u : (uint32_t)__popcll(__ballot(true)) / PS_LEAVE;
   {
     Lane s;
     lane_start_ray(s, L.o, L.d, L.time, FULL ? 0u : root);
@@ -1704,9 +1733,13 @@ __device__ __forceinline__ void trav_ray(Trav &L, const DevScene &sc, const LdsW
     L.oi = s.oi;
     L.word = s.word;
   }
-  L.tb = FLT_MAX;
-  L.best = MISS_WORD;
-  S.start(L);
+  if (resumed) {
+    S.resume(L);
+  } else {
+    L.tb = FLT_MAX;
+    L.best = MISS_WORD;
+    S.start(L);
+  }
   if (FULL) {
     L.rx = (as_u(L.inv.x) >> 31) * 16u;
     L.ry = (as_u(L.inv.y) >> 31) * 16u + 32u;
@@ -1714,10 +1747,23 @@ __device__ __forceinline__ void trav_ray(Trav &L, const DevScene &sc, const LdsW
     L.a = dot(L.d, L.d);
     L.ra = 1.0f / L.a;
     const uint32_t nodes = lds_addr(w.nodes), prims = lds_addr(w.prims);
-    while (L.word != CHILD_EMPTY) {
-      if (!(L.word & CHILD_LEAF)) {
-        trav_node_lds(L, nodes + L.word, S);
-      } else {
+    for (;;) {
+      /* a primitive in an instance costs several nodes: while two lanes or more wait with one for every lane at
+       * a node, the wave tests primitives (features room 3.34 -> 3.23 ms; without instances both each turn:
+       * prism 16.3, by that rule 17.1) */
+      const bool node = !(L.word & CHILD_LEAF);
+      bool nodes_now = true;
+      if (XF) {
+        const uint64_t going = __ballot(L.word != CHILD_EMPTY);
+        if (going == 0u) break;
+        const uint32_t nn = (uint32_t)__popcll(__ballot(node));
+        nodes_now = 3u * nn >= (uint32_t)__popcll(going);
+      } else if (L.word == CHILD_EMPTY) {
+        break;
+      }
+      if (node) {
+        if (nodes_now) trav_node_lds(L, nodes + L.word, S);
+      } else if (!XF || (!nodes_now && L.word != CHILD_EMPTY)) {
         /* one primitive per step: a lane on a leaf of 8 does not hold up the
          * lanes taking node steps; the leaf word counts its primitives down
          * and its offset up (the same order, so the same hits) */
@@ -1748,7 +1794,11 @@ __device__ __forceinline__ void trav_ray(Trav &L, const DevScene &sc, const LdsW
     for (;;) {
       const bool leaf = L.word >= CHILD_LEAF && L.word != CHILD_EMPTY, node = L.word < CHILD_LEAF;
       const uint32_t nn = (uint32_t)__popcll(__ballot(node)), nl = (uint32_t)__popcll(__ballot(leaf));
-      if (nn + nl == 0u) break;
+      if (nn + nl <= few) { /* few: 0 for less than PS_LEAVE */
+        if (nn + nl == 0u || !(node || leaf)) break;
+        S.leave(L);
+        return false;
+      }
       if (nn >= nl) {
         if (node) trav_node_global(L, sc.nodes + L.word, S);
       } else if (leaf) {
@@ -1766,6 +1816,7 @@ __device__ __forceinline__ void trav_ray(Trav &L, const DevScene &sc, const LdsW
       }
     }
   }
+  return true;
 }
 
 /* ------------------------------------------------- whole paths, one launch --- */
@@ -1778,7 +1829,8 @@ __device__ __forceinline__ void trav_ray(Trav &L, const DevScene &sc, const LdsW
  *   trace    every lane follows its ray (the LDS-cached traversal);
  *   sort     the block's paths change lanes so that they lie in the order of
  *            their material classes: per-wave ballots give every path its place,
- *            its 17 words of state travel through LDS in two rounds.  A wave
+ *            its 17 words of state travel through LDS in two rounds (a ray that
+ *            is still on its way keeps its lane).  A wave
  *            then shades one class, or two where a boundary falls inside it;
  *   shade    shade_vertex, as the wavefront; a path that ends writes its
  *            sample's XYZ contribution at its slot (k_resolve_xyz sums the
@@ -1800,21 +1852,25 @@ __device__ __forceinline__ void trav_ray(Trav &L, const DevScene &sc, const LdsW
  * a sphere field's 33 KB, at 6 waves per SIMD (80 VGPRs); 768 threads take
  * 29.4 ms where 512 take 29.2 and leave less room for larger scenes, 512
  * threads at 5 waves and no spills 36.4.  From memory it waits on node
- * fetches: two-wave blocks, so that few rays wait for the longest one of the
- * block, at 8 waves per SIMD: the 1M-triangle mesh takes 63.7 ms, 66.8 in
- * blocks of 256 threads, 73.4 at 6 waves, 68.6 / 69.1 with node and leaf steps
- * taken in another order than by majority (node-first / both each turn).  XF, EXT and
+ * fetches: two-wave blocks at 8 waves per SIMD, and rays that are left on their
+ * way while the others are shaded (trav_ray): the 1M-triangle mesh takes 46.8
+ * ms, 48.9 in blocks of 256 threads, 47.9 of 64, 49.4 at 6 waves (before rays
+ * were left: 63.6, and 68.6 / 69.1 with node and leaf steps taken in another
+ * order than by majority: node-first / both each turn).  XF, EXT and
  * MEDIA leave out of the registers what a batch has none of: without XF the
  * sphere field goes from 32.7 to 29.2 ms.
  *
  * A wave is refilled once 16 of its lanes are free: below that the camera
  * code costs more than the idle lanes (sphere field 32.8 ms at 1, 31.4 at 8 and
- * 16, 31.8 at 32, 33.9 at 64); what is left over sorts to the block's end.
+ * 16, 31.8 at 32, 33.9 at 64); what is left over sorts to the block's end.  From
+ * memory, once 4 are: tracing is more of the time there (mesh 48.2 ms at 16, 47.1
+ * at 8, 46.8 at 4 and 1).
  *
  * Whole calls, before this kernel -> now: sphere field 1920x1080 64 spp 60.5
- * -> 31.1 ms, prism 1024^2 64 spp 33.1 -> 17.7, mesh 4 views 8 spp 138.5 -> 68,
- * Cornell 256^2 16 spp 0.695 -> 0.616. */
+ * -> 29.2 ms, prism 1024^2 64 spp 33.1 -> 16.7, mesh 4 views 8 spp 138.5 -> 49,
+ * Cornell 256^2 16 spp 0.695 -> 0.58. */
 #define PS_REFILL 16u
+#define PS_REFILL_GLOBAL 4u
 #define PS_WORDS 9 /* LDS words per lane: stack entries, or one round of the exchange */
 /* lanes of mask m below this one */
 __device__ __forceinline__ uint32_t below(uint64_t m) {
@@ -1825,9 +1881,10 @@ template <int BLOCK, bool EXT, bool MEDIA, bool FULL, bool XF>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4 : (FULL ? 6 : 8)))) void k_paths(DevScene sc, GenParams gp,
                                                                                       PathsArgs pa) {
   constexpr uint32_t WAVES = BLOCK / 64;
-  static_assert(MC_COUNT * WAVES <= 64, "one lane of a wave per (class, wave) count");
+  static_assert((MC_COUNT + 1) * WAVES <= 64, "one lane of a wave per (class or free, wave) count");
   extern __shared__ __attribute__((aligned(128))) float4 scene[]; /* rows of a plane pair differ in address bit 4 */
-  __shared__ uint32_t cnt[64];   /* paths per (class, wave) */
+  __shared__ uint32_t cnt[64];   /* paths per (class, wave), then lanes per wave whose ray is not on its way */
+  __shared__ uint8_t nth[BLOCK]; /* per wave: its n-th such lane */
   __shared__ uint32_t pool[4];   /* sample ids at hand: [0] base and [1] length of the first range, [2] base of the
                                     second (pa.chunk long), [3] ids taken since the ranges were set */
   const LdsWindow win = {scene, scene + pa.lds_nodes * 8u, pa.lds_nodes, pa.lds_node_base, pa.lds_units, pa.lds_unit_base};
@@ -1835,7 +1892,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
   uint32_t *ex = reinterpret_cast<uint32_t *>(scene + pa.lds_nodes * 8u + pa.lds_units);
   TravStack<BLOCK, PS_WORDS> S;
   S.lst = lds_addr(ex + tid);
-  S.spill = pa.spill + (size_t)blockIdx.x * BLOCK * (STACK_TOTAL - PS_WORDS);
+  S.spill = pa.spill + (size_t)blockIdx.x * BLOCK * (TRAV_TOTAL - PS_WORDS);
   {
     const float4 *gn = reinterpret_cast<const float4 *>(sc.nodes + win.nb);
     auto local = [&](float f) { /* a child word for FULL (struct Trav) */
@@ -1868,31 +1925,42 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
   V o = mk(0.0f, 0.0f, 0.0f), d = o;
   float time = 0.0f;
   bool alive = ps.slot < n;
+  uint64_t under = 0; /* the wave's lanes whose ray was left on its way */
+  ps.t = 0.0f;
+  ps.hit = 0;
   if (alive) ps.meta = camera_sample(sc, gp, ps.slot, o, d, time, ps.rng);
   for (;;) {
     /* trace */
     uint32_t cls = MC_COUNT;
     Trav L;
-    L.tb = FLT_MAX;
-    L.best = MISS_WORD;
-    rays += (uint32_t)__popcll(__ballot(alive));
+    L.tb = ps.t;
+    L.best = ps.hit;
+    const bool resumed = ((under >> lane) & 1u) != 0u;
+    bool done = true;
+    rays += (uint32_t)__popcll(__ballot(alive && !resumed));
     if (alive) {
       L.o = o;
       L.d = d;
       L.time = time;
-      trav_ray<FULL, XF>(L, sc, win, S, FULL ? 0u : sc.jobs[ps.meta >> META_JOB_SHIFT].root);
-      if (MEDIA) {
-        Lane m;
-        m.o = o;
-        m.d = d;
-        m.tb = L.tb;
-        m.best = L.best;
-        lane_media(m, sc, ps.meta, ps.rng);
-        L.tb = m.tb;
-        L.best = m.best;
+      done = trav_ray<FULL, XF>(L, sc, win, S, FULL ? 0u : sc.jobs[ps.meta >> META_JOB_SHIFT].root, resumed);
+      if (done) {
+        if (MEDIA) {
+          Lane m;
+          m.o = o;
+          m.d = d;
+          m.tb = L.tb;
+          m.best = L.best;
+          lane_media(m, sc, ps.meta, ps.rng);
+          L.tb = m.tb;
+          L.best = m.best;
+        }
+        cls = L.best != MISS_WORD ? sc.mats[sc.info[as_u(sc.prims[L.best + 1u].w)].material].mclass : MC_MISS;
+      } else {
+        ps.t = L.tb;
+        ps.hit = L.best;
       }
-      cls = L.best != MISS_WORD ? sc.mats[sc.info[as_u(sc.prims[L.best + 1u].w)].material].mclass : MC_MISS;
     }
+    under = __ballot(!done);
     /* each path's place in class order */
     uint32_t rank = 0;
 #pragma unroll
@@ -1901,6 +1969,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
       if (lane == 0) cnt[c * WAVES + wave] = (uint32_t)__popcll(m);
       if (cls == c) rank = below(m);
     }
+    const uint32_t own_free = below(~under);
+    if (lane == 0) cnt[MC_COUNT * WAVES + wave] = 64u - (uint32_t)__popcll(under);
+    if (!FULL && done) nth[wave * 64u + own_free] = (uint8_t)lane;
     __syncthreads();
     if (tid == 0 && pool[3] >= pool[1]) { /* the first range is used up: the rest of the second follows, and a new one */
       const uint32_t over = pool[3] - pool[1];
@@ -1912,25 +1983,41 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
       exhausted = base >= n;
       pool[2] = base;
     }
-    uint32_t sum = lane < MC_COUNT * WAVES ? cnt[lane] : 0u;
+    uint32_t sum = lane < (MC_COUNT + 1) * WAVES ? cnt[lane] : 0u;
     const uint32_t own = sum;
 #pragma unroll
     for (uint32_t k = 1; k < 64u; k <<= 1) {
       const uint32_t up = __shfl_up(sum, k);
       if (lane >= k) sum += up;
     }
-    const uint32_t total = __builtin_amdgcn_readlane(sum, 63);
-    if (total == 0u) break; /* the same in every wave: nothing left to trace, and the last refill found no sample */
+    const uint32_t total = __builtin_amdgcn_readlane(sum, MC_COUNT * WAVES - 1);
+    const uint32_t left = BLOCK + total - __builtin_amdgcn_readlane(sum, 63); /* rays on their way */
+    if (total + left == 0u) break; /* the same in every wave: nothing left to trace, and the last refill found no sample */
     const uint32_t excl = sum - own;
     uint32_t start[MC_COUNT];
 #pragma unroll
     for (uint32_t c = 1; c < MC_COUNT; c++) start[c] = __builtin_amdgcn_readlane(excl, c * WAVES);
-    const uint32_t dest = __shfl(excl, (int)(min(cls, MC_COUNT - 1u) * WAVES + wave)) + rank;
+    /* the place in class order is that of the lane among those without a ray on its way */
+    const uint32_t at = FULL ? tid : own_free + __builtin_amdgcn_readlane(excl, MC_COUNT * WAVES + wave) - total;
+    uint32_t dest = __shfl(excl, (int)(min(cls, MC_COUNT - 1u) * WAVES + wave)) + rank;
+    if (!FULL) {
+      uint32_t first = 0, in = 0; /* the wave that holds the place, and its first one */
+#pragma unroll
+      for (uint32_t k = 1; k < WAVES; k++) {
+        const uint32_t f = __builtin_amdgcn_readlane(excl, MC_COUNT * WAVES + k) - total;
+        if (dest >= f) {
+          first = f;
+          in = k * 64u;
+        }
+      }
+      if (cls < MC_COUNT) dest = in + nth[in + dest - first];
+    }
     /* the paths change lanes */
     uint32_t *w = ex + dest;
     const uint32_t *r = ex + tid;
     const bool moves = cls < MC_COUNT;
-    alive = tid < total;
+    const bool shades = done && at < total;
+    alive = shades || !done;
     if (moves) {
       lds_store(w, as_u(o.x));
       lds_store(w + BLOCK, as_u(o.y));
@@ -1943,7 +2030,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
       lds_store(w + 8 * BLOCK, L.best);
     }
     __syncthreads();
-    if (alive) {
+    if (shades) {
       o = mk(__uint_as_float(lds_load(r)), __uint_as_float(lds_load(r + BLOCK)), __uint_as_float(lds_load(r + 2 * BLOCK)));
       d = mk(__uint_as_float(lds_load(r + 3 * BLOCK)), __uint_as_float(lds_load(r + 4 * BLOCK)),
              __uint_as_float(lds_load(r + 5 * BLOCK)));
@@ -1963,7 +2050,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
       lds_store(w + 7 * BLOCK, ps.slot);
     }
     __syncthreads();
-    if (alive) {
+    if (shades) {
       ps.T = make_float4(__uint_as_float(lds_load(r)), __uint_as_float(lds_load(r + BLOCK)),
                          __uint_as_float(lds_load(r + 2 * BLOCK)), __uint_as_float(lds_load(r + 3 * BLOCK)));
       ps.rng = (uint64_t)lds_load(r + 4 * BLOCK) | ((uint64_t)lds_load(r + 5 * BLOCK) << 32);
@@ -1972,12 +2059,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
     }
     __syncthreads(); /* the exchange is over: the memory is the stacks' again */
     /* shade */
-    if (alive) {
+    if (shades) {
       ps.o4 = make_float4(o.x, o.y, o.z, 0.0f);
       ps.d4 = make_float4(d.x, d.y, d.z, time);
       uint32_t c = 0;
 #pragma unroll
-      for (uint32_t k = 1; k < MC_COUNT; k++) c += tid >= start[k] ? 1u : 0u;
+      for (uint32_t k = 1; k < MC_COUNT; k++) c += at >= start[k] ? 1u : 0u;
       NextPath nx;
       float4 lit = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       int end;
@@ -2005,7 +2092,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(MEDIA ? 4
     }
     /* refill */
     const uint64_t idle = __ballot(!alive);
-    if ((uint32_t)__popcll(idle) >= PS_REFILL) {
+    if ((uint32_t)__popcll(idle) >= (FULL ? PS_REFILL : PS_REFILL_GLOBAL)) {
       uint32_t base = 0;
       if (lane == 0) base = atomicAdd(&pool[3], (uint32_t)__popcll(idle));
       base = __builtin_amdgcn_readfirstlane(base);
@@ -2871,7 +2958,7 @@ void launch_guide_infer(hipStream_t st, const DevScene &sc, const PathBuf &pb, c
                      st, sc, pb, ga, queue, count);
 }
 
-/* k_paths: blocks of 12 waves that share a scene in LDS, or of 4 that read it from memory */
+/* k_paths: blocks of 8 waves that share a scene in LDS, or of 2 that read it from memory */
 #define PS_BLOCK_LDS 512
 #define PS_BLOCK_GLOBAL 128
 uint32_t paths_block(bool full) { return full ? PS_BLOCK_LDS : PS_BLOCK_GLOBAL; }
@@ -2879,7 +2966,7 @@ size_t paths_lds_bytes(bool full, uint32_t nodes, uint32_t units) {
   return (size_t)nodes * sizeof(Bvh4Node) + (size_t)units * 16u + (size_t)PS_WORDS * paths_block(full) * 4u;
 }
 size_t paths_spill_words(bool full, uint32_t blocks) {
-  return (size_t)blocks * paths_block(full) * (STACK_TOTAL - PS_WORDS);
+  return (size_t)blocks * paths_block(full) * (TRAV_TOTAL - PS_WORDS);
 }
 
 typedef void (*paths_fn)(DevScene, GenParams, PathsArgs);
