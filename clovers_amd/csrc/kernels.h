@@ -168,6 +168,7 @@ size_t trace_spill_words(uint32_t blocks);
  * loop, or persistent waves refilling lanes from an atomic work counter */
 #define TRACE_SIMPLE 0
 #define TRACE_PERSISTENT 1
+#define TRACE_MAJORITY 4 /* only chosen by the library (guided bounces from memory) */
 #define TRACE_WW 2
 #define TRACE_LDS 3
 /* LDS-cached traversal: dynamic LDS bytes for a cached prefix of `nodes` wide

@@ -783,10 +783,17 @@ __global__ __launch_bounds__(LT_BLOCK) void k_trace_lds(DevScene sc, PathBuf pb,
 /* Closest-hit kernel, one ray per thread: the block's threads take rays
  * base + threadIdx.x in a grid-stride loop; each thread runs its ray to
  * completion (node or leaf per step).  Results as in k_trace below. */
+/* ORDER: a node or a primitive per lane and turn; while-while; or, for guided
+ * bounces in scenes that are not in LDS, a turn of nodes or of primitives, by
+ * what most lanes have (uneven batch of 6 scenes 14.3 ms; 15.2 with both each
+ * turn, 17.8 through the LDS window of its largest job's scene) */
+#define ORDER_BOTH 0
+#define ORDER_WW 1
+#define ORDER_MAJORITY 2
 /* MEDIA: the instance for batches with constant media (the media pass after
  * the tree raises the traversal's registers, so the other instances leave it
  * out; batches with media always trace with this kernel) */
-template <bool COUNT, int MODE, bool WW, bool MEDIA = false>
+template <bool COUNT, int MODE, int ORDER, bool MEDIA = false>
 /* 7 waves per SIMD for the rendering instances: the traversal waits on
  * dependent node fetches, and 72 VGPRs (a few spilled outside the node loop)
  * let 7 waves hide that latency instead of the 6 that 76 VGPRs allow */
@@ -808,7 +815,7 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu((CO
     if (active) lane_start(L, pb, i);
     else L.word = CHILD_EMPTY;
     const uint32_t v0 = nvisit, t0 = ntest;
-    if (WW) {
+    if (ORDER == ORDER_WW) {
       /* while-while: the wave descends interior nodes until every lane holds
        * a leaf (or is done), then all lanes test their leaf together */
       while (__any(L.word != CHILD_EMPTY)) {
@@ -822,6 +829,17 @@ __global__ __launch_bounds__(TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu((CO
           uint32_t c = lane_leaf(L, sc, any_xform);
           if (COUNT) ntest += c;
           lane_pop(L, lst, gst);
+        }
+      }
+    } else if (ORDER == ORDER_MAJORITY) {
+      for (;;) {
+        const bool leaf = L.word >= CHILD_LEAF && L.word != CHILD_EMPTY, node = L.word < CHILD_LEAF;
+        const uint32_t nn = (uint32_t)__popcll(__ballot(node)), nl = (uint32_t)__popcll(__ballot(leaf));
+        if (nn + nl == 0u) break;
+        if (nn >= nl) {
+          if (node) lane_node(L, sc, lst, gst);
+        } else if (leaf) {
+          if (lane_leaf_step(L, sc, any_xform)) lane_pop(L, lst, gst);
         }
       }
     } else {
@@ -2703,7 +2721,7 @@ uint32_t trace_grid_blocks() {
   int dev = 0, cus = 0, per_cu = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(k_trace_simple<false, MODE_EXTEND, false>),
+  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(k_trace_simple<false, MODE_EXTEND, ORDER_BOTH>),
                                                       TRACE_BLOCK, 0);
   if (cus < 1) cus = 1;
   if (per_cu < 1) per_cu = 1;
@@ -2734,13 +2752,13 @@ void launch_trace_lds(hipStream_t st, const DevScene &sc, const PathBuf &pb, con
                       size_t lds_bytes, bool counting, int mode) {
   if (sc.has_media) { /* the host plans media batches with the plain traversal; this only keeps them correct */
     if (mode == 1)
-      hipLaunchKernelGGL((k_trace_simple<false, MODE_PRIMARY, false, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc,
+      hipLaunchKernelGGL((k_trace_simple<false, MODE_PRIMARY, ORDER_BOTH, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc,
                          pb, ta);
     else if (counting)
-      hipLaunchKernelGGL((k_trace_simple<true, MODE_EXTEND, false, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb,
+      hipLaunchKernelGGL((k_trace_simple<true, MODE_EXTEND, ORDER_BOTH, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb,
                          ta);
     else
-      hipLaunchKernelGGL((k_trace_simple<false, MODE_EXTEND, false, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc,
+      hipLaunchKernelGGL((k_trace_simple<false, MODE_EXTEND, ORDER_BOTH, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc,
                          pb, ta);
     return;
   }
@@ -2756,38 +2774,40 @@ void launch_extend(hipStream_t st, const DevScene &sc, const PathBuf &pb, const 
                    bool counting, int variant) {
   if (sc.has_media) {
     if (counting)
-      hipLaunchKernelGGL((k_trace_simple<true, MODE_EXTEND, false, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb,
+      hipLaunchKernelGGL((k_trace_simple<true, MODE_EXTEND, ORDER_BOTH, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb,
                          ta);
     else
-      hipLaunchKernelGGL((k_trace_simple<false, MODE_EXTEND, false, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc,
+      hipLaunchKernelGGL((k_trace_simple<false, MODE_EXTEND, ORDER_BOTH, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc,
                          pb, ta);
   } else if (variant == TRACE_PERSISTENT) {
     if (counting)
       hipLaunchKernelGGL((k_trace<true, MODE_EXTEND>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
     else
       hipLaunchKernelGGL((k_trace<false, MODE_EXTEND>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
+  } else if (variant == TRACE_MAJORITY && !counting) {
+    hipLaunchKernelGGL((k_trace_simple<false, MODE_EXTEND, ORDER_MAJORITY>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
   } else if (variant == TRACE_WW) {
     if (counting)
-      hipLaunchKernelGGL((k_trace_simple<true, MODE_EXTEND, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
+      hipLaunchKernelGGL((k_trace_simple<true, MODE_EXTEND, ORDER_WW>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
     else
-      hipLaunchKernelGGL((k_trace_simple<false, MODE_EXTEND, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
+      hipLaunchKernelGGL((k_trace_simple<false, MODE_EXTEND, ORDER_WW>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
   } else {
     if (counting)
-      hipLaunchKernelGGL((k_trace_simple<true, MODE_EXTEND, false>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
+      hipLaunchKernelGGL((k_trace_simple<true, MODE_EXTEND, ORDER_BOTH>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
     else
-      hipLaunchKernelGGL((k_trace_simple<false, MODE_EXTEND, false>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
+      hipLaunchKernelGGL((k_trace_simple<false, MODE_EXTEND, ORDER_BOTH>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
   }
 }
 
 void launch_primary(hipStream_t st, const DevScene &sc, const PathBuf &pb, const TraceArgs &ta, uint32_t blocks,
                     int variant) {
   if (sc.has_media)
-    hipLaunchKernelGGL((k_trace_simple<false, MODE_PRIMARY, false, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb,
+    hipLaunchKernelGGL((k_trace_simple<false, MODE_PRIMARY, ORDER_BOTH, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb,
                        ta);
   else if (variant == TRACE_PERSISTENT)
     hipLaunchKernelGGL((k_trace<false, MODE_PRIMARY>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
   else
-    hipLaunchKernelGGL((k_trace_simple<false, MODE_PRIMARY, false>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
+    hipLaunchKernelGGL((k_trace_simple<false, MODE_PRIMARY, ORDER_BOTH>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
 }
 void launch_generate_debug(hipStream_t st, const DevScene &sc, const PathBuf &pb, const DebugArgs &da) {
   hipLaunchKernelGGL(k_generate_debug, dim3(grid_for(da.width * da.height, 256, 8192)), dim3(256), 0, st, sc, pb, da);
@@ -2795,10 +2815,10 @@ void launch_generate_debug(hipStream_t st, const DevScene &sc, const PathBuf &pb
 void launch_primary_counting(hipStream_t st, const DevScene &sc, const PathBuf &pb, const TraceArgs &ta,
                              uint32_t blocks) {
   if (sc.has_media)
-    hipLaunchKernelGGL((k_trace_simple<true, MODE_PRIMARY, false, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb,
+    hipLaunchKernelGGL((k_trace_simple<true, MODE_PRIMARY, ORDER_BOTH, true>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb,
                        ta);
   else
-    hipLaunchKernelGGL((k_trace_simple<true, MODE_PRIMARY, false>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
+    hipLaunchKernelGGL((k_trace_simple<true, MODE_PRIMARY, ORDER_BOTH>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, sc, pb, ta);
 }
 void launch_debug_color(hipStream_t st, const DevScene &sc, const PathBuf &pb, const DebugArgs &da,
                         const uint32_t *ray_counts, float *out) {
