@@ -229,12 +229,35 @@ __global__ __launch_bounds__(256) void k_bb_init(uint32_t n, const uint32_t *__r
   cid[i] = BB_LEAF | p;
 }
 
-/* nearest neighbour of every cluster among the PL_R on either side: least
- * union area, ties broken by a key of the pair alone -- the index distance,
- * then the parity of the lower index, then the lower index.  A strict order
- * on pairs makes every chain of choices end in a mutual pair (no longer
- * cycles), and among equal clusters it pairs (0,1), (2,3), ..., so that
- * coincident primitives still halve per iteration instead of forming a chain. */
+/* nearest neighbour of a cluster among the PL_R on either side: least union
+ * area, ties broken by a key of the pair alone -- the index distance, then the
+ * parity of the lower index, then the lower index.  A strict order on pairs
+ * makes every chain of choices end in a mutual pair (no longer cycles), and
+ * among equal clusters it pairs (0,1), (2,3), ..., so that coincident primitives
+ * still halve per iteration instead of forming a chain.  lo, hi: boxes of the
+ * clusters from index `first` on. */
+__device__ __forceinline__ uint32_t pl_nearest(int i, int cnt, int first, const float4 *lo, const float4 *hi) {
+  const float4 l = lo[i - first], h = hi[i - first];
+  float best = FLT_MAX;
+  int bj = -1;
+  uint32_t bkey = 0xFFFFFFFFu;
+  for (int d = -PL_R; d <= PL_R; d++) {
+    const int j = i + d;
+    if (d == 0 || j < 0 || j >= cnt) continue;
+    const float a = bb_area(bb_min(l, lo[j - first]), bb_max(h, hi[j - first]));
+    const uint32_t lo_i = (uint32_t)min(i, j);
+    /* |d| <= 16 (5 bits), parity (1 bit), lower index (26 bits, wraps only
+     * beyond 2^26 clusters, where it still orders the pairs of one window) */
+    const uint32_t key = ((uint32_t)abs(d) << 27) | ((lo_i & 1u) << 26) | (lo_i & 0x03FFFFFFu);
+    if (bj < 0 || a < best || (a == best && key < bkey)) {
+      best = a;
+      bj = j;
+      bkey = key;
+    }
+  }
+  return (uint32_t)bj;
+}
+
 __global__ __launch_bounds__(256) void k_pl_nn(uint32_t cnt, const float4 *__restrict__ cb, uint32_t *__restrict__ nn) {
   __shared__ float4 slo[256 + 2 * PL_R], shi[256 + 2 * PL_R];
   const int s = (int)(blockIdx.x * 256u) - PL_R;
@@ -247,27 +270,7 @@ __global__ __launch_bounds__(256) void k_pl_nn(uint32_t cnt, const float4 *__res
   }
   __syncthreads();
   const int i = (int)(blockIdx.x * 256u + threadIdx.x);
-  if (i >= (int)cnt) return;
-  const float4 lo = slo[threadIdx.x + PL_R], hi = shi[threadIdx.x + PL_R];
-  float best = FLT_MAX;
-  int bj = -1;
-  uint32_t bkey = 0xFFFFFFFFu;
-  for (int d = -PL_R; d <= PL_R; d++) {
-    const int j = i + d;
-    if (d == 0 || j < 0 || j >= (int)cnt) continue;
-    const int k = (int)threadIdx.x + PL_R + d;
-    const float a = bb_area(bb_min(lo, slo[k]), bb_max(hi, shi[k]));
-    const uint32_t lo_i = (uint32_t)min(i, j);
-    /* |d| <= 16 (5 bits), parity (1 bit), lower index (26 bits, wraps only
-     * beyond 2^26 clusters, where it still orders the pairs of one window) */
-    const uint32_t key = ((uint32_t)abs(d) << 27) | ((lo_i & 1u) << 26) | (lo_i & 0x03FFFFFFu);
-    if (bj < 0 || a < best || (a == best && key < bkey)) {
-      best = a;
-      bj = j;
-      bkey = key;
-    }
-  }
-  nn[i] = (uint32_t)bj;
+  if (i < (int)cnt) nn[i] = pl_nearest(i, (int)cnt, s, slo, shi);
 }
 
 /* per cluster: kept (1 in the low word) and starts a merge (1 in the high word) */
@@ -295,22 +298,77 @@ __device__ __forceinline__ void child_D(uint32_t id, float area, const float4 *_
   }
 }
 
+/* the new binary node of clusters a and b: its box, children, count, record
+ * units and the cost-optimal collapse's decisions: D(n, k) the least wide-tree
+ * cost of its subtree as at most k parts, F(n) = min(a leaf of at most
+ * LEAF_MAX_PRIMS primitives, a wide node W(n) = C_NODE A(n) + min_j
+ * D(left, j) + D(right, 4 - j)), and D(n, k) = min(F(n), min_j D(left, j) +
+ * D(right, k - j)).  bdec holds the j of W (bits 0-1), the j of D(n, 2..4)
+ * (bits 2-7, 0 = F whole) and the leaf flag (bit 8). */
+struct PlNodes {
+  float4 *bbox;
+  uint2 *bch;
+  uint4 *bmeta;
+  float4 *bD;
+  uint32_t *bdec;
+  const uint32_t *unit;
+  const float4 *src;
+};
+__device__ __forceinline__ void pl_merge(const PlNodes &t, uint32_t node, uint32_t a, uint32_t b, float4 lo, float4 hi,
+                                         float4 lo2, float4 hi2, float4 &ulo, float4 &uhi) {
+  const BMeta ma = child_meta(a, t.bmeta, t.unit, t.src), mb = child_meta(b, t.bmeta, t.unit, t.src);
+  ulo = bb_min(lo, lo2);
+  uhi = bb_max(hi, hi2);
+  const float A = bb_area(ulo, uhi), Aa = bb_area(lo, hi), Ab = bb_area(lo2, hi2);
+  const uint32_t count = ma.count + mb.count;
+  float da[4], db[4], dn[4];
+  child_D(a, Aa, t.bD, da);
+  child_D(b, Ab, t.bD, db);
+  float bw = FLT_MAX;
+  uint32_t dec = 1u;
+#pragma unroll
+  for (int jj = 1; jj <= 3; jj++) {
+    const float c = da[jj - 1] + db[3 - jj];
+    if (c < bw) {
+      bw = c;
+      dec = (uint32_t)jj;
+    }
+  }
+  const float W = DP_C_NODE * A + bw;
+  const float L = count <= LEAF_MAX_PRIMS ? DP_C_PRIM * A * (float)count : FLT_MAX;
+  const bool leafy = L <= W;
+  const float F = leafy ? L : W;
+  dn[0] = F;
+#pragma unroll
+  for (int k = 2; k <= 4; k++) {
+    float dk = F;
+    uint32_t sk = 0;
+#pragma unroll
+    for (int jj = 1; jj < k; jj++) {
+      const float c = da[jj - 1] + db[k - jj - 1];
+      if (c < dk) {
+        dk = c;
+        sk = (uint32_t)jj;
+      }
+    }
+    dn[k - 1] = dk;
+    dec |= sk << (2 * (k - 1));
+  }
+  dec |= leafy ? 0x100u : 0u;
+  t.bbox[2u * node] = ulo;
+  t.bbox[2u * node + 1u] = uhi;
+  t.bch[node] = make_uint2(a, b);
+  t.bmeta[node] = make_uint4(count, ma.units + mb.units, __float_as_uint(F), leafy ? 1u : 0u);
+  t.bD[node] = make_float4(dn[0], dn[1], dn[2], dn[3]);
+  t.bdec[node] = dec;
+}
+
 /* merge mutual pairs into new binary nodes (numbered node0 + merge prefix) and
- * compact the survivors in order; pre = exclusive prefix of the flags.  Each
- * new node gets its count, record units and the cost-optimal collapse's
- * decisions: D(n, k) the least wide-tree cost of its subtree as at most k
- * parts, F(n) = min(a leaf of at most LEAF_MAX_PRIMS primitives, a wide node
- * W(n) = C_NODE A(n) + min_j D(left, j) + D(right, 4 - j)), and
- * D(n, k) = min(F(n), min_j D(left, j) + D(right, k - j)).  bdec holds the j
- * of W (bits 0-1), the j of D(n, 2..4) (bits 2-7, 0 = F whole) and the leaf
- * flag (bit 8). */
+ * compact the survivors in order; pre = exclusive prefix of the flags */
 __global__ __launch_bounds__(256) void k_pl_compact(uint32_t cnt, const uint32_t *__restrict__ nn,
                                                     const uint64_t *__restrict__ pre, const float4 *__restrict__ cbA,
                                                     const uint32_t *__restrict__ cidA, float4 *__restrict__ cbB,
-                                                    uint32_t *__restrict__ cidB, uint32_t node0, float4 *__restrict__ bbox,
-                                                    uint2 *__restrict__ bch, uint4 *__restrict__ bmeta,
-                                                    float4 *__restrict__ bD, uint32_t *__restrict__ bdec,
-                                                    const uint32_t *__restrict__ unit, const float4 *__restrict__ src) {
+                                                    uint32_t *__restrict__ cidB, uint32_t node0, PlNodes t) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
   if (i >= cnt) return;
   const uint32_t j = nn[i];
@@ -322,52 +380,8 @@ __global__ __launch_bounds__(256) void k_pl_compact(uint32_t cnt, const uint32_t
   uint32_t id = cidA[i];
   if (mutual) {
     const uint32_t node = node0 + (uint32_t)(p >> 32);
-    const float4 lo2 = cbA[2u * j], hi2 = cbA[2u * j + 1u];
-    const uint32_t a = id, b = cidA[j];
-    const BMeta ma = child_meta(a, bmeta, unit, src), mb = child_meta(b, bmeta, unit, src);
-    const float4 ulo = bb_min(lo, lo2), uhi = bb_max(hi, hi2);
-    const float A = bb_area(ulo, uhi), Aa = bb_area(lo, hi), Ab = bb_area(lo2, hi2);
-    const uint32_t count = ma.count + mb.count;
-    float da[4], db[4], dn[4];
-    child_D(a, Aa, bD, da);
-    child_D(b, Ab, bD, db);
-    float bw = FLT_MAX;
-    uint32_t dec = 1u;
-#pragma unroll
-    for (int jj = 1; jj <= 3; jj++) {
-      const float c = da[jj - 1] + db[3 - jj];
-      if (c < bw) {
-        bw = c;
-        dec = (uint32_t)jj;
-      }
-    }
-    const float W = DP_C_NODE * A + bw;
-    const float L = count <= LEAF_MAX_PRIMS ? DP_C_PRIM * A * (float)count : FLT_MAX;
-    const bool leafy = L <= W;
-    const float F = leafy ? L : W;
-    dn[0] = F;
-#pragma unroll
-    for (int k = 2; k <= 4; k++) {
-      float dk = F;
-      uint32_t sk = 0;
-#pragma unroll
-      for (int jj = 1; jj < k; jj++) {
-        const float c = da[jj - 1] + db[k - jj - 1];
-        if (c < dk) {
-          dk = c;
-          sk = (uint32_t)jj;
-        }
-      }
-      dn[k - 1] = dk;
-      dec |= sk << (2 * (k - 1));
-    }
-    dec |= leafy ? 0x100u : 0u;
-    bbox[2u * node] = ulo;
-    bbox[2u * node + 1u] = uhi;
-    bch[node] = make_uint2(a, b);
-    bmeta[node] = make_uint4(count, ma.units + mb.units, __float_as_uint(F), leafy ? 1u : 0u);
-    bD[node] = make_float4(dn[0], dn[1], dn[2], dn[3]);
-    bdec[node] = dec;
+    float4 ulo, uhi;
+    pl_merge(t, node, id, cidA[j], lo, hi, cbA[2u * j], cbA[2u * j + 1u], ulo, uhi);
     lo = ulo;
     hi = uhi;
     id = node;
@@ -375,6 +389,81 @@ __global__ __launch_bounds__(256) void k_pl_compact(uint32_t cnt, const uint32_t
   cbB[2u * dst] = lo;
   cbB[2u * dst + 1u] = hi;
   cidB[dst] = id;
+}
+
+/* The last clusters, at most PL_TAIL of them: one block runs every iteration
+ * that is left, the clusters in LDS, with the same choices, order and numbers as
+ * the kernels above.  With those an iteration is six launches and a readback,
+ * whatever its size, and more than half of a tree's iterations are these (28 of
+ * 47 for 82k triangles): 1,280 / 82k triangles are uploaded in 1.0 / 7.8 ms
+ * instead of 1.8 / 8.6.  out: node0, iterations; no progress leaves more than one cluster (never: a
+ * chain of nearest neighbours ends in a mutual pair). */
+#define PL_TAIL 1024u
+__global__ __launch_bounds__(PL_TAIL) void k_pl_tail(uint32_t cnt, float4 *cb, uint32_t *cid, uint32_t node0, PlNodes t,
+                                                     uint32_t *out) {
+  __shared__ float4 lo[PL_TAIL], hi[PL_TAIL];
+  __shared__ uint32_t id[PL_TAIL], nn[PL_TAIL], keeps[PL_TAIL / 64], merges[PL_TAIL / 64];
+  const uint32_t i = threadIdx.x, wave = i >> 6, lane = i & 63u;
+  const uint64_t lt = (1ull << lane) - 1ull;
+  if (i < cnt) {
+    lo[i] = cb[2u * i];
+    hi[i] = cb[2u * i + 1u];
+    id[i] = cid[i];
+  }
+  uint32_t iters = 0;
+  __syncthreads();
+  while (cnt > 1u) {
+    if (i < cnt) nn[i] = pl_nearest((int)i, (int)cnt, 0, lo, hi);
+    __syncthreads();
+    const uint32_t j = i < cnt ? nn[i] : i;
+    const bool mutual = i < cnt && nn[j] == i, keep = i < cnt && !(mutual && j < i), merge = mutual && i < j;
+    const uint64_t mk = __ballot(keep), mm = __ballot(merge);
+    if (lane == 0) {
+      keeps[wave] = (uint32_t)__popcll(mk);
+      merges[wave] = (uint32_t)__popcll(mm);
+    }
+    __syncthreads();
+    uint32_t dst = (uint32_t)__popcll(mk & lt), node = node0 + (uint32_t)__popcll(mm & lt), kept = 0, merged = 0;
+    for (uint32_t w = 0; w < PL_TAIL / 64; w++) {
+      if (w < wave) {
+        dst += keeps[w];
+        node += merges[w];
+      }
+      kept += keeps[w];
+      merged += merges[w];
+    }
+    float4 l, h;
+    uint32_t c = 0;
+    if (keep) {
+      l = lo[i];
+      h = hi[i];
+      c = id[i];
+      if (merge) {
+        float4 ulo, uhi;
+        pl_merge(t, node, c, id[j], l, h, lo[j], hi[j], ulo, uhi);
+        l = ulo;
+        h = uhi;
+        c = node;
+      }
+    }
+    __syncthreads();
+    if (keep) {
+      lo[dst] = l;
+      hi[dst] = h;
+      id[dst] = c;
+    }
+    __threadfence_block(); /* the new nodes' costs are read by the next iteration */
+    __syncthreads();
+    iters++;
+    if (merged == 0u) break;
+    node0 += merged;
+    cnt = kept;
+  }
+  if (i == 0) {
+    cid[0] = id[0];
+    out[0] = node0;
+    out[1] = iters;
+  }
 }
 
 /* ------------------------------------------------------------ collapse --- */
@@ -634,15 +723,15 @@ int device_build_bvh(hipStream_t st, const DeviceBvhInput &in, Bvh4Node *nodes, 
     float4 *cbA = P.cb0, *cbB = P.cb1;
     uint32_t *cidA = P.cid0, *cidB = P.cid1;
     uint32_t cnt = n, node0 = 0, iters = 0;
-    while (cnt > 1) {
+    const PlNodes nodes_of = {P.bbox, P.bch, P.bmeta, P.bD, P.bdec, in.unit, in.src};
+    while (cnt > PL_TAIL) {
       const uint32_t gc = cdiv(cnt, 256);
       hipLaunchKernelGGL(k_pl_nn, dim3(gc), dim3(256), 0, st, cnt, (const float4 *)cbA, P.nn);
       hipLaunchKernelGGL(k_pl_flags, dim3(gc), dim3(256), 0, st, cnt, (const uint32_t *)P.nn, P.fl);
       BBCHK(hipGetLastError());
       BBCHK(scan<uint64_t>(st, P.fl, cnt, P.bsum, P.tot));
       hipLaunchKernelGGL(k_pl_compact, dim3(gc), dim3(256), 0, st, cnt, (const uint32_t *)P.nn,
-                         (const uint64_t *)P.fl, (const float4 *)cbA, (const uint32_t *)cidA, cbB, cidB, node0, P.bbox,
-                         P.bch, P.bmeta, P.bD, P.bdec, in.unit, in.src);
+                         (const uint64_t *)P.fl, (const float4 *)cbA, (const uint32_t *)cidA, cbB, cidB, node0, nodes_of);
       BBCHK(hipGetLastError());
       uint64_t tot = 0;
       BBCHK(hipMemcpyAsync(&tot, P.tot, 8, hipMemcpyDeviceToHost, st));
@@ -658,6 +747,15 @@ int device_build_bvh(hipStream_t st, const DeviceBvhInput &in, Bvh4Node *nodes, 
       std::swap(cbA, cbB);
       std::swap(cidA, cidB);
       iters++;
+    }
+    if (cnt > 1) {
+      uint32_t tail[2] = {0, 0};
+      hipLaunchKernelGGL(k_pl_tail, dim3(1), dim3(PL_TAIL), 0, st, cnt, cbA, cidA, node0, nodes_of, (uint32_t *)P.tot);
+      BBCHK(hipGetLastError());
+      BBCHK(hipMemcpyAsync(tail, P.tot, sizeof(tail), hipMemcpyDeviceToHost, st));
+      BBCHK(hipStreamSynchronize(st));
+      node0 = tail[0];
+      iters += tail[1];
     }
     if (node0 != n - 1) {
       *err = "device BVH build: wrong binary node count";
