@@ -10,8 +10,10 @@ precedes its timed draw(), render.rs:137-150).
 
 Prints one JSON line with Msamples/s (one sample = one camera path carrying 4
 hero wavelengths), the roofline of the dominant kernel (BVH traversal, its
-launch time measured with HIP events on the render stream: vector-ALU bound
-when the scene sits in LDS, memory bound otherwise), the CPU baseline (the
+launch time measured with HIP events on the render stream in renders whose
+bounces are separate launches: vector-ALU bound when the scene sits in LDS,
+memory bound otherwise; the timed steps run whole paths in one launch, with the
+same traversal inside), the CPU baseline (the
 CPU oracle -- a C++ restatement of the reference's renderer -- timed on this
 host's cores over a bounded slice of the same workload) and, nested as
 `time_to_rmse`, the metric's second half: the wall time the guided method

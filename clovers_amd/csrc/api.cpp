@@ -2,13 +2,18 @@
  * api.cpp -- the C ABI (include/clovers_hip.h) over the HIP renderer.
  *
  * clv_render is the drop-in for draw_cpu::draw (clovers-cli/src/draw_cpu.rs:26-98,
- * called at clovers-cli/src/render.rs:149).  A render is a sequence of
- * wavefront passes; pass p covers samples [p*k, p*k+k) of every pixel, with k
- * chosen so that a pass keeps ~4M paths in flight (enough waves for 256 CUs,
- * ~350 MB of path state).  Per pass:
+ * called at clovers-cli/src/render.rs:149).  A render is a sequence of passes;
+ * pass p covers samples [p*k, p*k+k) of every pixel.  A plain pass is one launch
+ * that runs whole paths (k_paths) and one that sums them:
+ *
+ *   paths                          camera, bounces and estimator of every sample
+ *   resolve                        per-pixel sums, in sample order
+ *
+ * Guided passes, and renders that are timed or counted per launch or tuned to
+ * another traversal, are wavefronts:
  *
  *   generate                       camera rays of all paths of the pass
- *   repeat max_depth+1 times:      reset counters; extend; shade
+ *   repeat max_depth+1 times:      reset counters; extend; [infer;] shade
  *   resolve                        per-sample estimator, per-pixel sums
  *
  * All launches go to the context's stream; the host never waits inside a
@@ -275,8 +280,9 @@ bool whole_paths(const clv_ctx *c, bool any_guide, uint32_t flags) {
 
 /* an untuned context's wavefront passes behind the last training round grow to
  * this many paths: the late bounces of a pass launch four kernels each for a
- * few paths (274 bytes of state and lobes per path, 4.6 GB) */
-#define MERGED_TARGET_PATHS (1u << 24)
+ * few paths (274 bytes of state and lobes per path, 9.2 GB; the guided prism
+ * takes 42.2 ms with 2^24 paths, 39.3 with 2^25, 38.2 with 2^26) */
+#define MERGED_TARGET_PATHS (1u << 25)
 
 clv_status paths_geometry(clv_ctx *c, const SceneRes *s, bool one_scene, const DevScene &ds, TraceGeom *g) {
   g->full = one_scene && paths_lds_bytes(true, s->n_nodes, s->prim_units) <= c->lds_block_bytes;

@@ -1,10 +1,12 @@
 /*
- * kernels.hip -- wavefront spectral path tracer for MI355X (gfx950).
+ * kernels.hip -- spectral path tracer for MI355X (gfx950).
  *
  * The reference evaluates one camera sample with a recursive function
  * (clovers-cli/src/trace.rs:21-122) per pixel per row thread
- * (draw_cpu.rs:101-146).  Here every sample is a path slot in HBM and a
- * bounce is two kernels over all live paths:
+ * (draw_cpu.rs:101-146).  Here a plain pass is one launch whose blocks carry
+ * paths in registers from the camera to their end (k_paths).  Where something
+ * happens between the bounces (the guiding network, timing, counting), every
+ * sample is a path slot in HBM and a bounce is two kernels over all live paths:
  *
  *   extend  closest hit of every queued ray (4-wide BVH, short per-lane stack
  *           in LDS); each hit is appended to one of five shading queues by

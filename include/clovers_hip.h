@@ -209,8 +209,8 @@ typedef struct {
   double render_ms;          /* device time of the render, HIP events on the context's stream */
   double extend_ms;          /* summed device time of the traversal launches (CLV_FLAG_TIME_KERNELS) */
   double build_ms;           /* host time of the last clv_scene_upload (spectra + BVHs) */
-  uint32_t extend_launches;  /* traversal launches of the render */
-  uint32_t passes;           /* wavefront passes (each covers a block of samples of every pixel) */
+  uint32_t extend_launches;  /* traversal launches of the render; one per pass that runs whole paths */
+  uint32_t passes;           /* passes (each covers a block of samples of every pixel) */
   uint32_t bvh_nodes;        /* wide nodes of the scene BVH */
   uint32_t bvh_width;        /* children per node */
   uint32_t node_bytes;       /* bytes per wide node */
@@ -350,7 +350,8 @@ typedef enum {
 typedef struct {
   uint32_t target_paths;    /* samples per wavefront pass (queue and path-state capacity).  At the default, 2^22, a
                                pass that runs whole paths in one launch (CLV_TRACE_LDS_CACHED, no guided job, no
-                               CLV_FLAG_TIME_KERNELS or _COUNT) holds up to 2^27: it needs 12 bytes per sample */
+                               CLV_FLAG_TIME_KERNELS or _COUNT) holds up to 2^27: it needs 12 bytes per sample;
+                               wavefront passes behind the last training round are joined up to 2^25 */
   uint32_t trace_kernel;    /* clv_trace_kernel */
   uint32_t lds_bytes;       /* dynamic LDS per block of CLV_TRACE_LDS_CACHED (<= 64512) */
   uint32_t shade_grid_cap;  /* largest grid of the shading kernel, in 256-thread blocks (the library also caps it
@@ -365,7 +366,7 @@ typedef struct {
                                the trained network in large passes without training */
   uint32_t use_graph;       /* 1 (default): a render repeated with identical arguments is captured as a hipGraph
                                on its second call and replayed from then on; never for CLV_FLAG_TIME_KERNELS
-                               or guided CLV_FLAG_GUIDE_KEEP */
+                               or a batch with a guided job */
   uint32_t guide_credit;    /* radiance a training record is credited with: 1 (default) only what arrives
                                through a specular chain or further bounces (direct light is the light-tree
                                half's to sample); 0 everything that reaches the path after the vertex */
@@ -374,7 +375,8 @@ typedef struct {
                                2^31 on), so every image sample uses the trained network */
   uint32_t tail_depth;      /* 0 (default): every bounce of a pass is a traversal and a shading launch over the
                                live paths; d > 0: from bounce d on, one launch traces and shades each remaining
-                               path to its end (the same results; fewer launches when few paths are left) */
+                               path to its end (the same results; fewer launches when few paths are left);
+                               without effect where whole paths run in one launch (trace_kernel) */
   uint32_t guide_photons;   /* light-traced training records per round (default 2^20, at most 2^24; 0 = none):
                                paths from the emitters aimed at the light-sampling targets, recorded at their
                                first diffuse hit after a specular chain */
@@ -398,9 +400,10 @@ clv_status clv_tuning_set(clv_ctx *ctx, const clv_tuning *t);
 clv_status clv_autotune(clv_ctx *ctx, const clv_job *jobs, uint32_t n_jobs, uint64_t trial_samples,
                         clv_tuning *best_out);
 
-/* The pass plan clv_render_batch would use for `jobs` under `tuning`
- * (target_paths, guide_train_spp, guide_rounds), computed on the host, no
- * device or uploaded scene needed (scene ids are not looked up).  Items are
+/* The plan of passes of `tuning`'s size for `jobs` (target_paths,
+ * guide_train_spp, guide_rounds), computed on the host, no device or uploaded
+ * scene needed (scene ids are not looked up).  clv_render_batch follows it,
+ * except that at the default target_paths it runs larger passes (see there).  Items are
  * in pass order; up to `cap` are written, *n_items and *n_passes receive the
  * full counts. */
 typedef struct {
