@@ -35,6 +35,13 @@ namespace {
 #define HELP_BYTES ((size_t)1 << 20)
 #define HELPERS 3u
 
+/* Pinned memory costs 0.4 ms and the first touch of its pages.  For a large copy that is what the runtime's own way
+ * into fresh pages costs more (a context's first four 2.8 MB images 2.4 ms, through the runtime 4.1); for small ones it
+ * is allocated once the context has sent this many times its size the runtime's way (a new context's first probe of
+ * 200x200 pixels 0.9 ms; pinned at once, a small first probe and normal map cost 0.8 ms more). */
+#define PIN_LARGE ((size_t)1 << 20)
+#define PIN_AFTER 4u
+
 inline void pause_cpu() { __builtin_ia32_pause(); }
 
 /* memory the runtime knows (pinned or device memory): it copies there by itself */
@@ -120,6 +127,7 @@ bool CopyOut::reserve() {
   stride_ = (most + COPY_CHUNK - 1) / COPY_CHUNK * COPY_CHUNK;
   const size_t need = stride_ * std::min<size_t>(2, windows_.size());
   if (pin_ && cap_ >= need) return true;
+  if (need < PIN_LARGE && direct_ < PIN_AFTER * need) return false;
   if (pin_) (void)hipHostFree(pin_);
   pin_ = nullptr;
   cap_ = 0;
@@ -245,7 +253,10 @@ hipError_t CopyOut::run(hipStream_t st, const std::vector<CopyArray> &arrays, co
   failed_ = 0;
   plan(segs);
   if (segs.empty() || !reserve()) {
-    for (const CopySeg &s : segs) direct(s);
+    for (const CopySeg &s : segs) {
+      direct(s);
+      direct_ += s.bytes;
+    }
     if (stats && err == hipSuccess) err = hipMemcpyAsync(stats_out, stats, 64, hipMemcpyDeviceToHost, st);
     const hipError_t e = hipStreamSynchronize(st);
     return err != hipSuccess ? err : e;

@@ -37,7 +37,7 @@ struct CopyArray {
  * three helpers copy what has arrived on to the caller's memory meanwhile, and
  * two windows alternate, so that the link's 51 GB/s is what bounds a large copy.
  * While the device is still rendering, the calling thread has the destination's
- * pages mapped.  A first-hit probe and a normal map at 1080p (41 MB) 3.9 ->
+ * pages mapped.  A context's first small copies go the runtime's way (PIN_AFTER).  A first-hit probe and a normal map at 1080p (41 MB) 3.9 ->
  * 1.8 ms, a 2.8 MB image's call 0.68 -> 0.50 ms, 2 x 7 MB 3.6 -> 2.7 ms.
  * With one helper the probe takes 2.2 ms, with seven 1.8; windows of 4 MB 2.0,
  * of 2 MB 2.3.
@@ -77,6 +77,7 @@ class CopyOut {
 
   char *pin_ = nullptr; /* the stats, the flags of both halves, the halves */
   size_t cap_ = 0, stride_ = 0; /* bytes of both halves, and from one to the next */
+  size_t direct_ = 0; /* bytes sent the runtime's way for want of pinned memory */
   uint32_t stamp_ = 0;
   /* the current run */
   hipStream_t st_ = nullptr;

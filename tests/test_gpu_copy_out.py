@@ -21,7 +21,10 @@ SIZES = [(1, 1), (127, 43), (128, 128), (16385, 1), (2048, 1024), (2099, 1000), 
 @pytest.fixture(scope="module")
 def scene():
     r = clovers_amd.Renderer(0)
-    return r, r.upload(synth.spheres(seed=3))
+    sid = r.upload(synth.spheres(seed=3))
+    for _ in range(3):  # a context's first small copies are the runtime's
+        r.primary_hits(sid, abi.render_opts(3001, 2003, 1, 1, seed=5))
+    return r, sid
 
 
 def _buffers(words, shift):
@@ -111,7 +114,7 @@ def test_contexts_beside_each_other(scene):
     def program(k):
         q = clovers_amd.Renderer(0)
         s = q.upload(synth.spheres(seed=3))
-        for _ in range(4):
+        for _ in range(8):
             got = q.primary_hits(s, abi.render_opts(w, h, 1, 1, seed=1))
             if not all(np.array_equal(a, b) for a, b in zip(got, want)):
                 bad.append(k)
