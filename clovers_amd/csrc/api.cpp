@@ -719,9 +719,67 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
   PassPlan pl;
   /* a frozen network is not trained: no training slices, every pass full size */
   const bool untuned = c->target_paths == DEFAULT_TARGET_PATHS;
-  plan_passes(dj, soff, whole && untuned ? WHOLE_TARGET_PATHS : c->target_paths, std::max<uint32_t>(1, c->guide.train_spp),
-              frozen ? 0u : c->guide.rounds, c->guide.warmup != 0, &pl);
-  if (!whole && untuned) merge_passes(&pl, MERGED_TARGET_PATHS);
+  GuideState &gs = c->guide;
+  /* the LDS window caches the scene with the most samples */
+  uint32_t big = 0;
+  for (uint32_t k = 1; k < n; k++)
+    if ((uint64_t)dj[k].width * dj[k].height * dj[k].spp > (uint64_t)dj[big].width * dj[big].height * dj[big].spp) big = k;
+  TraceGeom geom;
+  DevScene ds = DevScene();
+  int variant = trace_variant_for(c, any_media);
+  bool one_scene = true;
+  for (uint32_t k = 1; k < n; k++) one_scene = one_scene && sres[k] == sres[0];
+  /* Guided bounces, unless they are measured: the window of LDS pays where it holds at least half of the only scene
+   * (guided renders of 1M / 82k / 12k triangles, 1024x640, 32 spp: 43.6 / 30.2 / 21.0 ms with it, 34.8 / 25.1 / 18.9
+   * from memory; 1,280 triangles, of which the window holds less than half: 14.0 / 14.4, and 3.9 / 3.6 at 320x200,
+   * 16 spp) */
+  if (!whole && variant == TRACE_LDS && !(flags & (CLV_FLAG_TIME_KERNELS | CLV_FLAG_COUNT)) &&
+      !(one_scene && lds_trace_bytes(sres[big]->n_nodes / 2u, sres[big]->prim_units / 2u) <= c->lds_block_bytes))
+    variant = TRACE_MAJORITY;
+  /* the tail launch (k_tail): the resident grid of the plain traversal, never with per-launch timing or
+   * counting (those measure the wavefront traversal) */
+  const uint32_t tail_depth = (flags & (CLV_FLAG_TIME_KERNELS | CLV_FLAG_COUNT)) ? 0u : c->tail_depth;
+  /* light-traced training records: a round before the first pass (so the
+   * first samples are already guided) and one with every training pass */
+  const bool photon_rounds = any_guide && !frozen && gs.photons > 0 && gs.rounds > 0;
+  auto reserve = [&]() -> clv_status {
+    CHK(whole ? ensure_res(c, pl.max_paths) : ensure_paths(c, pl.max_paths));
+    CHK(ensure_pixels(c, (uint32_t)pixels));
+    CHK(ensure_tables(c, n, (uint32_t)pl.items.size()));
+    ds = arena_view(c);
+    ds.has_xforms = any_xform ? 1u : 0u;
+    ds.has_ext = any_ext ? 1u : 0u;
+    ds.has_media = any_media ? 1u : 0u;
+    geom = TraceGeom();
+    if (whole) CHK(paths_geometry(c, sres[big], one_scene, ds, &geom));
+    else CHK(trace_geometry(c, sres[big], pl.max_paths, &geom, variant));
+    if (tail_depth || photon_rounds) CHK(ensure_spill(c, std::max(c->spill_words, trace_spill_words(c->trace_blocks))));
+    if (!any_guide) return CLV_OK;
+    uint32_t recorded = 0; /* the largest pass that writes training records */
+    for (size_t p = 0; p < pl.paths.size(); p++)
+      if (!frozen && pl.train[p]) recorded = std::max(recorded, pl.paths[p]);
+    CHK(guide_ensure_lobes(c, pl.max_paths));
+    CHK(guide_ensure_paths(c, recorded));
+    return guide_ensure_partial(c, gs.step / 64u);
+  };
+  for (bool large = untuned;; large = false) {
+    pl = PassPlan();
+    plan_passes(dj, soff, whole && large ? WHOLE_TARGET_PATHS : c->target_paths, std::max<uint32_t>(1, gs.train_spp),
+                frozen ? 0u : gs.rounds, gs.warmup != 0, &pl);
+    if (!whole && large) merge_passes(&pl, MERGED_TARGET_PATHS);
+    const clv_status st = reserve();
+    if (st == CLV_OK) break;
+    if (st != CLV_ENOMEM || !large) return st;
+    /* no memory for large passes: those of the default size need 50 MB (whole paths) to 1.2 GB (guided) */
+    (void)hipGetLastError();
+    free_paths(c);
+    dfree(c->res);
+    c->res = nullptr;
+    c->cap_res = 0;
+    dfree(gs.lobes);
+    gs.lobes = nullptr;
+    gs.cap_lobes = 0;
+  }
   std::vector<uint32_t> job_left(n);
   for (uint32_t k = 0; k < n; k++) job_left[k] = dj[k].spp;
   for (DevItem &it : pl.items) {
@@ -732,50 +790,11 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
     if (job_left[it.job] == 0) it.flags |= ITEM_LAST;
   }
   const uint32_t passes = (uint32_t)pl.paths.size();
-  if (whole) CHK(ensure_res(c, pl.max_paths));
-  else CHK(ensure_paths(c, pl.max_paths));
-  CHK(ensure_pixels(c, (uint32_t)pixels));
-  CHK(ensure_tables(c, n, (uint32_t)pl.items.size()));
-  GuideState &gs = c->guide;
   if (any_guide) {
-    uint32_t recorded = 0; /* the largest pass that writes training records */
-    for (uint32_t p = 0; p < passes; p++)
-      if (!frozen && pl.train[p]) recorded = std::max(recorded, pl.paths[p]);
-    CHK(guide_ensure_lobes(c, pl.max_paths));
-    CHK(guide_ensure_paths(c, recorded));
-    CHK(guide_ensure_partial(c, gs.step / 64u));
     const bool fresh = !(flags & CLV_FLAG_GUIDE_KEEP) || !gs.init;
     if (fresh) CHK(guide_reset(c, guide_seed));
     if (gs.photons) CHK(guide_ensure_gate(c, n, fresh));
   }
-  /* the LDS window caches the scene with the most samples */
-  uint32_t big = 0;
-  for (uint32_t k = 1; k < n; k++)
-    if ((uint64_t)dj[k].width * dj[k].height * dj[k].spp > (uint64_t)dj[big].width * dj[big].height * dj[big].spp) big = k;
-  TraceGeom geom;
-  int variant = trace_variant_for(c, any_media);
-  bool one_scene = true;
-  for (uint32_t k = 1; k < n; k++) one_scene = one_scene && sres[k] == sres[0];
-  DevScene ds = arena_view(c);
-  ds.has_xforms = any_xform ? 1u : 0u;
-  ds.has_ext = any_ext ? 1u : 0u;
-  ds.has_media = any_media ? 1u : 0u;
-  /* Guided bounces, unless they are measured: the window of LDS pays where it holds at least half of the only scene
-   * (guided renders of 1M / 82k / 12k triangles, 1024x640, 32 spp: 43.6 / 30.2 / 21.0 ms with it, 34.8 / 25.1 / 18.9
-   * from memory; 1,280 triangles, of which the window holds less than half: 14.0 / 14.4, and 3.9 / 3.6 at 320x200,
-   * 16 spp) */
-  if (!whole && variant == TRACE_LDS && !(flags & (CLV_FLAG_TIME_KERNELS | CLV_FLAG_COUNT)) &&
-      !(one_scene && lds_trace_bytes(sres[big]->n_nodes / 2u, sres[big]->prim_units / 2u) <= c->lds_block_bytes))
-    variant = TRACE_MAJORITY;
-  if (whole) CHK(paths_geometry(c, sres[big], one_scene, ds, &geom));
-  else CHK(trace_geometry(c, sres[big], pl.max_paths, &geom, variant));
-  /* the tail launch (k_tail): the resident grid of the plain traversal, never with per-launch timing or
-   * counting (those measure the wavefront traversal) */
-  const uint32_t tail_depth = (flags & (CLV_FLAG_TIME_KERNELS | CLV_FLAG_COUNT)) ? 0u : c->tail_depth;
-  /* light-traced training records: a round before the first pass (so the
-   * first samples are already guided) and one with every training pass */
-  const bool photon_rounds = any_guide && !frozen && gs.photons > 0 && gs.rounds > 0;
-  if (tail_depth || photon_rounds) CHK(ensure_spill(c, std::max(c->spill_words, trace_spill_words(c->trace_blocks))));
   StreamDrain drain{c->stream}; /* dj and pl.items outlive every copy from them */
   HIPCHK(c, hipMemcpyAsync(c->jobs, dj.data(), n * sizeof(DevJob), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->items, pl.items.data(), pl.items.size() * sizeof(DevItem), hipMemcpyHostToDevice,
