@@ -351,7 +351,8 @@ typedef struct {
   uint32_t target_paths;    /* samples per wavefront pass (queue and path-state capacity).  At the default, 2^22, a
                                pass that runs whole paths in one launch (CLV_TRACE_LDS_CACHED, no guided job, no
                                CLV_FLAG_TIME_KERNELS or _COUNT) holds up to 2^27: it needs 12 bytes per sample;
-                               wavefront passes behind the last training round are joined up to 2^25 */
+                               wavefront passes behind the last training round are joined up to 2^25.
+                               Where memory is short, both keep to 2^22 */
   uint32_t trace_kernel;    /* clv_trace_kernel */
   uint32_t lds_bytes;       /* dynamic LDS per block of CLV_TRACE_LDS_CACHED (<= 64512) */
   uint32_t shade_grid_cap;  /* largest grid of the shading kernel, in 256-thread blocks (the library also caps it
