@@ -11,8 +11,6 @@
 #include <system_error>
 #include <utility>
 
-#include "kernels.h"
-
 namespace clv {
 
 namespace {
@@ -89,36 +87,51 @@ CopyOut::~CopyOut() {
 uint32_t *CopyOut::flags(size_t window) const { return (uint32_t *)(pin_ + 64) + (window & 1u) * MAX_FLAGS; }
 char *CopyOut::half(size_t window) const { return pin_ + PIN_HEAD + (window & 1u) * stride_; }
 
-/* windows_ and parts_ of a run, in the order in which the parts arrive */
+/* windows_ and parts_ of a run, in the order in which the parts arrive.  Windows lie where the segments need bytes and
+ * nowhere else: every window has parts, so that its half, and the flags that the caller waits for, are free for the
+ * window after the next only when all of it has been taken. */
 void CopyOut::plan(const std::vector<CopySeg> &segs) {
-  size_t n = 0, total = 0;
-  for (const CopyArray &a : *arrays_) n += (a.bytes + HALF_BYTES - 1) / HALF_BYTES;
+  struct Span {
+    uint32_t array;
+    size_t off, bytes;
+    uint32_t parts;
+  };
+  std::vector<Span> spans;
+  std::vector<CopySeg> in;
+  size_t total = 0;
   for (const CopySeg &s : segs) total += s.bytes;
   const size_t cut = total >= LARGE_RUN ? PART_LARGE : PART_SMALL;
-  windows_ = std::vector<Window>(n);
   parts_.clear();
-  size_t w = 0;
-  for (uint32_t a = 0; a < arrays_->size(); a++)
-    for (size_t off = 0; off < (*arrays_)[a].bytes; off += HALF_BYTES, w++) {
-      Window &win = windows_[w];
-      win.array = a;
-      win.off = off;
-      win.bytes = std::min(HALF_BYTES, (*arrays_)[a].bytes - off);
-      win.stamp = ++stamp_;
-      const size_t first = parts_.size();
-      for (const CopySeg &s : segs) {
-        if (s.array != a) continue;
-        size_t b = std::max(s.off, off);
-        const size_t e = std::min(s.off + s.bytes, off + win.bytes);
-        while (b < e) {
-          char *dst = (char *)s.dst + (b - s.off);
-          const size_t len = std::min(e - b, cut - (uintptr_t)dst % cut);
-          parts_.push_back({(uint32_t)w, b - off, len, dst});
-          b += len;
+  for (uint32_t a = 0; a < arrays_->size(); a++) {
+    in.clear();
+    for (const CopySeg &s : segs)
+      if (s.array == a) in.push_back(s);
+    std::sort(in.begin(), in.end(), [](const CopySeg &x, const CopySeg &y) { return x.off < y.off; });
+    const size_t first = spans.size();
+    for (const CopySeg &s : in)
+      for (size_t b = s.off, e = s.off + s.bytes; b < e;) {
+        /* on in the array's last window while it has room and no chunk or more lies between */
+        Span *w = spans.size() > first ? &spans.back() : nullptr;
+        if (!w || b >= w->off + HALF_BYTES || b - (w->off + w->bytes) >= COPY_CHUNK) {
+          spans.push_back({a, b & ~(size_t)15, 0, 0});
+          w = &spans.back();
         }
+        char *dst = (char *)s.dst + (b - s.off);
+        const size_t len = std::min(std::min(e, w->off + HALF_BYTES) - b, cut - (uintptr_t)dst % cut);
+        parts_.push_back({(uint32_t)spans.size() - 1u, b - w->off, len, dst});
+        w->bytes = b + len - w->off;
+        w->parts++;
+        b += len;
       }
-      win.left = (uint32_t)(parts_.size() - first);
-    }
+  }
+  windows_ = std::vector<Window>(spans.size());
+  for (size_t k = 0; k < spans.size(); k++) {
+    windows_[k].array = spans[k].array;
+    windows_[k].off = spans[k].off;
+    windows_[k].bytes = spans[k].bytes;
+    windows_[k].stamp = ++stamp_;
+    windows_[k].left = spans[k].parts;
+  }
 }
 
 bool CopyOut::reserve() {

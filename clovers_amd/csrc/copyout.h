@@ -15,6 +15,13 @@
 
 namespace clv {
 
+/* bytes behind one flag of launch_copy_out */
+#define COPY_CHUNK ((size_t)65536)
+/* k_copy_out (kernels.hip): `bytes` from device to pinned memory; flags[k] becomes `stamp` behind chunk k, and the 8
+ * words at `stats` (may be null) go with the first */
+void launch_copy_out(hipStream_t st, const void *src, void *dst, size_t bytes, uint32_t *flags, uint32_t stamp,
+                     const uint64_t *stats, uint64_t *stats_out);
+
 /* `bytes` of one device array from `off`, to the host address `dst` */
 struct CopySeg {
   uint32_t array;
@@ -22,7 +29,7 @@ struct CopySeg {
   void *dst;
 };
 
-/* a device array that is copied out whole (16-byte aligned, whole 4-byte words) */
+/* a device array of results (16-byte aligned, whole 4-byte words) */
 struct CopyArray {
   const void *dev;
   size_t bytes;

@@ -154,10 +154,6 @@ struct ResolveParams {
 void launch_reset_counts(hipStream_t st, uint32_t *counts, uint32_t in_slot, uint32_t out_slot, uint64_t *stats);
 void launch_set_count(hipStream_t st, uint32_t *counts, uint32_t slot, uint32_t value);
 /* zero n 64-bit words with a kernel (a memset node misbehaves in captured graphs) */
-/* bytes behind one flag of launch_copy_out */
-#define COPY_CHUNK ((size_t)65536)
-void launch_copy_out(hipStream_t st, const void *src, void *dst, size_t bytes, uint32_t *flags, uint32_t stamp,
-                     const uint64_t *stats, uint64_t *stats_out);
 void launch_zero_u64(hipStream_t st, uint64_t *p, uint32_t n);
 void launch_generate(hipStream_t st, const DevScene &sc, const PathBuf &pb, const GenParams &gp);
 /* persistent traversal: grid = resident blocks of the device; spill buffer of

@@ -28,6 +28,7 @@
 #include <stdint.h>
 
 #include "clv_layout.h"
+#include "copyout.h"
 #include "kernels.h"
 
 namespace clv {
