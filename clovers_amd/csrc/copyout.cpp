@@ -16,8 +16,17 @@ namespace clv {
 namespace {
 
 /* a window's half of the pinned memory: two of 8 MB keep the link busy (150 us
- * each) and pin no more than the 16 MB a context may have staged with */
+ * each) and pin no more than the 16 MB a context may have staged with.  Their
+ * pages' first touch costs 2 to 4 ms over the threads, which a context that
+ * copies once never earns back, so it starts with half of them and grows when
+ * it has sent GROW_AFTER.  First hits and normals at 1080p, a new context's
+ * calls 1 / 2 / steady: 9.0 / 6.4 / 6.3 ms the runtime's way, 10.5 / 3.3 / 3.3
+ * with 8 MB at once, 8.5 / 4.0 / 3.3 so (6.3 in the call that grows); with 2 MB
+ * first 7.1 / 3.8 / 3.2, but results of 3 to 25 MB take a sixth longer until
+ * then. */
+#define HALF_FIRST ((size_t)4 << 20)
 #define HALF_BYTES ((size_t)8 << 20)
+#define GROW_AFTER ((size_t)128 << 20)
 #define MAX_FLAGS (HALF_BYTES / COPY_CHUNK)
 #define PIN_HEAD (64 + 2 * MAX_FLAGS * sizeof(uint32_t))
 
@@ -33,10 +42,11 @@ namespace {
 #define HELP_BYTES ((size_t)1 << 20)
 #define HELPERS 3u
 
-/* Pinned memory costs 0.4 ms and the first touch of its pages.  For a large copy that is what the runtime's own way
- * into fresh pages costs more (a context's first four 2.8 MB images 2.4 ms, through the runtime 4.1); for small ones it
- * is allocated once the context has sent this many times its size the runtime's way (a new context's first probe of
- * 200x200 pixels 0.9 ms; pinned at once, a small first probe and normal map cost 0.8 ms more). */
+/* Pinned memory costs 0.1 ms and 0.03 ms per 64 KB of its first touch.  A render's image and counters earn that back in
+ * their first call (the first copies of a process the runtime's way cost 6 ms more, the next ones 0.45 ms where a
+ * 200x200 image takes 0.21), and so does a large first-hit probe (640x360: 1.36 ms, 1.75 the runtime's way).  For small
+ * probes, which have no counters, it is allocated once the context has sent this many times their size the runtime's
+ * way (200x200: first 0.54 ms, pinned at once 0.64; then 0.21 and 0.08). */
 #define PIN_LARGE ((size_t)1 << 20)
 #define PIN_AFTER 4u
 
@@ -85,12 +95,12 @@ CopyOut::~CopyOut() {
 }
 
 uint32_t *CopyOut::flags(size_t window) const { return (uint32_t *)(pin_ + 64) + (window & 1u) * MAX_FLAGS; }
-char *CopyOut::half(size_t window) const { return pin_ + PIN_HEAD + (window & 1u) * stride_; }
+char *CopyOut::half(size_t window) const { return pin_ + PIN_HEAD + (window & 1u) * cap_; }
 
 /* windows_ and parts_ of a run, in the order in which the parts arrive.  Windows lie where the segments need bytes and
  * nowhere else: every window has parts, so that its half, and the flags that the caller waits for, are free for the
  * window after the next only when all of it has been taken. */
-void CopyOut::plan(const std::vector<CopySeg> &segs) {
+void CopyOut::plan(const std::vector<CopySeg> &segs, size_t total) {
   struct Span {
     uint32_t array;
     size_t off, bytes;
@@ -98,8 +108,6 @@ void CopyOut::plan(const std::vector<CopySeg> &segs) {
   };
   std::vector<Span> spans;
   std::vector<CopySeg> in;
-  size_t total = 0;
-  for (const CopySeg &s : segs) total += s.bytes;
   const size_t cut = total >= LARGE_RUN ? PART_LARGE : PART_SMALL;
   parts_.clear();
   for (uint32_t a = 0; a < arrays_->size(); a++) {
@@ -112,12 +120,12 @@ void CopyOut::plan(const std::vector<CopySeg> &segs) {
       for (size_t b = s.off, e = s.off + s.bytes; b < e;) {
         /* on in the array's last window while it has room and no chunk or more lies between */
         Span *w = spans.size() > first ? &spans.back() : nullptr;
-        if (!w || b >= w->off + HALF_BYTES || b - (w->off + w->bytes) >= COPY_CHUNK) {
+        if (!w || b >= w->off + half_ || b - (w->off + w->bytes) >= COPY_CHUNK) {
           spans.push_back({a, b & ~(size_t)15, 0, 0});
           w = &spans.back();
         }
         char *dst = (char *)s.dst + (b - s.off);
-        const size_t len = std::min(std::min(e, w->off + HALF_BYTES) - b, cut - (uintptr_t)dst % cut);
+        const size_t len = std::min(std::min(e, w->off + half_) - b, cut - (uintptr_t)dst % cut);
         parts_.push_back({(uint32_t)spans.size() - 1u, b - w->off, len, dst});
         w->bytes = b + len - w->off;
         w->parts++;
@@ -134,24 +142,21 @@ void CopyOut::plan(const std::vector<CopySeg> &segs) {
   }
 }
 
-bool CopyOut::reserve() {
-  size_t most = 0;
-  for (const Window &w : windows_) most = std::max(most, w.bytes);
-  stride_ = (most + COPY_CHUNK - 1) / COPY_CHUNK * COPY_CHUNK;
-  const size_t need = stride_ * std::min<size_t>(2, windows_.size());
-  if (pin_ && cap_ >= need) return true;
-  if (need < PIN_LARGE && direct_ < PIN_AFTER * need) return false;
-  if (pin_) (void)hipHostFree(pin_);
-  pin_ = nullptr;
-  cap_ = 0;
+bool CopyOut::reserve(size_t total) {
+  if (pin_ && cap_ >= half_) return true;
+  if (!pin_ && !stats_ && total < PIN_LARGE && direct_ < PIN_AFTER * total) return false;
+  char *p = nullptr;
   /* coherent: the flags and what is behind them are read while the kernel runs */
-  if (hipHostMalloc((void **)&pin_, PIN_HEAD + need, hipHostMallocCoherent) != hipSuccess) {
+  if (hipHostMalloc((void **)&p, PIN_HEAD + 2 * half_, hipHostMallocCoherent) != hipSuccess) {
     (void)hipGetLastError();
-    pin_ = nullptr;
-    return false;
+    sent_ = 0; /* not again before as much has been sent again */
+    half_ = cap_;
+    return pin_ != nullptr;
   }
-  memset(pin_, 0, PIN_HEAD);
-  cap_ = need;
+  if (pin_) (void)hipHostFree(pin_);
+  memset(p, 0, PIN_HEAD);
+  pin_ = p;
+  cap_ = half_;
   return true;
 }
 
@@ -264,8 +269,10 @@ hipError_t CopyOut::run(hipStream_t st, const std::vector<CopyArray> &arrays, co
   launched_ = 0;
   next_ = 0;
   failed_ = 0;
-  plan(segs);
-  if (segs.empty() || !reserve()) {
+  size_t total = 0;
+  for (const CopySeg &s : segs) total += s.bytes;
+  half_ = sent_ < GROW_AFTER ? HALF_FIRST : HALF_BYTES;
+  if (segs.empty() || !reserve(total)) {
     for (const CopySeg &s : segs) {
       direct(s);
       direct_ += s.bytes;
@@ -274,11 +281,11 @@ hipError_t CopyOut::run(hipStream_t st, const std::vector<CopyArray> &arrays, co
     const hipError_t e = hipStreamSynchronize(st);
     return err != hipSuccess ? err : e;
   }
+  plan(segs, total);
   if (err == hipSuccess && !pump()) err = hipErrorLaunchFailure;
   if (err == hipSuccess) {
     map_pages(segs);
-    size_t total = 0;
-    for (const CopySeg &s : segs) total += s.bytes;
+    sent_ += total;
     if (landed(0, 0, 1, true)) {
       if (total >= HELP_BYTES) {
         start_helpers();

@@ -44,10 +44,11 @@ struct CopyArray {
  * three helpers copy what has arrived on to the caller's memory meanwhile, and
  * two windows alternate, so that the link's 51 GB/s is what bounds a large copy.
  * While the device is still rendering, the calling thread has the destination's
- * pages mapped.  A context's first small copies go the runtime's way (PIN_AFTER).  A first-hit probe and a normal map at 1080p (41 MB) 3.9 ->
- * 1.8 ms, a 2.8 MB image's call 0.68 -> 0.50 ms, 2 x 7 MB 3.6 -> 2.7 ms.
- * With one helper the probe takes 2.2 ms, with seven 1.8; windows of 4 MB 2.0,
- * of 2 MB 2.3.
+ * pages mapped.  A context's first small probes go the runtime's way
+ * (PIN_AFTER), its first large copies through small windows (HALF_FIRST).  A
+ * first-hit probe and a normal map at 1080p (41 MB) 3.9 -> 1.8 ms, a 2.8 MB
+ * image's call 0.68 -> 0.50 ms, 2 x 7 MB 3.6 -> 2.7 ms.  With one helper the
+ * probe takes 2.2 ms, with seven 1.8; windows of 4 MB 2.0, of 2 MB 2.3.
  */
 class CopyOut {
  public:
@@ -70,8 +71,8 @@ class CopyOut {
     size_t off, bytes; /* in the window */
     char *dst;
   };
-  void plan(const std::vector<CopySeg> &segs);
-  bool reserve();
+  void plan(const std::vector<CopySeg> &segs, size_t total);
+  bool reserve(size_t total);
   void map_pages(const std::vector<CopySeg> &segs);
   void start_helpers();
   void helper();
@@ -83,8 +84,10 @@ class CopyOut {
   char *half(size_t window) const;
 
   char *pin_ = nullptr; /* the stats, the flags of both halves, the halves */
-  size_t cap_ = 0, stride_ = 0; /* bytes of both halves, and from one to the next */
+  size_t cap_ = 0;      /* bytes of a half */
+  size_t half_ = 0;     /* largest window of the current run */
   size_t direct_ = 0; /* bytes sent the runtime's way for want of pinned memory */
+  size_t sent_ = 0;   /* bytes sent through the windows */
   uint32_t stamp_ = 0;
   /* the current run */
   hipStream_t st_ = nullptr;

@@ -15,6 +15,7 @@
 #include <mutex>
 #include <random>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "../clovers_amd/csrc/copyout.h"
@@ -69,6 +70,8 @@ struct Stream {
 
 std::vector<std::pair<const char *, size_t>> g_known; /* destinations that the runtime knows */
 std::atomic<size_t> g_link{0};                        /* bytes that launches have written */
+size_t g_pinned = 0, g_allocs = 0;                    /* bytes of pinned memory now; allocations so far */
+std::vector<std::pair<void *, size_t>> g_blocks;
 
 }  // namespace
 
@@ -82,9 +85,14 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
 hipError_t hipGetLastError(void) { return hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned int) {
   *p = aligned_alloc(4096, (n + 4095) / 4096 * 4096);
+  g_blocks.push_back({*p, n});
+  g_pinned += n;
+  g_allocs++;
   return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipHostFree(void *p) {
+  for (auto &b : g_blocks)
+    if (b.first == p) g_pinned -= std::exchange(b, {}).second;
   free(p);
   return hipSuccess;
 }
@@ -211,6 +219,18 @@ int main(int argc, char **argv) {
     good = one(fresh, cases[k], k) && good;
     printf("case %u, its next call: ", k);
     good = one(fresh, cases[k], k + 100) && good;
+  }
+  /* what a context pins: little until it has copied a lot, then the large windows, once */
+  {
+    const size_t before = g_pinned, allocs = g_allocs;
+    clv::CopyOut co;
+    for (uint32_t k = 0; k < 40; k++) {
+      printf("large call %u: ", k);
+      good = one(co, {{{16 * MB, F, F}}}, k) && good;
+      const size_t pinned = g_pinned - before;
+      if (k < 4 ? pinned > 9 * MB : k == 39 && (pinned < 16 * MB || pinned > 17 * MB)) good = false, printf("FAILED: pinned %zu\n", pinned);
+    }
+    if (g_allocs - allocs != 2) good = false, printf("FAILED: %zu allocations\n", g_allocs - allocs);
   }
   return good ? 0 : 1;
 }

@@ -1,7 +1,8 @@
 """Results on their way to the caller's memory (copyout.cpp), without a GPU: compiled against a stand-in for the
 runtime whose stream runs every launch at once, as a device that is always ahead of the caller, or in a thread of
 its own.  Destinations pinned and pageable in every order: each gets its bytes and nothing beside them is written, no
-call fails, and what the runtime copies by itself does not go through the windows too."""
+call fails, and what the runtime copies by itself does not go through the windows too.  A context's first large
+copies pin little memory: the first touch of its pages is part of their time."""
 import os
 import subprocess
 
