@@ -503,12 +503,12 @@ DevJob make_job(const SceneRes *s, const clv_camera_init &cam, const clv_render_
 /* ------------------------------------------------------------ guiding --- */
 clv_status guide_ensure_net(clv_ctx *c) {
   GuideState &g = c->guide;
-  if (g.P) return CLV_OK;
-  HIPCHK(c, dalloc(&g.P, GD_NPARAM));
-  HIPCHK(c, dalloc(&g.M, GD_NPARAM));
-  HIPCHK(c, dalloc(&g.V, GD_NPARAM));
-  HIPCHK(c, dalloc(&g.Wh, GD_NHALF));
-  HIPCHK(c, dalloc(&g.totals, 4));
+  /* each by itself: a call may have run out of memory between them */
+  if (!g.P) HIPCHK(c, dalloc(&g.P, GD_NPARAM));
+  if (!g.M) HIPCHK(c, dalloc(&g.M, GD_NPARAM));
+  if (!g.V) HIPCHK(c, dalloc(&g.V, GD_NPARAM));
+  if (!g.Wh) HIPCHK(c, dalloc(&g.Wh, GD_NHALF));
+  if (!g.totals) HIPCHK(c, dalloc(&g.totals, 4));
   if (!g.host_totals) {
     void *hp = nullptr;
     if (hipHostMalloc(&hp, 4 * sizeof(uint32_t), hipHostMallocDefault) == hipSuccess) g.host_totals = (uint32_t *)hp;
@@ -613,29 +613,30 @@ clv_status guide_reset(clv_ctx *c, uint64_t seed) {
 uint32_t gate_copies(uint32_t n_jobs) { return std::max<uint32_t>(1u, GATE_COPIES / n_jobs); }
 size_t gate_fresh_jobs(uint32_t n_jobs) { return std::max<uint32_t>(GATE_COPIES, n_jobs); }
 
-/* gate buffers for n jobs; clear = zero the counts (a fresh network) */
-clv_status guide_ensure_gate(clv_ctx *c, uint32_t n, bool clear) {
+/* zero the gate's counts (a fresh network) */
+clv_status guide_clear_gate(clv_ctx *c) {
   GuideState &g = c->guide;
-  if (n > g.gate_jobs) {
-    dfree(g.cells); dfree(g.cell_tot); dfree(g.gate); dfree(g.fresh);
-    g.cells = g.cell_tot = g.fresh = nullptr;
-    g.gate = nullptr;
-    g.gate_jobs = 0;
-    HIPCHK(c, dalloc(&g.cells, (size_t)n * GD_CELLS));
-    HIPCHK(c, dalloc(&g.cell_tot, n));
-    HIPCHK(c, dalloc(&g.fresh, gate_fresh_jobs(n) * GD_CELLS));
-    HIPCHK(c, dalloc(&g.gate, (size_t)n * GD_CELLS));
-    g.gate_jobs = n;
-    clear = true;
-  }
-  if (clear) {
-    HIPCHK(c, hipMemsetAsync(g.cells, 0, (size_t)g.gate_jobs * GD_CELLS * sizeof(uint32_t), c->stream));
-    HIPCHK(c, hipMemsetAsync(g.cell_tot, 0, (size_t)g.gate_jobs * sizeof(uint32_t), c->stream));
-    HIPCHK(c, hipMemsetAsync(g.fresh, 0, gate_fresh_jobs(g.gate_jobs) * GD_CELLS * sizeof(uint32_t),
-                             c->stream));
-    g.gate_valid = false;
-  }
+  HIPCHK(c, hipMemsetAsync(g.cells, 0, (size_t)g.gate_jobs * GD_CELLS * sizeof(uint32_t), c->stream));
+  HIPCHK(c, hipMemsetAsync(g.cell_tot, 0, (size_t)g.gate_jobs * sizeof(uint32_t), c->stream));
+  HIPCHK(c, hipMemsetAsync(g.fresh, 0, gate_fresh_jobs(g.gate_jobs) * GD_CELLS * sizeof(uint32_t), c->stream));
+  g.gate_valid = false;
   return CLV_OK;
+}
+
+/* gate buffers for n jobs; new ones hold no counts */
+clv_status guide_ensure_gate(clv_ctx *c, uint32_t n) {
+  GuideState &g = c->guide;
+  if (n <= g.gate_jobs) return CLV_OK;
+  dfree(g.cells); dfree(g.cell_tot); dfree(g.gate); dfree(g.fresh);
+  g.cells = g.cell_tot = g.fresh = nullptr;
+  g.gate = nullptr;
+  g.gate_jobs = 0;
+  HIPCHK(c, dalloc(&g.cells, (size_t)n * GD_CELLS));
+  HIPCHK(c, dalloc(&g.cell_tot, n));
+  HIPCHK(c, dalloc(&g.fresh, gate_fresh_jobs(n) * GD_CELLS));
+  HIPCHK(c, dalloc(&g.gate, (size_t)n * GD_CELLS));
+  g.gate_jobs = n;
+  return guide_clear_gate(c);
 }
 
 /* light-traced records of a round (k_guide_photons) behind the record slots
@@ -760,7 +761,9 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
       if (!frozen && pl.train[p]) recorded = std::max(recorded, pl.paths[p]);
     CHK(guide_ensure_lobes(c, pl.max_paths));
     CHK(guide_ensure_paths(c, recorded));
-    return guide_ensure_partial(c, gs.step / 64u);
+    CHK(guide_ensure_partial(c, gs.step / 64u));
+    CHK(guide_ensure_net(c));
+    return gs.photons ? guide_ensure_gate(c, n) : CLV_OK;
   };
   for (bool large = untuned;; large = false) {
     pl = PassPlan();
@@ -793,7 +796,7 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
   if (any_guide) {
     const bool fresh = !(flags & CLV_FLAG_GUIDE_KEEP) || !gs.init;
     if (fresh) CHK(guide_reset(c, guide_seed));
-    if (gs.photons) CHK(guide_ensure_gate(c, n, fresh));
+    if (fresh && gs.photons) CHK(guide_clear_gate(c));
   }
   StreamDrain drain{c->stream}; /* dj and pl.items outlive every copy from them */
   HIPCHK(c, hipMemcpyAsync(c->jobs, dj.data(), n * sizeof(DevJob), hipMemcpyHostToDevice, c->stream));
