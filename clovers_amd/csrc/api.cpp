@@ -360,6 +360,42 @@ clv_status ensure_res(clv_ctx *c, uint32_t n) {
   return CLV_OK;
 }
 
+/* gives back the buffers that hold more than `keep` paths of a pass (sample contributions, path state, lobes), which
+ * any render allocates again; true if there were some */
+bool free_passes(clv_ctx *c, uint32_t keep) {
+  GuideState &g = c->guide;
+  bool any = false;
+  if (c->cap_paths > keep) {
+    free_paths(c);
+    any = true;
+  }
+  if (c->cap_res > keep) {
+    dfree(c->res);
+    c->res = nullptr;
+    c->cap_res = 0;
+    any = true;
+  }
+  if (g.cap_lobes > keep) {
+    dfree(g.lobes);
+    g.lobes = nullptr;
+    g.cap_lobes = 0;
+    any = true;
+  }
+  return any;
+}
+
+/* A context keeps the buffers of its largest passes, up to 9.2 GB.  A call that finds no memory runs again once they
+ * are given back. */
+template <class CALL>
+clv_status with_room(clv_ctx *c, CALL call) {
+  clv_status st = call();
+  if (st == CLV_ENOMEM && free_passes(c, DEFAULT_TARGET_PATHS)) {
+    (void)hipGetLastError();
+    st = call();
+  }
+  return st;
+}
+
 void free_pixels(clv_ctx *c) {
   dfree(c->acc32); dfree(c->acc64); dfree(c->accsq); dfree(c->out); dfree(c->out_sq); dfree(c->ids); dfree(c->ts);
   c->acc32 = nullptr; c->acc64 = c->accsq = nullptr; c->out = c->out_sq = nullptr; c->ids = nullptr; c->ts = nullptr;
@@ -576,7 +612,7 @@ clv_status guide_ensure_paths(clv_ctx *c, uint32_t paths) {
 /* fresh parameters: He-normal hidden layers, a small output layer (broad,
  * nearly uniform lobes), zero biases, zero Adam moments */
 clv_status guide_reset(clv_ctx *c, uint64_t seed) {
-  CHK(guide_ensure_net(c));
+  CHK(with_room(c, [&] { return guide_ensure_net(c); }));
   GuideState &g = c->guide;
   std::vector<float> P(GD_NPARAM, 0.0f);
   uint64_t st = seed * 0x9E3779B97F4A7C15ull + 0x632BE59BD9B4E019ull;
@@ -765,23 +801,20 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
     CHK(guide_ensure_net(c));
     return gs.photons ? guide_ensure_gate(c, n) : CLV_OK;
   };
-  for (bool large = untuned;; large = false) {
+  for (bool large = untuned, again = false;;) {
     pl = PassPlan();
     plan_passes(dj, soff, whole && large ? WHOLE_TARGET_PATHS : c->target_paths, std::max<uint32_t>(1, gs.train_spp),
                 frozen ? 0u : gs.rounds, gs.warmup != 0, &pl);
     if (!whole && large) merge_passes(&pl, MERGED_TARGET_PATHS);
     const clv_status st = reserve();
     if (st == CLV_OK) break;
-    if (st != CLV_ENOMEM || !large) return st;
-    /* no memory for large passes: those of the default size need 50 MB (whole paths) to 1.2 GB (guided) */
+    if (st != CLV_ENOMEM || again) return st;
+    /* no memory: once more without the buffers of earlier large passes, and, where these passes are large ones, at
+     * the default size, which needs 50 MB (whole paths) to 1.2 GB (guided) */
     (void)hipGetLastError();
-    free_paths(c);
-    dfree(c->res);
-    c->res = nullptr;
-    c->cap_res = 0;
-    dfree(gs.lobes);
-    gs.lobes = nullptr;
-    gs.cap_lobes = 0;
+    if (!free_passes(c, large ? 0u : DEFAULT_TARGET_PATHS) && !large) return st;
+    large = false;
+    again = true;
   }
   std::vector<uint32_t> job_left(n);
   for (uint32_t k = 0; k < n; k++) job_left[k] = dj[k].spp;
@@ -1252,7 +1285,6 @@ clv_status device_bvh(clv_ctx *c, const HostScene &hs, const ArenaBase &b, Devic
 }
 
 clv_status upload_scene(clv_ctx *c, const clv_scene_desc *desc, uint32_t builder, uint32_t *scene_id) {
-  if (!c || !scene_id || builder > CLV_BUILD_DEVICE) return CLV_EINVAL;
   HIPCHK(c, hipSetDevice(c->device));
   HostScene hs;
   std::string err;
@@ -1361,11 +1393,12 @@ clv_status upload_scene(clv_ctx *c, const clv_scene_desc *desc, uint32_t builder
 
 extern "C" {
 clv_status clv_scene_upload(clv_ctx *c, const clv_scene_desc *desc, uint32_t *scene_id) {
-  return upload_scene(c, desc, CLV_BUILD_HOST, scene_id);
+  return clv_scene_upload_ex(c, desc, CLV_BUILD_HOST, scene_id);
 }
 
 clv_status clv_scene_upload_ex(clv_ctx *c, const clv_scene_desc *desc, uint32_t builder, uint32_t *scene_id) {
-  return upload_scene(c, desc, builder, scene_id);
+  if (!c || !scene_id || builder > CLV_BUILD_DEVICE) return CLV_EINVAL;
+  return with_room(c, [&] { return upload_scene(c, desc, builder, scene_id); });
 }
 
 clv_status clv_scene_validate(const clv_scene_desc *desc, clv_scene_info *info) {
@@ -1570,19 +1603,23 @@ clv_status clv_guide_eval(clv_ctx *c, const float *in, uint32_t n, float *raw, f
   HIPCHK(c, hipSetDevice(c->device));
   if (!c->guide.init) CHK(guide_reset(c, 1));
   float *din = nullptr, *draw = nullptr, *dlob = nullptr;
-  clv_status st = CLV_OK;
-  hipError_t e = dalloc(&din, 7 * (size_t)n);
-  if (e == hipSuccess) e = dalloc(&draw, (size_t)GD_OUT * n);
-  if (e == hipSuccess) e = dalloc(&dlob, (size_t)GD_OUT * n);
-  if (e == hipSuccess) e = hipMemcpyAsync(din, in, 7 * sizeof(float) * n, hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess) {
-    launch_guide_eval(c->stream, din, n, c->guide.Wh, c->guide.P, draw, dlob);
-    e = hipGetLastError();
+  clv_status st = with_room(c, [&]() -> clv_status {
+    if (!din) HIPCHK(c, dalloc(&din, 7 * (size_t)n));
+    if (!draw) HIPCHK(c, dalloc(&draw, (size_t)GD_OUT * n));
+    if (!dlob) HIPCHK(c, dalloc(&dlob, (size_t)GD_OUT * n));
+    return CLV_OK;
+  });
+  if (st == CLV_OK) {
+    hipError_t e = hipMemcpyAsync(din, in, 7 * sizeof(float) * n, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) {
+      launch_guide_eval(c->stream, din, n, c->guide.Wh, c->guide.P, draw, dlob);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess && raw) e = hipMemcpyAsync(raw, draw, sizeof(float) * GD_OUT * n, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess && lobes) e = hipMemcpyAsync(lobes, dlob, sizeof(float) * GD_OUT * n, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) st = fail(c, e == hipErrorOutOfMemory ? CLV_ENOMEM : CLV_EDEVICE, hipGetErrorString(e));
   }
-  if (e == hipSuccess && raw) e = hipMemcpyAsync(raw, draw, sizeof(float) * GD_OUT * n, hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess && lobes) e = hipMemcpyAsync(lobes, dlob, sizeof(float) * GD_OUT * n, hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  if (e != hipSuccess) st = fail(c, e == hipErrorOutOfMemory ? CLV_ENOMEM : CLV_EDEVICE, hipGetErrorString(e));
   dfree(din);
   dfree(draw);
   dfree(dlob);
@@ -1597,8 +1634,10 @@ clv_status clv_guide_grad(clv_ctx *c, const float *samples, uint32_t n, float *g
   HIPCHK(c, hipSetDevice(c->device));
   if (!c->guide.init) CHK(guide_reset(c, 1));
   GuideState &g = c->guide;
-  CHK(guide_ensure_paths(c, (n + GD_SLOTS - 1) / GD_SLOTS));
-  CHK(guide_ensure_partial(c, (n + 63) / 64));
+  CHK(with_room(c, [&]() -> clv_status {
+    CHK(guide_ensure_paths(c, (n + GD_SLOTS - 1) / GD_SLOTS));
+    return guide_ensure_partial(c, (n + 63) / 64);
+  }));
   const uint32_t stamp = ++g.stamp;
   std::vector<GuideRec> recs(n);
   std::vector<float> recL(n);
@@ -1742,9 +1781,14 @@ clv_status clv_primary_hits(clv_ctx *c, uint32_t scene_id, const clv_render_opts
   if (it == c->scenes.end()) return fail(c, CLV_EINVAL, "unknown scene id");
   HIPCHK(c, hipSetDevice(c->device));
   const uint32_t W = o->width, H = o->height, WH = W * H;
-  CHK(ensure_paths(c, WH));
-  CHK(ensure_pixels(c, WH));
-  CHK(ensure_tables(c, 1, 1));
+  TraceGeom geom;
+  const int variant = trace_variant_for(c, it->second->n_media > 0);
+  CHK(with_room(c, [&]() -> clv_status {
+    CHK(ensure_paths(c, WH));
+    CHK(ensure_pixels(c, WH));
+    CHK(ensure_tables(c, 1, 1));
+    return trace_geometry(c, it->second, 0, &geom, variant);
+  }));
   DevJob jb = make_job(it->second, it->second->camera, o);
   DevItem item;
   memset(&item, 0, sizeof(item));
@@ -1771,9 +1815,6 @@ clv_status clv_primary_hits(clv_ctx *c, uint32_t scene_id, const clv_render_opts
   ta.n_direct = WH;
   ta.ids = c->ids;
   ta.ts = c->ts;
-  TraceGeom geom;
-  const int variant = trace_variant_for(c, it->second->n_media > 0);
-  CHK(trace_geometry(c, it->second, 0, &geom, variant));
   ta.spill = c->spill;
   fill_trace_args(&ta, geom);
   if (variant == TRACE_LDS)
@@ -1862,11 +1903,13 @@ clv_status clv_render_debug(clv_ctx *c, uint32_t scene_id, const clv_render_opts
   if (it == c->scenes.end()) return fail(c, CLV_EINVAL, "unknown scene id");
   HIPCHK(c, hipSetDevice(c->device));
   const uint32_t W = o->width, H = o->height, WH = W * H;
-  CHK(ensure_paths(c, WH));
-  CHK(ensure_pixels(c, WH));
-  CHK(ensure_tables(c, 1, 1));
   const uint32_t blocks = c->trace_blocks;
-  CHK(ensure_spill(c, trace_spill_words(blocks)));
+  CHK(with_room(c, [&]() -> clv_status {
+    CHK(ensure_paths(c, WH));
+    CHK(ensure_pixels(c, WH));
+    CHK(ensure_tables(c, 1, 1));
+    return ensure_spill(c, trace_spill_words(blocks));
+  }));
   DevJob jb = make_job(it->second, it->second->camera, o);
   StreamDrain drain{c->stream}; /* jb outlives the copy from it */
   HIPCHK(c, hipMemcpyAsync(c->jobs, &jb, sizeof(jb), hipMemcpyHostToDevice, c->stream));

@@ -35,13 +35,16 @@ def test_network_and_gate_have_room():
     render()  # what the runtime allocates once per process
     want, few, used = render()
     most = torch.empty(free_bytes() - used - (512 << 20), dtype=torch.uint8, device="cuda")
-    passes = []
-    for spare in range(160 << 20, -1, -(4 << 20)):  # the gate's buffers take 18 MB
+
+    def fits(spare):
         img, n, _ = render(used + spare)
         assert np.array_equal(img, want), spare
-        passes.append(n)
-        if passes.count(few) <= len(passes) - 8:  # eight below what the large passes need
-            break
+        return n == few
+    spare = 160 << 20
+    assert fits(spare)
+    while fits(spare - (16 << 20)):
+        spare -= 16 << 20
+    for k in range(1, 7):  # through the 18 MB of the gate's buffers
+        fits(spare - k * (4 << 20))
     del most
     torch.cuda.empty_cache()
-    assert passes[0] == few and passes[-1] > few, passes
