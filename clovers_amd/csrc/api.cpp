@@ -182,7 +182,9 @@ struct clv_ctx {
 
 namespace {
 
+/* the runtime keeps a failed call's error until it is asked: it is not the next call's, nor another library's */
 clv_status fail(clv_ctx *c, clv_status s, const std::string &msg) {
+  if (s != CLV_EINVAL) (void)hipGetLastError();
   if (c) c->err = msg;
   return s;
 }
@@ -389,10 +391,7 @@ bool free_passes(clv_ctx *c, uint32_t keep) {
 template <class CALL>
 clv_status with_room(clv_ctx *c, CALL call) {
   clv_status st = call();
-  if (st == CLV_ENOMEM && free_passes(c, DEFAULT_TARGET_PATHS)) {
-    (void)hipGetLastError();
-    st = call();
-  }
+  if (st == CLV_ENOMEM && free_passes(c, DEFAULT_TARGET_PATHS)) st = call();
   return st;
 }
 
@@ -811,7 +810,6 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
     if (st != CLV_ENOMEM || again) return st;
     /* no memory: once more without the buffers of earlier large passes, and, where these passes are large ones, at
      * the default size, which needs 50 MB (whole paths) to 1.2 GB (guided) */
-    (void)hipGetLastError();
     if (!free_passes(c, large ? 0u : DEFAULT_TARGET_PATHS) && !large) return st;
     large = false;
     again = true;

@@ -16,9 +16,9 @@ MB = 1 << 20
 def most():
     """all memory but 12 GB, held once: taking it takes seconds"""
     torch.zeros(1, device="cuda")
-    t = torch.empty(torch.cuda.mem_get_info()[0] - (12 << 30), dtype=torch.uint8, device="cuda")
-    yield t
-    del t
+    kept = [torch.empty(torch.cuda.mem_get_info()[0] - (12 << 30), dtype=torch.uint8, device="cuda")]
+    yield  # not the tensor: a fixture's value outlives its end
+    kept.clear()
     torch.cuda.empty_cache()
 
 
