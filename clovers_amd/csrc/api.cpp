@@ -137,6 +137,12 @@ struct clv_ctx {
   uint32_t *shadeq[MC_COUNT] = {nullptr};
   F3 *res = nullptr;         /* sample contributions of a whole-path pass, by slot */
   uint32_t cap_res = 0;
+  /* wavefront [0] and whole-path [1] passes of an untuned context that found no memory: the smallest that failed
+   * (0: none) and the device memory that was free beside them */
+  struct {
+    uint32_t paths = 0;
+    size_t free = 0;
+  } no_room[2];
   /* accumulators */
   uint32_t cap_pixels = 0;
   float *acc32 = nullptr;
@@ -360,6 +366,12 @@ clv_status ensure_res(clv_ctx *c, uint32_t n) {
   HIPCHK(c, dalloc(&c->res, n));
   c->cap_res = n;
   return CLV_OK;
+}
+
+/* bytes free on the current device */
+size_t free_memory() {
+  size_t free = 0, total = 0;
+  return hipMemGetInfo(&free, &total) == hipSuccess ? free : 0;
 }
 
 /* gives back the buffers that hold more than `keep` paths of a pass (sample contributions, path state, lobes), which
@@ -800,17 +812,31 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
     CHK(guide_ensure_net(c));
     return gs.photons ? guide_ensure_gate(c, n) : CLV_OK;
   };
+  auto &no_room = c->no_room[whole ? 1 : 0];
   for (bool large = untuned, again = false;;) {
     pl = PassPlan();
     plan_passes(dj, soff, whole && large ? WHOLE_TARGET_PATHS : c->target_paths, std::max<uint32_t>(1, gs.train_spp),
                 frozen ? 0u : gs.rounds, gs.warmup != 0, &pl);
     if (!whole && large) merge_passes(&pl, MERGED_TARGET_PATHS);
+    if (large && no_room.paths && pl.max_paths >= no_room.paths) {
+      /* a try costs what 25 allocations and frees do (60 to 110 ms for guided passes): not again before more memory
+       * is free than there was */
+      if (free_memory() <= no_room.free) {
+        large = false;
+        continue;
+      }
+      no_room.paths = 0;
+    }
     const clv_status st = reserve();
     if (st == CLV_OK) break;
     if (st != CLV_ENOMEM || again) return st;
     /* no memory: once more without the buffers of earlier large passes, and, where these passes are large ones, at
      * the default size, which needs 50 MB (whole paths) to 1.2 GB (guided) */
     if (!free_passes(c, large ? 0u : DEFAULT_TARGET_PATHS) && !large) return st;
+    if (large && pl.max_paths > DEFAULT_TARGET_PATHS) {
+      no_room.paths = pl.max_paths;
+      no_room.free = free_memory();
+    }
     large = false;
     again = true;
   }
