@@ -92,7 +92,6 @@ struct GuideState {
   float *bweight = nullptr;
   uint32_t *totals = nullptr;                      /* [0] valid records, [1] [2] mean weights, [3] Adam steps */
   uint32_t *host_totals = nullptr;                 /* pinned: a round's valid-record count read back */
-  uint32_t t = 0;                                  /* Adam steps taken */
   uint32_t stamp = 0;                              /* last pass id */
   bool init = false, trained = false;
   /* training schedule (clv_tuning) */
@@ -124,7 +123,6 @@ struct GuideState {
 
 struct clv_ctx {
   int device = 0;
-  bool capturing = false;    /* the render's launch sequence is being captured as a graph: no host reads */
   hipStream_t stream = nullptr;
   std::string err;
   std::map<uint32_t, SceneRes *> scenes;
@@ -182,8 +180,6 @@ struct clv_ctx {
   hipGraphExec_t gexec = nullptr;
   std::string gsig;
   std::string last_sig;     /* signature of the previous eager render: a repeat is captured */
-  uint32_t g_stamps = 0, g_t_after = 0, g_rounds = 0;
-  bool g_trained_after = false;
 };
 
 namespace {
@@ -648,7 +644,6 @@ clv_status guide_reset(clv_ctx *c, uint64_t seed) {
   HIPCHK(c, hipMemsetAsync(g.totals, 0, 4 * sizeof(uint32_t), c->stream)); /* [3]: no Adam steps yet */
   launch_guide_halves(c->stream, g.P, g.Wh);
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  g.t = 0;
   g.init = true;
   g.trained = false;
   return CLV_OK;
@@ -705,17 +700,16 @@ void guide_train_round(clv_ctx *c, uint32_t paths, uint32_t stamp, float *grad_o
                        (unsigned long long *)c->stats + 4);
   const uint32_t step = grad_out ? cap : g.step;
   const uint32_t epochs = grad_out ? 1u : std::max<uint32_t>(1u, g.epochs);
-  /* steps past the round's valid records are empty (the kernels skip them);
-   * outside a stream capture the count is read back so they are not launched
-   * at all -- the same parameters either way */
+  /* steps past the round's valid records are empty (the kernels skip them):
+   * the count is read back so they are not launched at all -- the same
+   * parameters either way */
   uint32_t used = cap;
-  if (!grad_out && !c->capturing && g.host_totals &&
+  if (!grad_out && g.host_totals &&
       hipMemcpyAsync(g.host_totals, g.totals, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream) == hipSuccess &&
       hipStreamSynchronize(c->stream) == hipSuccess)
     used = std::min(cap, g.host_totals[0]);
   for (uint32_t e = 0; e < epochs; e++)
     for (uint32_t b = 0; b < used; b += step) {
-      if (!grad_out) g.t++;
       launch_guide_step(c->stream, g.rec, g.recL, g.list, g.totals, cap, b, std::min(step, cap - b), wclip, g.P, g.M,
                         g.V, g.Wh, g.partial, g.lr, grad_out);
     }
@@ -906,8 +900,8 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
   uint32_t rounds_run = 0;
   bool any_sq = false;
   for (uint32_t k = 0; k < n; k++) any_sq = any_sq || jobs[k].xyz_sq_out;
-  /* every launch of the render; no host synchronisation inside, so the
-   * sequence can be captured as a graph */
+  /* every launch of the render; without guided jobs no host synchronisation
+   * inside, so the sequence can be captured as a graph */
   auto enqueue = [&]() -> clv_status {
   if (whole) {
     for (uint32_t p = 0; p < passes; p++) {
@@ -1035,9 +1029,7 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
   const bool use_graph = c->use_graph && !timing && !any_guide;
   std::string sig;
   if (use_graph) {
-    /* everything a launch argument depends on; pass ids of guided renders
-     * are left out: a replay reuses the captured ones, which only the same
-     * (deterministic) render can have written */
+    /* everything a launch argument of an unguided render depends on */
     auto add = [&sig](const void *p, size_t b) { sig.append((const char *)p, b); };
     add(dj.data(), dj.size() * sizeof(DevJob));
     add(pl.items.data(), pl.items.size() * sizeof(DevItem));
@@ -1045,19 +1037,12 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
     add(pl.paths.data(), pl.paths.size() * 4);
     add(pl.res.data(), pl.res.size() * 4);
     add(pl.depth.data(), pl.depth.size() * 4);
-    add(pl.train.data(), pl.train.size());
-    const uint32_t sc[14] = {(uint32_t)whole, flags, any_sq, any_guide, frozen, (uint32_t)variant, c->grid_cap, ds.has_xforms,
-                             gs.train_spp, ds.has_ext, gs.credit, tail_depth, photon_rounds ? gs.photons : 0u,
-                             photon_rounds ? gs.pre_rounds : 0u};
+    const uint32_t sc[8] = {(uint32_t)whole, flags, any_sq, (uint32_t)variant, c->grid_cap, ds.has_xforms, ds.has_ext, tail_depth};
     add(sc, sizeof(sc));
-    const float gf[5] = {gs.alpha, gs.lr, gs.wclip, (float)gs.records, gs.gate_density};
-    add(gf, sizeof(gf));
     add(&geom, sizeof(geom));
     add(&pb, sizeof(pb));
-    const void *ptrs[] = {c->shadeq[0], c->shadeq[1], c->shadeq[2], c->shadeq[3],
-                          c->shadeq[4], c->acc32, c->acc64, c->accsq, c->out, c->out_sq, c->counts, c->stats,
-                          c->spill, c->cie, c->res, c->jobs, c->items, gs.lobes, gs.rec, gs.gcnt, gs.list, gs.bcount,
-                          gs.bweight, gs.totals, gs.P, gs.M, gs.V, gs.Wh, gs.partial, gs.cells, gs.cell_tot, gs.gate};
+    const void *ptrs[] = {c->shadeq[0], c->shadeq[1], c->shadeq[2], c->shadeq[3], c->shadeq[4], c->acc32, c->acc64,
+                          c->accsq, c->out, c->out_sq, c->counts, c->stats, c->spill, c->cie, c->res, c->jobs, c->items};
     add(ptrs, sizeof(ptrs));
     for (auto &a : c->arena) add(&a.p, sizeof(a.p));
   }
@@ -1068,23 +1053,15 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
   if (use_graph) c->last_sig = sig;
   if (repeat && c->gexec && c->gsig == sig) {
     HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
-    gs.stamp += c->g_stamps;
-    gs.t = c->g_t_after;
-    gs.trained = c->g_trained_after;
-    if (photon_rounds) gs.gate_valid = true;
-    rounds_run = c->g_rounds;
   } else {
     bool capturing = false;
-    const uint32_t stamp0 = gs.stamp;
     if (repeat) {
       if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
       c->gexec = nullptr;
       c->gsig.clear();
       capturing = hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) == hipSuccess;
     }
-    c->capturing = capturing;
     clv_status st = enqueue();
-    c->capturing = false;
     if (capturing) {
       hipGraph_t g = nullptr;
       hipError_t e = hipStreamEndCapture(c->stream, &g);
@@ -1096,10 +1073,6 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
         return fail(c, CLV_EDEVICE, std::string("graph capture: ") + hipGetErrorString(e));
       }
       c->gsig = sig;
-      c->g_stamps = gs.stamp - stamp0;
-      c->g_t_after = gs.t;
-      c->g_trained_after = gs.trained;
-      c->g_rounds = rounds_run;
       HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
     } else if (st != CLV_OK) {
       return st;
@@ -1616,7 +1589,6 @@ clv_status clv_guide_set_params(clv_ctx *c, const float *in, uint32_t n) {
   HIPCHK(c, hipMemsetAsync(g.V, 0, GD_NPARAM * sizeof(float), c->stream));
   launch_guide_halves(c->stream, g.P, g.Wh);
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  g.t = 0;
   g.trained = true;
   return CLV_OK;
 }
