@@ -1699,7 +1699,7 @@ clv_status clv_autotune(clv_ctx *c, const clv_job *jobs, uint32_t n, uint64_t tr
     uint32_t target, kernel, lds;
   };
   std::vector<Cand> cands;
-  for (uint32_t lg = 22; lg <= 26; lg++) {
+  for (uint32_t lg = 22; lg <= 26; lg++) { /* 2^22: the automatic size */
     const uint32_t tgt = 1u << lg;
     if (lg > 22 && (uint64_t)(tgt >> 1) >= tsamples) break; /* larger passes than the work change nothing */
     cands.push_back({tgt, CLV_TRACE_LDS_CACHED, 64512});
@@ -1741,10 +1741,11 @@ clv_status clv_autotune(clv_ctx *c, const clv_job *jobs, uint32_t n, uint64_t tr
   }
   /* the best shape with the late bounces in one launch (k_tail): fewer launches where few paths are
    * left, which pays on small images; not for batches with guided jobs, whose vertices in the tail
-   * sample the plain mixture */
+   * sample the plain mixture, nor for whole paths in one launch, which have no tail */
   bool any_guided = false;
   for (uint32_t k = 0; k < n; k++) any_guided = any_guided || jobs[k].opts.guiding == CLV_GUIDE_ON;
-  if (!any_guided && best_ms < 1e300) {
+  CHK(clv_tuning_set(c, &best));
+  if (!any_guided && best_ms < 1e300 && !whole_paths(c, false, 0u)) {
     const clv_tuning shape = best;
     for (uint32_t d = 2; d <= 4; d++) {
       clv_tuning t = shape;

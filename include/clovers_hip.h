@@ -345,14 +345,17 @@ typedef enum {
   CLV_TRACE_WW = 2,         /* one ray per thread, node steps and leaf steps in separate loops */
   CLV_TRACE_LDS_CACHED = 3  /* 768-thread blocks, top of the BVH and leading records cached in LDS; renders without
                                guided jobs run every path from the camera to its end in one launch per pass, from
-                               LDS if the scene of all jobs fits in lds_bytes whole, else from memory */
+                               LDS if the scene of all jobs fits in lds_bytes whole, else from memory; guided
+                               renders read the scene from memory where LDS holds less than half of it */
 } clv_trace_kernel;
 typedef struct {
-  uint32_t target_paths;    /* samples per wavefront pass (queue and path-state capacity).  At the default, 2^22, a
-                               pass that runs whole paths in one launch (CLV_TRACE_LDS_CACHED, no guided job, no
-                               CLV_FLAG_TIME_KERNELS or _COUNT) holds up to 2^27: it needs 12 bytes per sample;
-                               wavefront passes behind the last training round are joined up to 2^25.
-                               Where memory is short, both keep to 2^22 */
+  uint32_t target_paths;    /* samples per wavefront pass (queue and path-state capacity).  The default, 2^22,
+                               stands for the automatic size; any other value is kept to (2^22 - 1 asks for passes
+                               of the default size and no larger ones).  Automatic: a pass that runs whole paths in
+                               one launch (CLV_TRACE_LDS_CACHED, no guided job, no CLV_FLAG_TIME_KERNELS or _COUNT)
+                               holds up to 2^27, at 12 bytes per sample beside up to 140 MB of traversal stacks;
+                               wavefront passes behind the last training round are joined up to 2^25 (9.2 GB).  Where
+                               memory is short, both keep to 2^22; a later call that finds none gets theirs */
   uint32_t trace_kernel;    /* clv_trace_kernel */
   uint32_t lds_bytes;       /* dynamic LDS per block of CLV_TRACE_LDS_CACHED (<= 64512) */
   uint32_t shade_grid_cap;  /* largest grid of the shading kernel, in 256-thread blocks (the library also caps it
@@ -394,10 +397,11 @@ clv_status clv_tuning_get(const clv_ctx *ctx, clv_tuning *out);
 clv_status clv_tuning_set(clv_ctx *ctx, const clv_tuning *t);
 /* Autotuner: renders a shortened copy of the batch (the same jobs with fewer
  * samples, about `trial_samples` in all; 0 = 64M) under each candidate launch
- * shape -- pass sizes 2^22..2^26 paths x {LDS-cached traversal with a 64 KB or
- * 16 KB cache, plain traversal}, then the best of them with tail_depth 2, 3
- * and 4 unless a job is guided -- keeps the fastest on the context and
- * returns it.  Outputs of the trials are discarded. */
+ * shape -- the automatic pass size (2^22) and 2^23..2^26 paths x {LDS-cached
+ * traversal with a 64 KB or 16 KB cache, plain traversal}, then the best of
+ * them with tail_depth 2, 3 and 4 unless a job is guided or whole paths run in
+ * one launch -- keeps the fastest on the context and returns it.  Outputs of
+ * the trials are discarded. */
 clv_status clv_autotune(clv_ctx *ctx, const clv_job *jobs, uint32_t n_jobs, uint64_t trial_samples,
                         clv_tuning *best_out);
 
