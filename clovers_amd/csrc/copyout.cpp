@@ -17,16 +17,17 @@ namespace {
 
 /* a window's half of the pinned memory: two of 8 MB keep the link busy (150 us
  * each) and pin no more than the 16 MB a context may have staged with.  Their
- * pages' first touch costs 2 to 4 ms over the threads, which a context that
- * copies once never earns back, so it starts with half of them and grows when
- * it has sent GROW_AFTER.  First hits and normals at 1080p, a new context's
- * calls 1 / 2 / steady: 9.0 / 6.4 / 6.3 ms the runtime's way, 10.5 / 3.3 / 3.3
- * with 8 MB at once, 8.5 / 4.0 / 3.3 so (6.3 in the call that grows); with 2 MB
- * first 7.1 / 3.8 / 3.2, but results of 3 to 25 MB take a sixth longer until
- * then. */
+ * pages' first touch costs 2 to 4 ms over the threads where the device does not
+ * hide it, which a context that copies once never earns back, so it starts with
+ * half of them, and the first copy that these do not hold after GROW_AFTER bytes
+ * gets the larger ones.  First hits and normals at 1080p, a new context's calls
+ * 1 / 2 / 3: 8.7 / 6.1 / 6.0 ms the runtime's way, 10.7 / 3.4 / 3.4 with 8 MB at
+ * once, 8.0 / 5.0 / 3.3 so; with 2 MB first a tenth less in the first call, but
+ * results of 3 to 25 MB take a sixth longer until then.  (With 4 MB for good,
+ * calls that return 14 MB take 1 to 3% longer.) */
 #define HALF_FIRST ((size_t)4 << 20)
 #define HALF_BYTES ((size_t)8 << 20)
-#define GROW_AFTER ((size_t)128 << 20)
+#define GROW_AFTER ((size_t)48 << 20)
 #define MAX_FLAGS (HALF_BYTES / COPY_CHUNK)
 #define PIN_HEAD (64 + 2 * MAX_FLAGS * sizeof(uint32_t))
 
@@ -157,6 +158,7 @@ bool CopyOut::reserve(size_t total) {
   memset(p, 0, PIN_HEAD);
   pin_ = p;
   cap_ = half_;
+  touched_[0] = touched_[1] = 0;
   return true;
 }
 
@@ -164,12 +166,20 @@ bool CopyOut::reserve(size_t total) {
  * array's faults cost more than its copy (25 MB: 1.0 ms with huge pages and 4.7
  * without, against 0.9 of copying), and the device is busy meanwhile.  (Helpers
  * that map their own parts as well only wait for each other: a 2.8 MB image
- * 0.56 ms instead of 0.50.) */
+ * 0.56 ms instead of 0.50.)  Then the pinned pages of the first two windows,
+ * where they have not been touched yet. */
 void CopyOut::map_pages(const std::vector<CopySeg> &segs) {
+  const auto here = [this] { return __atomic_load_n(flags(0), __ATOMIC_RELAXED) == windows_[0].stamp; };
+  bool can = true;
   for (const CopySeg &s : segs)
-    for (size_t at = 0; s.bytes >= HELP_BYTES && at < s.bytes; at += HELP_BYTES) {
-      if (__atomic_load_n(flags(0), __ATOMIC_RELAXED) == windows_[0].stamp) return;
-      if (!map_range((char *)s.dst + at, std::min(HELP_BYTES, s.bytes - at))) return;
+    for (size_t at = 0; can && s.bytes >= HELP_BYTES && at < s.bytes; at += HELP_BYTES) {
+      if (here()) return;
+      can = map_range((char *)s.dst + at, std::min(HELP_BYTES, s.bytes - at));
+    }
+  for (size_t w = 0; w < std::min<size_t>(2, windows_.size()); w++)
+    for (; touched_[w] < windows_[w].bytes; touched_[w] += 4096) {
+      if (here()) return;
+      (void)*(const volatile char *)(half(w) + touched_[w]);
     }
 }
 
@@ -271,7 +281,7 @@ hipError_t CopyOut::run(hipStream_t st, const std::vector<CopyArray> &arrays, co
   failed_ = 0;
   size_t total = 0;
   for (const CopySeg &s : segs) total += s.bytes;
-  half_ = sent_ < GROW_AFTER ? HALF_FIRST : HALF_BYTES;
+  half_ = cap_ == HALF_BYTES || (sent_ >= GROW_AFTER && total > 2 * HALF_FIRST) ? HALF_BYTES : HALF_FIRST;
   if (segs.empty() || !reserve(total)) {
     for (const CopySeg &s : segs) {
       direct(s);

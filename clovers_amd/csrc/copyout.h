@@ -86,6 +86,7 @@ class CopyOut {
   char *pin_ = nullptr; /* the stats, the flags of both halves, the halves */
   size_t cap_ = 0;      /* bytes of a half */
   size_t half_ = 0;     /* largest window of the current run */
+  size_t touched_[2] = {0, 0}; /* bytes of the halves whose pages the caller has touched ahead */
   size_t direct_ = 0; /* bytes sent the runtime's way for want of pinned memory */
   size_t sent_ = 0;   /* bytes sent through the windows */
   uint32_t stamp_ = 0;
