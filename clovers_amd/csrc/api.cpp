@@ -1699,11 +1699,17 @@ clv_status clv_autotune(clv_ctx *c, const clv_job *jobs, uint32_t n, uint64_t tr
     uint32_t target, kernel, lds;
   };
   std::vector<Cand> cands;
+  bool any_guided = false;
+  for (uint32_t k = 0; k < n; k++) any_guided = any_guided || jobs[k].opts.guiding == CLV_GUIDE_ON;
   for (uint32_t lg = 22; lg <= 26; lg++) { /* 2^22: the automatic size */
     const uint32_t tgt = 1u << lg;
     if (lg > 22 && (uint64_t)(tgt >> 1) >= tsamples) break; /* larger passes than the work change nothing */
-    cands.push_back({tgt, CLV_TRACE_LDS_CACHED, 64512});
-    cands.push_back({tgt, CLV_TRACE_LDS_CACHED, 16384});
+    /* whole paths: the automatic size holds the trial in one pass, so another size that does is the same render here,
+     * though not where the batch has more samples than its trial */
+    if (any_guided || lg == 22 || tgt < tsamples) {
+      cands.push_back({tgt, CLV_TRACE_LDS_CACHED, 64512});
+      cands.push_back({tgt, CLV_TRACE_LDS_CACHED, 16384});
+    }
     cands.push_back({tgt, CLV_TRACE_SIMPLE, 64512});
   }
   clv_tuning best = start;
@@ -1742,8 +1748,6 @@ clv_status clv_autotune(clv_ctx *c, const clv_job *jobs, uint32_t n, uint64_t tr
   /* the best shape with the late bounces in one launch (k_tail): fewer launches where few paths are
    * left, which pays on small images; not for batches with guided jobs, whose vertices in the tail
    * sample the plain mixture, nor for whole paths in one launch, which have no tail */
-  bool any_guided = false;
-  for (uint32_t k = 0; k < n; k++) any_guided = any_guided || jobs[k].opts.guiding == CLV_GUIDE_ON;
   CHK(clv_tuning_set(c, &best));
   if (!any_guided && best_ms < 1e300 && !whole_paths(c, false, 0u)) {
     const clv_tuning shape = best;

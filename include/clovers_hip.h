@@ -397,11 +397,11 @@ clv_status clv_tuning_get(const clv_ctx *ctx, clv_tuning *out);
 clv_status clv_tuning_set(clv_ctx *ctx, const clv_tuning *t);
 /* Autotuner: renders a shortened copy of the batch (the same jobs with fewer
  * samples, about `trial_samples` in all; 0 = 64M) under each candidate launch
- * shape -- the automatic pass size (2^22) and 2^23..2^26 paths x {LDS-cached
- * traversal with a 64 KB or 16 KB cache, plain traversal}, then the best of
- * them with tail_depth 2, 3 and 4 unless a job is guided or whole paths run in
- * one launch -- keeps the fastest on the context and returns it.  Outputs of
- * the trials are discarded. */
+ * shape -- the automatic pass size (2^22) and 2^23..2^26 paths (sizes that give
+ * other passes than it) x {LDS-cached traversal with a 64 KB or 16 KB cache,
+ * plain traversal}, then the best of them with tail_depth 2, 3 and 4 unless a
+ * job is guided or whole paths run in one launch -- keeps the fastest on the
+ * context and returns it.  Outputs of the trials are discarded. */
 clv_status clv_autotune(clv_ctx *ctx, const clv_job *jobs, uint32_t n_jobs, uint64_t trial_samples,
                         clv_tuning *best_out);
 

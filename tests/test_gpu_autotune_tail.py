@@ -1,5 +1,5 @@
-"""The autotuner tries the tail launch only where there is one: a batch whose fastest shape runs whole paths in one
-launch keeps the tail setting it had."""
+"""The autotuner tries only what makes a difference: a batch whose fastest shape runs whole paths in one launch keeps
+the tail setting it had, and its pass size stays automatic unless a smaller one is faster."""
 import pytest
 
 import clovers_amd
@@ -19,3 +19,15 @@ def test_whole_paths_have_no_tail_to_tune(tail):
                 assert best["tail_depth"] == tail
             assert r.tuning() == best
         assert best["trace_kernel"] == abi.TRACE_LDS_CACHED  # twice as fast on this scene
+
+
+@pytest.mark.parametrize("spp", [3, 15, 32])
+def test_a_size_that_gives_the_same_passes_is_not_chosen(spp):
+    """the trial in one pass is the automatic size's; a set size that holds the trial too is kept to in renders of
+    more samples, so it is no candidate"""
+    with clovers_amd.Renderer(0) as r:
+        sid = r.upload(synth.spheres())
+        n = 1920 * 1080 * spp
+        best = r.autotune([(sid, abi.render_opts(1920, 1080, spp, 12, seed=1))])
+        assert best["trace_kernel"] == abi.TRACE_LDS_CACHED  # twice as fast on this scene
+        assert best["target_paths"] == 1 << 22 or best["target_paths"] < n
