@@ -9,11 +9,11 @@ region (uploaded once, like the reference's scene initialisation that
 precedes its timed draw(), render.rs:137-150).
 
 Prints one JSON line with Msamples/s (one sample = one camera path carrying 4
-hero wavelengths), the roofline of the dominant kernel (BVH traversal, its
-launch time measured with HIP events on the render stream in renders whose
-bounces are separate launches: vector-ALU bound when the scene sits in LDS,
-memory bound otherwise; the timed steps run whole paths in one launch, with the
-same traversal inside), the CPU baseline (the
+hero wavelengths), the roofline of the timed steps' kernel (k_paths, which runs
+whole paths; vector-ALU bound when the scene sits in LDS, bound by node fetches
+otherwise) and in it that of the traversal in renders whose bounces are separate
+launches, timed with HIP events on the render stream (the only one for workloads
+without a profile of k_paths), the CPU baseline (the
 CPU oracle -- a C++ restatement of the reference's renderer -- timed on this
 host's cores over a bounded slice of the same workload) and, nested as
 `time_to_rmse`, the metric's second half: the wall time the guided method
@@ -100,6 +100,35 @@ def profiled_shape(workload):
     base = t["kernel"].split("<")[0]
     kern = [k for n, k in names.items() if n == base]
     return {"target_paths": t["target_paths"], "trace_kernel": kern[0]} if kern else None
+
+
+def paths_roofline(workload, samples, ms_per_step):
+    """the whole-path kernel over a timed step (its launches and the summing of
+    the samples, 1% of it), from the committed rocprofv3 passes of the same
+    workload (profiles/counters.json and traffic.json, per sample); None if it
+    has none"""
+    try:
+        with open(os.path.join(ROOT, "profiles", "counters.json")) as f:
+            c = json.load(f)[workload + "_paths"]
+        with open(os.path.join(ROOT, "profiles", "traffic.json")) as f:
+            t = json.load(f)[workload + "_paths"]
+    except (OSError, KeyError, ValueError):
+        return None
+    n = samples / c["samples_per_launch"]
+    util = c["SQ_THREAD_CYCLES_VALU"] / (64.0 * c["SQ_ACTIVE_INST_VALU"])
+    insts = c["SQ_INSTS_VALU"] * n
+    ops = insts * 64.0 * util / (ms_per_step * 1e-3) / 1e12
+    traffic = (t["fetch_bytes_per_launch"] + t["write_bytes_per_launch"]) * n
+    gbs = traffic / (ms_per_step * 1e-3) / 1e9
+    valu = ops / VALU_PEAK_TLANE > gbs / HBM_PEAK_GBS
+    ach, peak, unit = (ops, VALU_PEAK_TLANE, "T lane-op/s") if valu else (gbs, HBM_PEAK_GBS, "GB/s")
+    return {"bound": "valu" if valu else "hbm", "achieved": round(ach, 3), "peak": peak, "unit": unit,
+            "frac": round(ach / peak, 4), "kernel": "%s (whole paths)" % c["kernel"].split("<")[0],
+            "traffic": int(traffic), "valu_insts_per_step": int(insts), "valu_utilization": round(util, 4),
+            "valu_tlane_ops": round(ops, 3), "measured_gbs": round(gbs, 1),
+            "note": "VALU instructions x 64 lanes x lane utilisation, or FETCH_SIZE + WRITE_SIZE bytes (between L2 and "
+                    "the memory side, register spills and traversal stacks among them), of the profiled launches per "
+                    "sample (profiles/counters.json, traffic.json) over the device time of a timed step"}
 
 
 def view_jobs(sid, w, opts_fn):
@@ -462,7 +491,7 @@ def main():
     nonfinite = int(sum((~np.isfinite(img)).any(axis=-1).sum() for img, _ in outs))
     log("non-finite pixels: %d" % nonfinite)
 
-    # dominant kernel: traversal.  Its committed counter profile (profiles/) was
+    # the traversal in launches of its own.  Its committed counter profile (profiles/) was
     # taken at one launch shape; the roofline renders use that shape, whatever
     # the autotuner picked for the timed steps, so per-launch counters and
     # per-launch times describe the same launches
@@ -545,6 +574,11 @@ def main():
                                  "visits x 128 B + "
                                  "primitive tests x record bytes + 48 B of ray stream per ray; " + lds_note})
     r.close()
+    # without guided jobs the LDS-cached traversal stands for whole paths in one launch
+    whole = args.workload != "batch64" and tuning["trace_kernel"] == abi.TRACE_LDS_CACHED
+    paths = paths_roofline(args.workload, samples, ms_per_step) if whole else None
+    if paths:
+        roofline = dict(paths, traversal=roofline)
 
     cpu = None
     if not args.no_cpu_baseline and scene is not None:
@@ -566,7 +600,7 @@ def main():
                    "samples_per_step": samples, "nonfinite_pixels": nonfinite, "device_ms_per_step": round(ms_per_step, 3),
                    "wall_ms_per_step_with_readback": round(wall_ms_per_step, 3),
                    "wall_msamples_per_s_with_readback": round(samples / (wall_ms_per_step / 1e3) / 1e6, 3),
-                   "parallelism": "1 GPU, wavefront",
+                   "parallelism": "1 GPU, %s" % ("whole paths in one launch" if whole else "wavefront"),
                    "scene_builder": args.builder, "scene_build_ms": round(build_ms, 1),
                    "tuning": dict(tuning, trace_kernel=abi.TRACE_NAMES[tuning["trace_kernel"]]),
                    "autotune_ms": round(tune_ms, 1)}),

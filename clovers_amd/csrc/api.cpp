@@ -277,8 +277,9 @@ bool whole_paths(const clv_ctx *c, bool any_guide, uint32_t flags) {
   return c->trace_variant == TRACE_LDS && !any_guide && !(flags & (CLV_FLAG_TIME_KERNELS | CLV_FLAG_COUNT));
 }
 
-/* a pass of k_paths keeps 12 bytes per sample, so an untuned context runs the
- * samples of a whole render in one (up to 1.6 GB of contributions) */
+/* a pass of k_paths keeps 12 bytes per sample, beside the traversal stacks of its
+ * resident blocks (100 MB with the scene in LDS, 136 MB from memory), so an untuned
+ * context runs the samples of a whole render in one (up to 1.6 GB of contributions) */
 #define DEFAULT_TARGET_PATHS (1u << 22)
 #define WHOLE_TARGET_PATHS (1u << 27)
 
@@ -825,7 +826,7 @@ clv_status render_jobs(clv_ctx *c, const clv_job *jobs, uint32_t n) {
     if (st == CLV_OK) break;
     if (st != CLV_ENOMEM || again) return st;
     /* no memory: once more without the buffers of earlier large passes, and, where these passes are large ones, at
-     * the default size, which needs 50 MB (whole paths) to 1.2 GB (guided) */
+     * the default size, which needs 50 MB beside the stacks (whole paths) to 1.2 GB (guided) */
     if (!free_passes(c, large ? 0u : DEFAULT_TARGET_PATHS) && !large) return st;
     if (large && pl.max_paths > DEFAULT_TARGET_PATHS) {
       no_room.paths = pl.max_paths;

@@ -1873,8 +1873,9 @@ __device__ __forceinline__ bool trav_ray(Trav &L, const DevScene &sc, const LdsW
  * a sphere field's 33 KB, at 6 waves per SIMD (80 VGPRs); 768 threads take
  * 29.4 ms where 512 take 29.2 and leave less room for larger scenes, 512
  * threads at 5 waves and no spills 36.4.  From memory it waits on node
- * fetches: two-wave blocks at 8 waves per SIMD, and rays that are left on their
- * way while the others are shaded (trav_ray): the 1M-triangle mesh takes 46.8
+ * fetches (with stacks and spills 5.2 TB/s behind L2, as a large copy): two-wave
+ * blocks at 8 waves per SIMD, and rays that are left on their way while the
+ * others are shaded (trav_ray): the 1M-triangle mesh takes 46.8
  * ms, 48.9 in blocks of 256 threads, 47.9 of 64, 49.4 at 6 waves (before rays
  * were left: 63.6, and 68.6 / 69.1 with node and leaf steps taken in another
  * order than by majority: node-first / both each turn).  XF, EXT and
