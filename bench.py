@@ -524,7 +524,8 @@ def main():
                 "the mesh BVH (226k nodes, 29 MB) and triangles (80 MB) exceed the LDS window and L2; node and "
                 "triangle fetches come from HBM / the MALL (FETCH_SIZE in profiles/)")
     if args.workload == "batch64":
-        lds_note = ("per-ray figures from a counting render at 1/16 of each job's samples over all 64 scenes; "
+        lds_note = ("the timed steps take node and primitive turns by majority, these one of each a lane; "
+                    "per-ray figures from a counting render at 1/16 of each job's samples over all 64 scenes; "
                     "record bytes are those of the job with the most samples")
     kname = TRACE_KERNELS[roof_tuning["trace_kernel"]]
     traffic = measured_traffic(args.workload, kname, roof_tuning["target_paths"])
